@@ -1,278 +1,278 @@
 // Batched tall-skinny least squares, FP32: `count` independent problems
-// min ||A x - b||, A m x n row-major (n <= 32, m >= n), one wavefront each.
+// min ||A x - b||, A m x n row-major (n <= 32, m >= n), one workgroup each.
 //
 // numax's `lstsq` (numax/linalg/qr.mojo:746-821) is blocked Householder QR
-// (geqr2_panel, panel.mojo:1975-2073, with LAPACK dlarfg's convention:
-// beta = -sign(alpha) sqrt(alpha^2 + sigma), tau = (beta - alpha) / beta,
-// v = x / (alpha - beta), tau = 0 when sigma = 0), Q^T b applied panel by
-// panel (qr.mojo:470-534), then the upper-triangular solve with R
-// (qr.mojo:536-612).  Here the same reflectors are applied as a streaming
-// (TSQR-style) factorization: the wavefront keeps the running 32 x 33
-// triangle [R | Q^T b] in lanes 0..31 and brings the next 32 rows of [A | b]
-// into lanes 32..63; each of the 32 column steps builds one reflector over
-// row k of the triangle and the 32 new rows (the triangle is zero below its
-// diagonal), so the 1024 x 33 problem is read exactly once.  Column sums
-// across the wavefront use recursive halving; the reflector's coefficients
-// are broadcast from lanes through scalar registers.
+// (geqr2_panel, panel.mojo:1975-2073), Q^T b applied panel by panel
+// (qr.mojo:470-534), then the upper-triangular solve with R
+// (qr.mojo:536-612).  Here the n reflectors are applied one column at a time
+// to [A | b] held whole in registers, and x comes from R and the first n
+// entries of Q^T b; R can differ from numax's in the sign of a row whose
+// column is already zero below the diagonal, x does not.
+//
+// What bounds it: not HBM (each problem is read once) but the chain of n
+// dependent reflectors per problem -- a sum over all rows, a square root and
+// a division, an update -- so the layout is chosen for the shortest step and
+// two problems share a CU to fill each other's waits.
+//
+// Layout: a thread holds 32 rows of columns c and c + 16, c = lane % 16; the
+// four 16-lane rows of a wavefront and the wavefronts hold different rows.
+// The reflector's column x then reaches the other columns of its rows as a
+// DPP row broadcast inside the multiply-adds, dot products need no reduction
+// across columns, and what is left of the cross-lane work is one value per
+// column over the row groups (two lane-swap steps in a wavefront, one LDS
+// round and one barrier across them).  With a row per lane instead, every
+// step reduced 33 values over 256 threads and read them back: 165 LDS reads
+// and 126 shuffles a step, and 4096 problems of 1024 x 32 took 6.55 ms.
+// In this layout they take 0.64 ms (10.5x; 865 GB/s of the 4.8 TB/s a copy
+// reaches): about 210 instructions a step and wavefront, 60 % of the time in
+// issue, the rest in the step's barrier and LDS round.
 #include <math.h>
 
 #include "nmx_internal.h"
 
 namespace {
 
-constexpr int kCols = 33;  // 32 columns of A, then b
+constexpr int kRows = 32;              // rows a thread holds
+constexpr int kGroupPad = kRows + 4;   // LDS stride of a row group's column (b128 aligned, banks apart)
 
-// Sum NV per-lane partials over the 64 lanes (recursive halving); lane l
-// ends with the total of partial l / (64 / NV).
-template <int NV>
-__device__ __forceinline__ float halving_sum(float (&s)[NV], int lane) {
-  int m = 32;
-#pragma unroll
-  for (int w = NV / 2; w >= 1; w >>= 1, m >>= 1) {
-    const bool hi = (lane & m) != 0;
-#pragma unroll
-    for (int k = 0; k < w; k++) {
-      const float keep = hi ? s[w + k] : s[k];
-      const float send = hi ? s[k] : s[w + k];
-      s[k] = keep + __shfl_xor(send, m);
-    }
-  }
-  float v = s[0];
-#pragma unroll
-  for (; m >= 1; m >>= 1) v += __shfl_xor(v, m);
-  return v;
+// lane L of each 16-lane row to the whole row (folds into the consuming instruction)
+template <int L>
+__device__ __forceinline__ float row_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + L, 0xF, 0xF, true));
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+// v(lane) + v(lane ^ 16), then the same over lane ^ 32
+__device__ __forceinline__ float sum_rows16(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// lanes 0..31: a(lane) + a(lane + 32); lanes 32..63: b(lane - 32) + b(lane)
+__device__ __forceinline__ float sum_halves(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-constexpr int pow2_at_least(int x) { return x <= 1 ? 1 : 2 * pow2_at_least((x + 1) / 2); }
-
-// One reflector: column K of the stacked [triangle; new rows], applied to
-// columns K+1 .. 32 (b included).  `in` marks the lanes the reflector spans
-// (lane K of the triangle and every new row).
-template <int K>
-__device__ __forceinline__ void reflect(float (&r)[kCols], int lane) {
-  constexpr int NJ = kCols - 1 - K;  // columns to the right, b included
-  constexpr int P2 = pow2_at_least(NJ);
-  const bool below = lane >= 32;
-  const float alpha = readlane_f(r[K], K);
-  // sigma = sum over the new rows of x^2
-  float sq[1] = {below ? r[K] * r[K] : 0.f};
-  const float sigma = readlane_f(halving_sum<1>(sq, lane), 0);
-  float tau = 0.f, beta = alpha, scale = 0.f;
-  if (sigma != 0.f) {
-    beta = -copysignf(sqrtf(alpha * alpha + sigma), alpha);
-    tau = (beta - alpha) / beta;
-    scale = 1.f / (alpha - beta);
-  }
-  // v: 1 on row K of the triangle, x * scale on the new rows, 0 elsewhere
-  const float vl = below ? r[K] * scale : (lane == K ? 1.f : 0.f);
-  if (below) r[K] = 0.f;           // annihilated by the reflector
-  if (lane == K) r[K] = beta;      // R_kk
-  if (NJ > 0 && tau != 0.f) {
-    // w_j = sum_lanes v * r[j], j = K+1 .. 32
-    float p[P2];
-#pragma unroll
-    for (int j = 0; j < P2; j++) p[j] = (j < NJ) ? vl * r[K + 1 + j] : 0.f;
-    const float tot = halving_sum<P2>(p, lane);
-    constexpr int SPREAD = 64 / P2;
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-      const float wj = readlane_f(tot, j * SPREAD);
-      r[K + 1 + j] -= tau * vl * wj;
-    }
-  }
-}
-
-template <int K>
-__device__ __forceinline__ void reflect_all(float (&r)[kCols], int lane) {
-  if constexpr (K < 32) {
-    reflect<K>(r, lane);
-    reflect_all<K + 1>(r, lane);
-  }
-}
-
-__global__ void __launch_bounds__(256) gels_tsqr_kernel(int count, int m, int n, const float* __restrict__ A,
-                                                        const float* __restrict__ B, float* __restrict__ X) {
-  const int lane = threadIdx.x & 63;
-  const int waves = gridDim.x * (blockDim.x / 64);
-  for (int p = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); p < count; p += waves) {
-    const float* Ap = A + (int64_t)p * m * n;
-    const float* Bp = B + (int64_t)p * m;
-    const __amdgpu_buffer_rsrc_t ra = buf_rsrc(Ap);
-    const __amdgpu_buffer_rsrc_t rb = buf_rsrc(Bp);
-    float r[kCols];
-    // the triangle starts as [I_pad | 0]: a unit diagonal on the columns past
-    // n keeps R non-singular there, and those unknowns come out 0
-#pragma unroll
-    for (int j = 0; j < kCols; j++) r[j] = (lane < 32 && j == lane && j >= n && j < 32) ? 1.f : 0.f;
-    for (int r0 = 0; r0 < m; r0 += 32) {
-      // next 32 rows of [A | b] into lanes 32..63 (zero past m / past n)
-      const int row = r0 + lane - 32;
-      const bool ld = lane >= 32 && row < m;
-      const uint32_t rowoff = (uint32_t)(ld ? row : 0) * (uint32_t)n;
-#pragma unroll
-      for (int j = 0; j < 32; j++) {
-        const float a = buf_load<float>(ra, (ld & (j < n)) ? 4u * (rowoff + (uint32_t)j) : kBufOob);
-        if (lane >= 32) r[j] = a;
-      }
-      const float bv = buf_load<float>(rb, ld ? 4u * (uint32_t)row : kBufOob);
-      if (lane >= 32) r[32] = bv;
-      reflect_all<0>(r, lane);
-    }
-    // R x = (Q^T b)[0:32] by back substitution (qr.mojo:536-612's _trsv)
-    float acc = r[32];
-#pragma unroll
-    for (int c = 31; c >= 0; c--) {
-      const float xc = readlane_f(acc, c) / readlane_f(r[c], c);
-      if (lane == c) acc = xc;
-      else if (lane < c) acc -= r[c] * xc;
-    }
-    if (lane < n) X[(int64_t)p * n + lane] = acc;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Flat Householder for m <= 1024: one 256-thread workgroup per problem, the
-// whole m x 33 [A | b] in registers (thread t holds rows t, t+256, t+512,
-// t+768), one reflector per column over all m rows -- 32 steps per problem
-// instead of the streaming form's 32 per 32 rows.  Per step: sigma and the
-// 33 - K column dot products reduced in the wavefront (recursive halving)
-// and across the four wavefronts through LDS (one barrier each), alpha from
-// the row-K thread through LDS; the update is four rows per thread.  The
-// reflectors are geqr2_panel's (the same dlarfg convention as above), so R
-// and Q^T b are numax's up to rounding.  Rows are loaded coalesced (eight
-// rows per wavefront instruction) and transposed through LDS.
-// ---------------------------------------------------------------------------
-constexpr int kFlatT = 256;               // threads per problem
-constexpr int kFlatR = 4;                 // rows per thread
-constexpr int kFlatMaxM = kFlatT * kFlatR;
-constexpr int kFlatWaves = kFlatT / 64;
-
-struct FlatLds {
-  float stage[64][kCols + 3];    // 64 rows of [A | b] per load round (stride 36: 16-byte aligned)
-  // per step (double-buffered): each wavefront's column sums (sigma last),
-  // then row K's own values
-  float part[2][kFlatWaves + 1][kCols];
-  float alpha[2];
+template <int NW>
+struct GelsLds {
+  float x[NW][4][kGroupPad];                               // the reflector's column, per row group
+  __attribute__((aligned(16))) float part[2][NW][16][2];   // column sums by wavefront (columns c, c + 16)
+  __attribute__((aligned(16))) float part_b[2][NW < 4 ? 4 : NW];
+  float row[2][34];                                        // row K: columns (c, c + 16) interleaved, then b
+  float R[32][33];                                         // written and read by wavefront 0 only
+  float y[32];
 };
 
-template <int K>
-__device__ __forceinline__ void flat_step(float (&r)[kFlatR][kCols], int t, int n, FlatLds& L) {
-  if (K >= n) return;  // uniform
-  constexpr int NJ = kCols - 1 - K;    // columns to the right, b included
-  constexpr int P2 = pow2_at_least(NJ);
-  constexpr int SPREAD = 64 / P2;
-  const int lane = t & 63, wave = t >> 6;
+// Reflector K.  Rows 0 .. K-1 have left the registers (they are zero there
+// and their R is in LDS), so sums over all rows are sums over rows >= K:
+// S = |x|^2 with x the column including row K, beta = -sign(alpha) sqrt(S),
+// and with w = x - beta e_K the reflector is I - w w^T / (beta (beta - alpha));
+// w^T A_j = x^T A_j - beta A_Kj needs only the sums.  beta - alpha has no
+// cancellation.  S = 0 leaves the column (f = 0).
+template <int K, int NW, int SETS>
+__device__ __forceinline__ void gels_step(float (&a)[SETS][kRows], float (&b)[2], int t, GelsLds<NW>& L) {
+  constexpr int set = K >> 4, lk = K & 15;
+  constexpr int s0 = set;  // sets before it hold finished columns only
   constexpr int buf = K & 1;
-  // with x the column below K: sigma = x^T x and u_j = x^T A[:, j] now; the
-  // reflector's v is 1 on row K and x * scale below, so v^T A[:, j] =
-  // A[K][j] + scale * u_j once alpha gives scale
-  float sg = 0.f;
-  float p[P2];
+  // opaque per step: the lane masks built from t are made where they are
+  // used, not hoisted (32 steps of them spilled)
+  asm volatile("" : "+v"(t));
+  const int lane = t & 63, wave = NW == 1 ? 0 : t >> 6;
+  const int c = lane & 15, g = lane >> 4;
+  // b is held two rows a lane: it meets the column through LDS (own wavefront, in order)
+  float* xg = L.x[wave][g];
+  if (c == lk) {
 #pragma unroll
-  for (int q = 0; q < P2; q++) p[q] = 0.f;
+    for (int r = 0; r < kRows; r += 4)
+      *(float4*)(xg + r) = make_float4(a[set][r], a[set][r + 1], a[set][r + 2], a[set][r + 3]);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const float2 xb = *(const float2*)(xg + 2 * c);
+  if (t < 16) {
 #pragma unroll
-  for (int i = 0; i < kFlatR; i++) {
-    const int row = t + kFlatT * i;
-    const float x = row > K ? r[i][K] : 0.f;
-    sg += x * x;
+    for (int s = s0; s < SETS; s++) L.row[buf][2 * c + s] = a[s][K];
+  }
+  if (t == K / 2) L.row[buf][32] = b[K & 1];
+  float p[SETS];
 #pragma unroll
-    for (int j = 0; j < NJ; j++) p[j] += x * r[i][K + 1 + j];
-    if (row == K) {
-      L.alpha[buf] = r[i][K];
+  for (int s = s0; s < SETS; s++) {
+    float q0 = 0.f, q1 = 0.f;
 #pragma unroll
-      for (int j = 0; j < NJ; j++) L.part[buf][kFlatWaves][j] = r[i][K + 1 + j];  // row K's A[K][j]
+    for (int r = 0; r < kRows; r += 2) {
+      q0 = fmaf(row_bcast<lk>(a[set][r]), a[s][r], q0);
+      q1 = fmaf(row_bcast<lk>(a[set][r + 1]), a[s][r + 1], q1);
+    }
+    p[s] = q0 + q1;
+  }
+  float pb = xb.x * b[0] + xb.y * b[1];
+  pb = dpp_add<0xB1>(pb);   // quad_perm 1,0,3,2
+  pb = dpp_add<0x4E>(pb);   // quad_perm 2,3,0,1
+  pb = dpp_add<0x141>(pb);  // row_half_mirror
+  pb = dpp_add<0x140>(pb);  // row_mirror
+  if constexpr (SETS - s0 == 2) {
+    const float v = sum_rows16(sum_halves(p[0], p[1]));
+    if (g == 0 || g == 2) L.part[buf][wave][c][g >> 1] = v;
+  } else {
+    const float v = sum_rows16(sum_halves(p[SETS - 1], p[SETS - 1]));
+    if (g == 0) L.part[buf][wave][c][SETS - 1] = v;
+  }
+  pb = sum_rows16(sum_halves(pb, pb));
+  if (lane == 0) L.part_b[buf][wave] = pb;
+  if (NW == 1) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+  float tot[2] = {0.f, 0.f}, tb = 0.f;
+#pragma unroll(NW < 8 ? NW : 8)
+  for (int w = 0; w < NW; w++) {
+    const float2 v = *(const float2*)L.part[buf][w][c];
+    tot[0] += v.x;
+    tot[1] += v.y;
+    tb += L.part_b[buf][w];
+  }
+  const float2 rk = *(const float2*)&L.row[buf][2 * c];
+  const float bk = L.row[buf][32];
+  const float S = row_bcast<lk>(tot[set]);
+  const float alpha = row_bcast<lk>(set ? rk.y : rk.x);
+  const float beta = -copysignf(sqrtf(S), alpha);
+  const float i0 = S == 0.f ? 0.f : 1.f / beta, i1 = S == 0.f ? 0.f : 1.f / (beta - alpha);
+  const float wk = alpha - beta;
+  float f[SETS];
+#pragma unroll
+  for (int s = s0; s < SETS; s++) {
+    const float rks = s ? rk.y : rk.x;
+    const float fs = (tot[s] - beta * rks) * i0 * i1;
+    f[s] = 16 * s + c > K ? fs : 0.f;  // finished columns and K itself stay
+    if (t < 16) {
+      const int col = 16 * s + c;
+      if (col >= K) L.R[K][col] = col == K ? beta : rks - f[s] * wk;
     }
   }
-  const float tot = halving_sum<P2>(p, lane);
+  const float fb = (tb - beta * bk) * i0 * i1;
+  if (t == 0) L.y[K] = bk - fb * wk;
+  // the other sets first: x is read from its own set's registers
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) sg += __shfl_xor(sg, m);
-  if (lane % SPREAD == 0 && lane / SPREAD < NJ) L.part[buf][wave][lane / SPREAD] = tot;
-  if (lane == 0) L.part[buf][wave][kCols - 1] = sg;
-  __syncthreads();
-  float sigma = 0.f;
+  for (int s = SETS - 1; s >= s0; s--)
 #pragma unroll
-  for (int w = 0; w < kFlatWaves; w++) sigma += L.part[buf][w][kCols - 1];
-  const float alpha = L.alpha[buf];
-  if (sigma == 0.f) return;  // uniform: tau = 0, column K already triangular
-  const float beta = -copysignf(sqrtf(alpha * alpha + sigma), alpha);
-  const float tau = (beta - alpha) / beta;
-  const float scale = 1.f / (alpha - beta);
-  float f[NJ];  // tau * v^T A[:, j]
+    for (int r = 0; r < kRows; r++) a[s][r] = fmaf(row_bcast<lk>(a[set][r]), -f[s], a[s][r]);
+  b[0] -= xb.x * fb;
+  b[1] -= xb.y * fb;
+  // row K is finished
+  if (t < 16) {
 #pragma unroll
-  for (int j = 0; j < NJ; j++) {
-    float u = 0.f;
-#pragma unroll
-    for (int w = 0; w < kFlatWaves; w++) u += L.part[buf][w][j];
-    f[j] = tau * (L.part[buf][kFlatWaves][j] + scale * u);
+    for (int s = s0; s < SETS; s++) a[s][K] = 0.f;
   }
-#pragma unroll
-  for (int i = 0; i < kFlatR; i++) {
-    const int row = t + kFlatT * i;
-    if (row == K) {
-      r[i][K] = beta;
-#pragma unroll
-      for (int j = 0; j < NJ; j++) r[i][K + 1 + j] -= f[j];
-    } else if (row > K) {
-      const float v = r[i][K] * scale;
-#pragma unroll
-      for (int j = 0; j < NJ; j++) r[i][K + 1 + j] -= f[j] * v;
-    }
+  if (t == K / 2) b[K & 1] = 0.f;
+}
+
+template <int K, int NW, int SETS>
+__device__ __forceinline__ void gels_steps(float (&a)[SETS][kRows], float (&b)[2], int t, int n, GelsLds<NW>& L) {
+  if constexpr (K < 16 * SETS) {
+    if (K >= n) return;  // uniform
+    gels_step<K, NW, SETS>(a, b, t, L);
+    gels_steps<K + 1, NW, SETS>(a, b, t, n, L);
   }
 }
 
-template <int K>
-__device__ __forceinline__ void flat_all(float (&r)[kFlatR][kCols], int t, int n, FlatLds& L) {
-  if constexpr (K < 32) {
-    flat_step<K>(r, t, n, L);
-    flat_all<K + 1>(r, t, n, L);
-  }
-}
-
-__global__ void __launch_bounds__(kFlatT) gels_flat_kernel(int count, int m, int n, const float* __restrict__ A,
-                                                           const float* __restrict__ B, float* __restrict__ X) {
-  __shared__ FlatLds L;
-  const int t = threadIdx.x;
+// NW wavefronts hold 128 NW rows at a time; a taller problem goes through in
+// chunks, the triangle and Q^T b of the rows so far as the next chunk's first
+// 32 rows (a sequential TSQR).  SETS: 16-column register sets (n <= 16 SETS).
+template <int NW, int SETS>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)))
+gels_kernel(int count, int m, int n, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ X) {
+  __shared__ GelsLds<NW> L;
+  const int t = threadIdx.x, lane = t & 63;
+  const int grp = t >> 4;  // row group
+  constexpr int kChunk = 128 * NW;
   for (int p = blockIdx.x; p < count; p += gridDim.x) {
-    const float* Ap = A + (int64_t)p * m * n;
-    const float* Bp = B + (int64_t)p * m;
-    float r[kFlatR][kCols];
-    // 64 rows per round: thread t loads element t % 64 .. of rows (t / 64) + 4 k
-    // -- consecutive threads read consecutive elements of the packed problem
+    // rows past m read 0 by the descriptors' range check
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(A + (int64_t)p * m * n), (short)0, 4 * m * n, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B + (int64_t)p * m), (short)0, 4 * m, 0x00020000);
+    float a[SETS][kRows], b[2];
+    int done = 0;  // rows factored so far
+    for (;;) {
+      // row group 0 of a later chunk is the triangle (rows 0..31), the rest new rows
+      const bool tri = done > 0 && grp == 0;
+      int c = lane & 15;
+      asm volatile("" : "+v"(c));  // as in the steps
+      const int row0 = done > 0 ? done + (grp - 1) * kRows : grp * kRows;
+      if (tri) {
 #pragma unroll
-    for (int i = 0; i < kFlatR; i++) {
+        for (int s = 0; s < SETS; s++)
 #pragma unroll
-      for (int round = 0; round < 4; round++) {
-        const int r0 = i * kFlatT + round * 64;  // first row of this round
-        __syncthreads();
-        for (int e = t; e < 64 * n; e += kFlatT) {
-          const int rr = e / n, cc = e % n;
-          L.stage[rr][cc] = r0 + rr < m ? Ap[(int64_t)(r0 + rr) * n + cc] : 0.f;
+          for (int r = 0; r < kRows; r++) {
+            const int col = 16 * s + c;
+            a[s][r] = r <= col && col < n ? L.R[r][col] : 0.f;
+          }
+#pragma unroll
+        for (int i = 0; i < 2; i++) b[i] = 2 * c + i < n ? L.y[2 * c + i] : 0.f;
+      } else {
+#pragma unroll
+        for (int s = 0; s < SETS; s++) {
+          // columns past n start out of range and stay there (a row group's
+          // offsets span 31 n elements, under 4 KB)
+          uint32_t off = 16 * s + c < n ? 4u * ((uint32_t)row0 * (uint32_t)n + (uint32_t)(16 * s + c)) : 0x80000000u;
+#pragma unroll
+          for (int r = 0; r < kRows; r++, off += 4u * (uint32_t)n) a[s][r] = buf_load<float>(ra, off);
         }
-        if (t < 64) L.stage[t][32] = r0 + t < m ? Bp[r0 + t] : 0.f;
-        __syncthreads();
-        if ((t >> 6) == round) {
 #pragma unroll
-          for (int c = 0; c < kCols; c++) r[i][c] = c < n || c == 32 ? L.stage[t & 63][c] : 0.f;
-        }
+        for (int i = 0; i < 2; i++) b[i] = buf_load<float>(rb, 4u * (uint32_t)(row0 + 2 * c + i));
       }
+      gels_steps<0, NW, SETS>(a, b, t, n, L);
+      done += done > 0 ? kChunk - kRows : kChunk;
+      if (done >= m) break;
+      if (NW > 1) __syncthreads();  // the last step's sums are read before the next chunk's first are written
+      else __builtin_amdgcn_wave_barrier();
     }
-    __syncthreads();
-    flat_all<0>(r, t, n, L);
-    // R x = (Q^T b)[0:n] in wavefront 0 (rows 0..31 are its lanes' first rows)
+    // R x = (Q^T b)[0:n] in wavefront 0, a row per lane; the reciprocals of
+    // the diagonal once for all lanes, each quotient corrected by its residual
+    // (a division inside the chain costs four times as much)
     if (t < 64) {
-      float acc = t < n ? r[0][32] : 0.f;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      int i = lane & 31;
+      asm volatile("" : "+v"(i));  // its lane masks are not worth keeping across problems
+      const bool live = i < n;
+      float rr[16 * SETS];
 #pragma unroll
-      for (int c = 31; c >= 0; c--) {
-        if (c < n) {  // uniform
-          const float xc = readlane_f(acc, c) / readlane_f(r[0][c], c);
-          if (t == c) acc = xc;
-          else if (t < c) acc -= r[0][c] * xc;
+      for (int q = 0; q < 16 * SETS; q++) rr[q] = live && q >= i && q < n ? L.R[i][q] : 0.f;
+      float acc = live ? L.y[i] : 0.f;
+      const float diag = live ? L.R[i][i] : 1.f;
+      const float inv = 1.f / diag;
+#pragma unroll
+      for (int q = 16 * SETS - 1; q >= 0; q--) {
+        if (q < n) {  // uniform
+          float v = acc * inv;
+          const float v2 = fmaf(fmaf(-v, diag, acc), inv, v);
+          v = v2 == v2 ? v2 : v;  // a zero diagonal keeps its infinity
+          const float xq = readlane_f(v, q);
+          if (i == q) acc = xq;
+          else if (i < q) acc -= rr[q] * xq;
         }
       }
-      if (t < n) X[(int64_t)p * n + t] = acc;
+      if (lane < n) X[(int64_t)p * n + lane] = acc;
     }
-    __syncthreads();
+    // the next problem's first sums go to the buffer that this one's last
+    // step, when n is odd, may still be reading
+    if (NW > 1) __syncthreads();
   }
+}
+
+template <int NW>
+int gels_launch(nmx_ctx* ctx, int count, int m, int n, const float* A, const float* B, float* X) {
+  // 128 registers a thread: 16 wavefronts of it fit a CU
+  const int grid = std::min(count, ctx->num_cus * (16 / NW));
+  if (n <= 16) gels_kernel<NW, 1><<<grid, 64 * NW, 0, ctx->stream>>>(count, m, n, A, B, X);
+  else gels_kernel<NW, 2><<<grid, 64 * NW, 0, ctx->stream>>>(count, m, n, A, B, X);
+  NMX_HIP(ctx, hipGetLastError());
+  return NMX_OK;
 }
 
 }  // namespace
@@ -288,17 +288,11 @@ NMX_API int nmx_batched_gels_f32(nmx_ctx* ctx, int count, int m, int n, const fl
   if (!X) return -7;
   if ((int64_t)m * n * 4 >= 0x7FFFFFFF) return NMX_ERR_UNSUPPORTED;
   ProfScope ps(ctx, K_TSQR, 0.0, 4.0 * (double)count * ((double)m * n + m + n));
-  if (m <= kFlatMaxM) {
-    // one workgroup per problem, the whole problem in registers
-    const int grid = std::min(count, ctx->num_cus * 16);
-    gels_flat_kernel<<<grid, kFlatT, 0, ctx->stream>>>(count, m, n, A, B, X);
-  } else {
-    // taller problems stream through one wavefront, 32 rows at a time
-    const int waves = 4;
-    int grid = ceil_div(count, waves);
-    if (grid > ctx->num_cus * 8) grid = ctx->num_cus * 8;
-    gels_tsqr_kernel<<<grid, 64 * waves, 0, ctx->stream>>>(count, m, n, A, B, X);
-  }
-  NMX_HIP(ctx, hipGetLastError());
-  return NMX_OK;
+  // the fewest wavefronts that hold the problem (128 rows each): a smaller
+  // workgroup has a shorter step and more problems share a CU
+  if (m <= 128) return gels_launch<1>(ctx, count, m, n, A, B, X);
+  if (m <= 256) return gels_launch<2>(ctx, count, m, n, A, B, X);
+  if (m <= 512) return gels_launch<4>(ctx, count, m, n, A, B, X);
+  if (m <= 1024) return gels_launch<8>(ctx, count, m, n, A, B, X);
+  return gels_launch<16>(ctx, count, m, n, A, B, X);
 }

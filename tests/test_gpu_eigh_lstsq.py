@@ -106,6 +106,35 @@ def test_lstsq_batched_matches_oracle(m, n, count):
         assert np.max(np.abs(a64.T @ r)) <= 1e-3 * np.linalg.norm(a64) * np.linalg.norm(b64)
 
 
+@pytest.mark.parametrize("m,n", [(1, 1), (2, 2), (31, 16), (32, 17), (64, 16), (128, 32), (129, 31), (256, 15),
+                                 (257, 32), (512, 8), (513, 17), (1024, 16), (1025, 32), (2048, 32), (2049, 5),
+                                 (4032, 32), (4033, 31)])
+def test_lstsq_batched_at_the_edges_of_its_row_and_column_tiles(m, n):
+    """128 rows a wavefront, 1 to 16 wavefronts, 16-column register sets, and
+    chunks of 2048 - 32 rows past 2048.  Backward stable, so the solution is
+    within a few m n eps of exact for these well-conditioned problems."""
+    count = 5
+    rng = np.random.default_rng(1000 * m + n)
+    a = rng.standard_normal((count, m, n))
+    if m < 2 * n:  # square or nearly: keep the condition number small
+        a[:, np.arange(n), np.arange(n)] += 2.0 * np.sqrt(m)
+    a = a.astype(np.float32)
+    b = rng.standard_normal((count, m)).astype(np.float32)
+    a[3] = 0.0 if n == 1 else a[3]  # a zero column: non-finite, and only there
+    x = nl.lstsq_batched(a, b).cpu().numpy().astype(np.float64)
+    eps = np.finfo(np.float32).eps
+    for p in range(count):
+        if n == 1 and p == 3:
+            assert not np.isfinite(x[p]).any()
+            continue
+        a64, b64 = a[p].astype(np.float64), b[p].astype(np.float64)
+        xo = np.linalg.lstsq(a64, b64, rcond=None)[0]
+        sv = np.linalg.svd(a64, compute_uv=False)
+        kappa = sv[0] / sv[-1]
+        bound = 4 * n * np.sqrt(m) * eps * kappa * (np.linalg.norm(b64) / sv[-1] + np.linalg.norm(xo))
+        assert np.linalg.norm(x[p] - xo) <= bound, f"problem {p}"
+
+
 def test_lstsq_tall_6x3_known_answer():
     from tests.golden import kat
     g = np.load(__import__("os").path.join(__import__("os").path.dirname(__file__), "golden", "goldens.npz"))
