@@ -14,10 +14,11 @@
 //    A row-major in rows 0 .. n^2 - 1 and b in rows n^2 .. n^2 + n - 1,
 //    answers (n, batch).  Up to n = 8 one thread owns one problem in
 //    registers, as map_blocks' lane does, and neighbouring threads read
-//    neighbouring addresses; larger n use the wavefront kernel with the
-//    batch as element stride.
+//    neighbouring addresses; larger n take a lane per row
+//    (map_blocks_seg.h).
 #include <math.h>
 
+#include "map_blocks_seg.h"
 #include "nmx_internal.h"
 
 // every a - b * c below is a multiply, then a subtraction: numax's loops
@@ -38,53 +39,32 @@ enum SmallOp {
   OP_DET_PIV,          // PivotedLU.det (_array/lu.mojo:112-123)
   OP_SLOGDET,          // slogdet through lu_factor (_array/lu.mojo:125-162, :236-258)
   OP_SLOGDET_CHOL,     // slogdet_cholesky of a factor (_array/cholesky.mojo:95-116)
-  OP_SOLVE_PIV,        // lu_factor + PivotedLU.solve (_array/lu.mojo:92-110, :165-216)
-  OP_SOLVE_CHOL,       // cholesky + cholesky_solve (_array/cholesky.mojo:26-92)
 };
 
 __host__ __device__ constexpr bool op_is_solve(int op) {
-  return op == OP_SOLVE || op == OP_SOLVE_PIV || op == OP_SOLVE_CHOL;
+  return op == OP_SOLVE;
 }
 __host__ __device__ constexpr bool op_is_matrix(int op) { return op == OP_LU || op == OP_INVERSE; }
 
 template <typename T>
 struct SmallArgs {
   int op, count;
-  const int32_t* n;     // orders (row-major layout); nullptr: every problem has order n0 (map_blocks)
-  int n0;
-  const int64_t* offA;  // row-major layout: element offsets of each matrix / vector
+  const int32_t* n;     // orders
+  const int64_t* offA;  // element offsets of each matrix / vector
   const int64_t* offB;
-  int64_t batch;        // map_blocks layout: problems (the element stride)
   int64_t a_elems, b_elems;
-  const T* A;           // matrices (map_blocks: the whole (k_in, batch) array)
-  const T* B;           // right-hand sides (map_blocks: same as A)
+  const T* A;           // matrices
+  const T* B;           // right-hand sides
   T* X;                 // matrix or vector results
   T* s1;                // scalar results
   T* s2;
 };
 
+// Where problem p lives: its order, and the first element of its matrix, its
+// right-hand side and its result.  False: skip it.
 template <typename T>
-__device__ __forceinline__ T guard(T x) {  // guard_nonzero(x, 1e-30), numax/core/numeric.mojo:346-364
-  const T f = (T)1e-30;
-  const T m = fabs(x);
-  return (m >= f || m != m) ? x : copysign(f, x);
-}
-
-// Where problem p lives: its order, and the first element and element
-// stride of its matrix, its right-hand side and its result.  False: skip it.
-template <typename T>
-__device__ __forceinline__ bool locate(const SmallArgs<T>& a, int p, int& n, int64_t& ao, int64_t& bo, int64_t& xo,
-                                       int64_t& es) {
-  if (!a.n) {
-    n = a.n0;
-    es = a.batch;
-    ao = p;
-    bo = (int64_t)n * n * a.batch + p;
-    xo = p;
-    return true;
-  }
+__device__ __forceinline__ bool locate(const SmallArgs<T>& a, int p, int& n, int64_t& ao, int64_t& bo, int64_t& xo) {
   n = a.n[p];
-  es = 1;
   if (n < 1 || n > kSmallMax) return false;
   ao = a.offA[p];
   if (ao < 0 || ao + (int64_t)n * n > a.a_elems) return false;
@@ -164,22 +144,6 @@ __device__ int lds_lu_piv(T* M, T* v, int n, int lane) {
   return sign;
 }
 
-// cholesky (_array/cholesky.mojo:26-58), left-looking, in place in the lower
-// triangle (the upper is left as read; nothing below reads it).
-template <typename T>
-__device__ void lds_cholesky(T* M, int n, int lane) {
-  for (int j = 0; j < n; j++) {
-    T acc = (lane >= j && lane < n) ? M[lane * kLd + j] : (T)0;
-    if (lane >= j && lane < n)
-      for (int k = 0; k < j; k++) acc = acc - M[lane * kLd + k] * M[j * kLd + k];
-    if (lane == j) M[j * kLd + j] = sqrt(guard(acc));
-    __syncthreads();
-    const T ljj = M[j * kLd + j];
-    if (lane > j && lane < n) M[lane * kLd + j] = acc / ljj;
-    __syncthreads();
-  }
-}
-
 // forward_substitution (_array/triangular.mojo:24-43) of the vector in v,
 // in place: row i subtracts l_ij x_j for j = 0 .. i-1 in that order, which
 // the column sweep keeps (lane i accumulates row i's total as x_j appear).
@@ -219,33 +183,21 @@ __global__ void __launch_bounds__(64) small_wave_kernel(SmallArgs<T> a) {
   const int lane = threadIdx.x;
   for (int p = blockIdx.x; p < a.count; p += gridDim.x) {
     int n;
-    int64_t ao, bo, xo, es;
-    if (!locate(a, p, n, ao, bo, xo, es)) continue;
-    for (int e = lane; e < n * n; e += 64) M[(e / n) * kLd + e % n] = a.A[ao + e * es];
-    if (op_is_solve(a.op) && lane < n) V[lane] = a.B[bo + lane * es];
+    int64_t ao, bo, xo;
+    if (!locate(a, p, n, ao, bo, xo)) continue;
+    for (int e = lane; e < n * n; e += 64) M[(e / n) * kLd + e % n] = a.A[ao + e];
+    if (op_is_solve(a.op) && lane < n) V[lane] = a.B[bo + lane];
     __syncthreads();
     switch (a.op) {
       case OP_LU:
         lds_lu(M, n, lane);
-        for (int e = lane; e < n * n; e += 64) a.X[xo + e * es] = M[(e / n) * kLd + e % n];
+        for (int e = lane; e < n * n; e += 64) a.X[xo + e] = M[(e / n) * kLd + e % n];
         break;
       case OP_SOLVE:
         lds_lu(M, n, lane);
         lds_forward(M, V, n, lane, true);
         lds_back<T, false>(M, V, n, lane);
-        if (lane < n) a.X[xo + lane * es] = V[lane];
-        break;
-      case OP_SOLVE_PIV:
-        lds_lu_piv(M, V, n, lane);
-        lds_forward(M, V, n, lane, true);
-        lds_back<T, false>(M, V, n, lane);
-        if (lane < n) a.X[xo + lane * es] = V[lane];
-        break;
-      case OP_SOLVE_CHOL:
-        lds_cholesky(M, n, lane);
-        lds_forward(M, V, n, lane, false);
-        lds_back<T, true>(M, V, n, lane);
-        if (lane < n) a.X[xo + lane * es] = V[lane];
+        if (lane < n) a.X[xo + lane] = V[lane];
         break;
       case OP_INVERSE:
         if constexpr (INV) {
@@ -267,7 +219,7 @@ __global__ void __launch_bounds__(64) small_wave_kernel(SmallArgs<T> a) {
             }
           }
           __syncthreads();
-          for (int e = lane; e < n * n; e += 64) a.X[xo + e * es] = V[(e % n) * kLd + e / n];
+          for (int e = lane; e < n * n; e += 64) a.X[xo + e] = V[(e % n) * kLd + e / n];
         }
         break;
       case OP_DET:
@@ -462,7 +414,7 @@ int small_rowmajor(nmx_ctx* ctx, int op, int count, const int32_t* n, const int6
   if ((op_is_solve(op) || op_is_matrix(op)) && !X) return -7;
   if (!op_is_solve(op) && !op_is_matrix(op) && !s1) return -8;
   if (op == OP_SLOGDET && !s2) return -9;
-  SmallArgs<double> a{op, count, n, 0, offA, offB, 0, a_elems, b_elems, A, B, X, s1, s2};
+  SmallArgs<double> a{op, count, n, offA, offB, a_elems, b_elems, A, B, X, s1, s2};
   return small_launch<double>(ctx, a);
 }
 
@@ -489,9 +441,8 @@ int map_blocks_api(nmx_ctx* ctx, int kind, int n, int64_t batch, const T* xs, T*
     }
   }
   if (batch > INT32_MAX) return -4;
-  const int op = kind == 0 ? OP_SOLVE_PIV : kind == 1 ? OP_SOLVE_CHOL : OP_SOLVE;
-  SmallArgs<T> a{op, (int)batch, nullptr, n, nullptr, nullptr, batch, 0, 0, xs, xs, ys, nullptr, nullptr};
-  return small_launch<T>(ctx, a);
+  ProfScope ps(ctx, K_BATCH, 0.0, 0.0);
+  return map_blocks_seg(ctx, kind, n, batch, xs, ys);
 }
 
 }  // namespace

@@ -144,6 +144,30 @@ def test_map_blocks_solve_f64_bit_exact(n, kind):
         np.testing.assert_array_equal(ys[:, p], _oracle_step(kind, mats[p], rhss[p]), err_msg=f"{kind} n={n} p={p}")
 
 
+@pytest.mark.parametrize("n,batch", [(9, 1), (15, 17), (16, 16), (17, 15), (24, 33), (25, 16), (31, 5), (32, 31),
+                                     (33, 8), (47, 9), (48, 7), (49, 17), (63, 1), (64, 23)])
+def test_map_blocks_lane_per_row_edges_bit_exact(n, batch):
+    """The padded orders' edges, batches that are no multiple of a workgroup's
+    problems, and matrices of small integers: tied pivots, zero pivots and a
+    zero column, whose infinities and NaNs must land where numax's do."""
+    rng = np.random.default_rng(7 * n + batch)
+    for kind in ("lu", "cholesky", "nopivot"):
+        mats = []
+        for p in range(batch):
+            if kind == "cholesky":
+                mats.append(_spd(rng, n))
+                continue
+            m = rng.integers(-2, 3, (n, n)).astype(np.float64)
+            if p % 3 == 2:
+                m[:, rng.integers(0, n)] = 0.0
+            mats.append(m)
+        rhss = [rng.standard_normal(n) for _ in range(batch)]
+        ys = nl.map_blocks_solve(_soa(mats, rhss), n, kind).cpu().numpy()
+        for p in range(batch):
+            np.testing.assert_array_equal(ys[:, p], _oracle_step(kind, mats[p], rhss[p]),
+                                          err_msg=f"{kind} n={n} p={p}")
+
+
 def test_map_blocks_known_answer():
     """tests/core/test_map_blocks.mojo:192-218: one Array-tier solve per lane
     over the hashed SPD batch agrees with the host solve at 1e-12."""
