@@ -22,6 +22,16 @@
 // registers (NP = 32 packs two matrices per wavefront, NP = 64 one); rows
 // are register indices.  A matrix of order n < NP is padded with zero rows
 // and columns, which only ever rotate by exact exchanges (a_pq = 0).
+//
+// What bounds it: vector issue, about 640 instructions a step of a 64-wide
+// wavefront (192 for the rows of A, 320 for the columns of A and V, 90 for
+// the rotation, 32 to pick a_pq).  A pair's lanes are neighbours, so the
+// other lane's entry is a DPP operand of the multiply (quad_perm on even
+// steps, wave_shl / wave_shr on odd ones) and the rotations reach the rows as
+// broadcast LDS reads.  As lane shuffles through LDS, two a register row plus
+// two a rotation, they bound the kernel: 65,536 matrices of order 24 to 64
+// took 77.8 ms; they take 25.5 ms now, with the
+// same eigenvalues bit for bit.
 #include <math.h>
 
 #include "nmx_internal.h"
@@ -35,69 +45,144 @@ __device__ __forceinline__ float guard_f(float x) {
   return (m >= kFloorF || m != m) ? x : copysignf(kFloorF, x);
 }
 
-// (m ? a : b) for a wave-uniform 64-bit mask, as an opaque v_cndmask (a plain
-// ?: between two register-array elements can be folded into an indexed load,
-// which would move the array to scratch memory).
-__device__ __forceinline__ float sel_m(uint64_t m, float a, float b) {
-  float r;
-  asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(b), "v"(a), "s"(m));
-  return r;
+// v of the lane `CTRL` names (a DPP control; folds into the consuming instruction)
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+constexpr int kSwapPairs = 0xB1;  // quad_perm 1,0,3,2: lane ^ 1
+constexpr int kFromNext = 0x130;  // wave_shl:1: lane + 1
+constexpr int kFromPrev = 0x138;  // wave_shr:1: lane - 1
+
+// x of the pair's other lane (OFF = 0: lane ^ 1; OFF = 1: lane + 1 on a first
+// lane, lane - 1 on a second; lanes without a pair get any value)
+template <int OFF>
+__device__ __forceinline__ float other(float x, bool isP) {
+  if constexpr (OFF == 0) return dpp<kSwapPairs>(x);
+  // both on every lane: a DPP move reads lanes a branch would have turned off
+  const float next = dpp<kFromNext>(x), prev = dpp<kFromPrev>(x);
+  return isP ? next : prev;
 }
 
-// reg[idx(lane)] where idx's bit b is set exactly on the lanes of mask m[b]:
-// a select tree whose masks are constants of the lane pattern.
-template <int NP>
-__device__ __forceinline__ float pick_lane(const float (&r)[NP], const uint64_t (&m)[6]) {
-  float a[32], b[16], c[8], d[4], e[2];
-  if constexpr (NP == 64) {
-#pragma unroll
-    for (int i = 0; i < 32; i++) a[i] = sel_m(m[0], r[2 * i + 1], r[2 * i]);
-#pragma unroll
-    for (int i = 0; i < 16; i++) b[i] = sel_m(m[1], a[2 * i + 1], a[2 * i]);
-#pragma unroll
-    for (int i = 0; i < 8; i++) c[i] = sel_m(m[2], b[2 * i + 1], b[2 * i]);
-#pragma unroll
-    for (int i = 0; i < 4; i++) d[i] = sel_m(m[3], c[2 * i + 1], c[2 * i]);
-#pragma unroll
-    for (int i = 0; i < 2; i++) e[i] = sel_m(m[4], d[2 * i + 1], d[2 * i]);
-    return sel_m(m[5], e[1], e[0]);
+// a[L+1] on every first lane L of a pair (lanes L = OFF, OFF+2, ... of each
+// segment): the two candidates of each quad by lane parity, then the quads
+// merged by bank-masked moves.
+template <int NP, int OFF, int G = 0>
+__device__ __forceinline__ float pick_next(const float (&a)[NP], bool upper, float x) {
+  if constexpr (4 * G < NP) {
+    constexpr int r0 = 4 * G + 1 + OFF, r1 = 4 * G + 3 + OFF;  // a[L+1] of the quad's two first lanes
+    const float lo = a[r0], hi = a[r1 < NP ? r1 : NP - 1];
+    const float cand = upper ? hi : lo;
+    constexpr int row = G / 4;  // 16-lane row; with 32-lane segments the other segment's too
+    constexpr int rows = NP == 64 ? 1 << row : (1 << row) | (1 << (row + 2));
+    x = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(cand), 0xE4, rows, 1 << (G % 4), false));
+    return pick_next<NP, OFF, G + 1>(a, upper, x);
   } else {
-#pragma unroll
-    for (int i = 0; i < 16; i++) b[i] = sel_m(m[0], r[2 * i + 1], r[2 * i]);
-#pragma unroll
-    for (int i = 0; i < 8; i++) c[i] = sel_m(m[1], b[2 * i + 1], b[2 * i]);
-#pragma unroll
-    for (int i = 0; i < 4; i++) d[i] = sel_m(m[2], c[2 * i + 1], c[2 * i]);
-#pragma unroll
-    for (int i = 0; i < 2; i++) e[i] = sel_m(m[3], d[2 * i + 1], d[2 * i]);
-    (void)a;
-    return sel_m(m[4], e[1], e[0]);
+    return x;
   }
 }
 
-// One step of the ordering: rotate the pairs (OFF, OFF+1), (OFF+2, OFF+3),
-// ... of every segment, exchanging the two indices of each pair.
+// x := alpha x + beta (the pair's other lane's x) for four registers, the
+// second product rounded first.  OFF = 1 adds both neighbours' products, one
+// of which has a zero coefficient.  Written out because the compiler folds
+// no DPP move into the second multiply-add; s_nop 1 gives the two wait states
+// between a vector write and a DPP read of the same register.
+template <int OFF>
+__device__ __forceinline__ void rotate_col4(float& x0, float& x1, float& x2, float& x3, float alpha, float beta,
+                                            float beta_next, float beta_prev) {
+  float t0, t1, t2, t3;
+  if constexpr (OFF == 0) {
+    asm volatile(
+        "s_nop 1\n"
+        "v_mul_f32_dpp %4, %0, %9 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %5, %1, %9 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %6, %2, %9 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %7, %3, %9 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_fma_f32 %0, %8, %0, %4\n"
+        "v_fma_f32 %1, %8, %1, %5\n"
+        "v_fma_f32 %2, %8, %2, %6\n"
+        "v_fma_f32 %3, %8, %3, %7\n"
+        : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
+        : "v"(alpha), "v"(beta));
+  } else {
+    asm volatile(
+        "s_nop 1\n"
+        "v_mul_f32_dpp %4, %0, %10 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n"
+        "v_mul_f32_dpp %5, %1, %10 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n"
+        "v_mul_f32_dpp %6, %2, %10 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n"
+        "v_mul_f32_dpp %7, %3, %10 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n"
+        "v_fmac_f32_dpp %4, %0, %9 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n"
+        "v_fmac_f32_dpp %5, %1, %9 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n"
+        "v_fmac_f32_dpp %6, %2, %9 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n"
+        "v_fmac_f32_dpp %7, %3, %9 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n"
+        "v_fma_f32 %0, %8, %0, %4\n"
+        "v_fma_f32 %1, %8, %1, %5\n"
+        "v_fma_f32 %2, %8, %2, %6\n"
+        "v_fma_f32 %3, %8, %3, %7\n"
+        : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
+        : "v"(alpha), "v"(beta_next), "v"(beta_prev));
+  }
+}
+
+// A rotated and exchanged pair of rows (r, r + 1): p = s x + c y, q = c x - s y.
+// Which product is rounded first is written out, here and above: equal
+// diagonals rotate by the sign of a rounding error, so the order in which the
+// eigenvalues come out follows it.  The six pairs that round c y first keep
+// the order these results have had since the kernel's first build.
 template <int NP, int OFF>
-__device__ __forceinline__ void jacobi_step(float (&a)[NP], float (&v)[NP], float& d, int& player, int lane, int L,
-                                            int base, const uint64_t (&mnext)[6]) {
-  const bool isP = (((L - OFF) & 1) == 0) && (L >= OFF) && (L + 1 < NP);
-  const bool isQ = (((L - OFF) & 1) == 1) && (L >= 1 + OFF);
-  const int partner = isP ? lane + 1 : (isQ ? lane - 1 : lane);
+__device__ __forceinline__ void rotate_row(int r, float& p, float& q, float x, float y, float c, float s) {
+  const bool cy_first = NP == 64 && OFF == 1 && r >= 13 && r <= 23;
+  p = cy_first ? __builtin_fmaf(s, x, c * y) : __builtin_fmaf(c, y, s * x);
+  q = __builtin_fmaf(c, x, -(s * y));
+}
+
+// The columns of V, eight rows at a time while they hold rows below nmax
+// (uniform).  Recursive, so that every register index is a constant early.
+template <int NP, int OFF, int I0>
+__device__ __forceinline__ void rotate_rows(float (&v)[NP], int nmax, float alpha, float beta, float beta_next,
+                                            float beta_prev) {
+  if constexpr (I0 < NP) {
+    if (I0 < nmax) {
+#pragma unroll
+      for (int i = I0; i < I0 + 8; i += 4)
+        rotate_col4<OFF>(v[i], v[i + 1], v[i + 2], v[i + 3], alpha, beta, beta_next, beta_prev);
+    }
+    rotate_rows<NP, OFF, I0 + 8>(v, nmax, alpha, beta, beta_next, beta_prev);
+  }
+}
+
+// LDS written by some lanes of a wavefront is read by the others of it
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// One step of the ordering: rotate the pairs (OFF, OFF+1), (OFF+2, OFF+3),
+// ... of every segment, exchanging the two indices of each pair.  cs: this
+// segment's NP/2 rotations in LDS.
+template <int NP, int OFF>
+__device__ __forceinline__ void jacobi_step(float (&a)[NP], float (&v)[NP], float& d, int& player, int L, int nmax,
+                                            float2* cs) {
+  const bool odd = L & 1;
+  const bool isP = OFF == 0 ? !odd : (odd && L + 1 < NP);
+  const bool isQ = OFF == 0 ? odd : (!odd && L >= 1);
   // the pair's rotation, computed on its first lane (_array/eigen.mojo:34-75)
-  const float apq_own = pick_lane<NP>(a, mnext);  // a[L+1][L]: a_pq on a first lane
-  const float d_next = __shfl(d, lane + 1 < 64 ? lane + 1 : lane);
+  const float apq_own = pick_next<NP, OFF>(a, L & 2, 0.f);  // a[L+1][L]: a_pq on a first lane
+  const float d_next = OFF == 0 ? dpp<kSwapPairs>(d) : dpp<kFromNext>(d);
   float c, s, t;
   {
     const float twice = 2.f * apq_own;
     const float den = d_next - d;
-    const float radius = sqrtf(den * den + twice * twice);
+    const float radius = sqrtf(__builtin_fmaf(twice, twice, den * den));
     const float safe = guard_f(fabsf(den) + radius);
     t = copysignf(1.f, den) * twice / safe;
-    c = 1.f / sqrtf(1.f + t * t);
+    c = 1.f / sqrtf(__builtin_fmaf(t, t, 1.f));
     s = t * c;
   }
-  const float c_o = __shfl(c, partner), s_o = __shfl(s, partner), t_o = __shfl(t, partner);
-  const float apq_o = __shfl(apq_own, partner), d_o = __shfl(d, partner);
+  if (isP) cs[L >> 1] = make_float2(c, s);
+  wave_lds_order();
+  const float c_o = other<OFF>(c, isP), s_o = other<OFF>(s, isP), t_o = other<OFF>(t, isP);
+  const float apq_o = other<OFF>(apq_own, isP), d_o = other<OFF>(d, isP);
   if (isQ) {
     c = c_o;
     s = s_o;
@@ -105,27 +190,34 @@ __device__ __forceinline__ void jacobi_step(float (&a)[NP], float (&v)[NP], floa
   }
   const float apq = isQ ? apq_o : apq_own;
   // diagonal after the rotation and the exchange
-  const float d_new = isP ? d_next + t * apq : (isQ ? d_o - t * apq : d);
-  // rows: register pairs (r, r+1), r = OFF, OFF+2, ... (every column)
+  const float d_new = isP || isQ ? __builtin_fmaf(isP ? t : -t, apq, isP ? d_next : d_o) : d;
+  // rows: register pairs (r, r+1), r = OFF, OFF+2, ... (every column); the
+  // rotations come two pairs to a broadcast LDS read
 #pragma unroll
-  for (int r = OFF; r + 1 < NP; r += 2) {
-    const float cr = __shfl(c, base + r), sr = __shfl(s, base + r);
-    const float x = a[r], y = a[r + 1];
-    a[r] = sr * x + cr * y;
-    a[r + 1] = cr * x - sr * y;
+  for (int r = OFF; r + 1 < NP; r += 4) {
+    const float4 w = *(const float4*)(cs + (r >> 1));  // c, s of pairs r and r + 2
+    {
+      const float x = a[r], y = a[r + 1];
+      rotate_row<NP, OFF>(r, a[r], a[r + 1], x, y, w.x, w.y);
+    }
+    if (r + 3 < NP) {
+      const float x = a[r + 2 < NP ? r + 2 : 0], y = a[r + 3 < NP ? r + 3 : 0];
+      rotate_row<NP, OFF>(r + 2, a[r + 2 < NP ? r + 2 : 0], a[r + 3 < NP ? r + 3 : 0], x, y, w.z, w.w);
+    }
   }
+  wave_lds_order();
   // columns of A and V (with the exchange): new = alpha own + beta partner's
   const float alpha = isP ? s : (isQ ? -s : 1.f);
   const float beta = (isP || isQ) ? c : 0.f;
+  const float beta_next = isP ? c : 0.f, beta_prev = isQ ? c : 0.f;
 #pragma unroll
-  for (int i = 0; i < NP; i++) {
-    const float oa = __shfl(a[i], partner);
-    const float ov = __shfl(v[i], partner);
-    a[i] = alpha * a[i] + beta * oa;
-    v[i] = alpha * v[i] + beta * ov;
-  }
+  for (int i = 0; i < NP; i += 4)
+    rotate_col4<OFF>(a[i], a[i + 1], a[i + 2], a[i + 3], alpha, beta, beta_next, beta_prev);
+  // V's rows past the matrix's order are never read
+  rotate_rows<NP, OFF, 0>(v, nmax, alpha, beta, beta_next, beta_prev);
   d = d_new;
-  player = __shfl(player, partner);
+  const int player_o = __float_as_int(other<OFF>(__int_as_float(player), isP));
+  player = isP || isQ ? player_o : player;
 }
 
 struct EighArgs {
@@ -143,22 +235,15 @@ struct EighArgs {
 };
 
 template <int NP>
-__global__ void __launch_bounds__(256) syevj_kernel(EighArgs args, int cls) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NP == 64 ? 2 : 4)))
+syevj_kernel(EighArgs args, int cls) {
   constexpr int PPW = 64 / NP;  // matrices per wavefront
+  __shared__ __attribute__((aligned(16))) float2 rot[256 / NP][NP / 2];
   const int lane = threadIdx.x & 63;
   const int L = lane & (NP - 1);       // slot within the segment
-  const int base = lane & ~(NP - 1);   // first lane of the segment
+  float2* cs = rot[threadIdx.x / NP];
   const int seg = lane / NP;
   const int begin = args.cls[2 * cls], count = args.cls[2 * cls + 1];
-
-  // masks of the lanes whose (L + 1) mod NP has bit b set (for a_{L,L+1})
-  // and whose L has bit b set (for the initial diagonal)
-  uint64_t mnext[6], mself[6];
-#pragma unroll
-  for (int b = 0; b < 6; b++) {
-    mnext[b] = __ballot((((L + 1) & (NP - 1)) >> b) & 1);
-    mself[b] = __ballot((L >> b) & 1);
-  }
 
   for (;;) {
     int slot0 = 0;
@@ -170,22 +255,22 @@ __global__ void __launch_bounds__(256) syevj_kernel(EighArgs args, int cls) {
     const int p = live ? args.order[begin + slot] : 0;
     const int n = live ? args.n[p] : 0;
     const float* A = args.A + (live ? args.offA[p] : 0);
-    (void)seg;
-
+    // V rows a wavefront needs: the larger of its matrices' orders
+    const int nmax = NP == 64 ? n : max(n, __shfl_xor(n, 32));
     float a[NP], v[NP];
 #pragma unroll
     for (int i = 0; i < NP; i++) {
       a[i] = (i < n && L < n) ? A[(int64_t)i * n + L] : 0.f;
       v[i] = (i == L) ? 1.f : 0.f;
     }
-    float d = pick_lane<NP>(a, mself);
+    float d = L < n ? A[(int64_t)L * n + L] : 0.f;
     int player = L;
 
     for (int sw = 0; sw < args.sweeps; sw++) {
 #pragma unroll 1
       for (int step = 0; step < NP; step += 2) {
-        jacobi_step<NP, 0>(a, v, d, player, lane, L, base, mnext);
-        jacobi_step<NP, 1>(a, v, d, player, lane, L, base, mnext);
+        jacobi_step<NP, 0>(a, v, d, player, L, __builtin_amdgcn_readfirstlane(nmax), cs);
+        jacobi_step<NP, 1>(a, v, d, player, L, __builtin_amdgcn_readfirstlane(nmax), cs);
       }
     }
     // padding players (>= n) only ever exchanged; each real player's value
