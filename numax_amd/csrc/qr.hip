@@ -13,6 +13,9 @@
 // reductions (shuffles within a wavefront, LDS across them).  T is built
 // from the Gram matrix V^T V, itself one GEMM of an explicit V (unit
 // diagonal, zeros above), which the three block-reflector products use too.
+// Panels of at most 16 columns, numax's default width, take two launches each
+// instead: a register panel that leaves T too, and one fused application.
+// lstsq of 2500 x 300 FP32: 21.3 ms -> 1.8 ms.
 #include <math.h>
 
 #include "nmx_internal.h"
@@ -226,8 +229,405 @@ int apply_reflector(nmx_ctx* ctx, const Reflector<T>& w, int rows, int nb, int w
   return gemm_launch<T>(ctx, 0, 0, rows, width, nb, T(-1), w.V, nb, w.Y, width, T(1), C, ldc);
 }
 
+// ---- panels of at most 16 columns (numax's default width) --------------------
+//
+// The panel in registers: a thread holds R rows of one column (c = lane % 16),
+// so the reflector's column reaches the other columns of its rows as a DPP
+// broadcast inside a 16-lane row, and one value per column crosses the row
+// groups of a step.  What bounds it is the chain of steps (two sums' worth of
+// multiply-adds, one LDS round and barrier, a root and two divisions); the
+// streaming kernel above walked the panel in memory three times a column.
+// 2500 x 16 FP32: 627 us -> 41 us.  T comes with it: a step's sums over the
+// finished columns are the V^T v_K that larft_panel (panel.mojo:2076-2169)
+// builds it from.
+constexpr int kNarrow = 16;
+
+template <int L>
+__device__ __forceinline__ float row_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + L, 0xF, 0xF, true));
+}
+template <int L>
+__device__ __forceinline__ double row_bcast(double v) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, 0x150 + L, 0xF, 0xF, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), 0x150 + L, 0xF, 0xF, true);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// acc += x(lane K of the 16-lane row) * y for four registers, the broadcast as
+// the multiply-add's DPP operand (the compiler makes a move of it, which would
+// double the instructions and keep R broadcast values live).  s_nop 1: the two
+// wait states between a vector write and a DPP read of the same register.
+#define NMX_FMAC_DPP4(TYPE, D0, D1, D2, D3, X0, X1, X2, X3, S0, S1, S2, S3, CONS)                                  \
+  asm volatile("s_nop 1\n"                                                                                         \
+               "v_fmac_" TYPE "_dpp %0, %4, %8 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                      \
+               "v_fmac_" TYPE "_dpp %1, %5, %9 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                      \
+               "v_fmac_" TYPE "_dpp %2, %6, %10 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                     \
+               "v_fmac_" TYPE "_dpp %3, %7, %11 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                     \
+               : "+v"(D0), "+v"(D1), "+v"(D2), "+v"(D3)                                                            \
+               : "v"(X0), "v"(X1), "v"(X2), "v"(X3), "v"(S0), "v"(S1), "v"(S2), "v"(S3), "n"(CONS))
+template <int K>
+__device__ __forceinline__ void fmac_bcast4(float& d0, float& d1, float& d2, float& d3, float x0, float x1, float x2,
+                                            float x3, float s0, float s1, float s2, float s3) {
+  NMX_FMAC_DPP4("f32", d0, d1, d2, d3, x0, x1, x2, x3, s0, s1, s2, s3, K);
+}
+template <int K>
+__device__ __forceinline__ void fmac_bcast4(double& d0, double& d1, double& d2, double& d3, double x0, double x1,
+                                            double x2, double x3, double s0, double s1, double s2, double s3) {
+  NMX_FMAC_DPP4("f64", d0, d1, d2, d3, x0, x1, x2, x3, s0, s1, s2, s3, K);
+}
+// x -= x(lane K) * s in place, four registers
+#define NMX_FMAC_DPP4_SELF(TYPE, X0, X1, X2, X3, S, CONS)                                     \
+  asm volatile("s_nop 1\n"                                                                    \
+               "v_fmac_" TYPE "_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
+               "v_fmac_" TYPE "_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
+               "v_fmac_" TYPE "_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
+               "v_fmac_" TYPE "_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
+               : "+v"(X0), "+v"(X1), "+v"(X2), "+v"(X3)                                       \
+               : "v"(S), "n"(CONS))
+template <int K>
+__device__ __forceinline__ void fmac_self4(float& x0, float& x1, float& x2, float& x3, float s) {
+  NMX_FMAC_DPP4_SELF("f32", x0, x1, x2, x3, s, K);
+}
+template <int K>
+__device__ __forceinline__ void fmac_self4(double& x0, double& x1, double& x2, double& x3, double s) {
+  NMX_FMAC_DPP4_SELF("f64", x0, x1, x2, x3, s, K);
+}
+
+template <typename T, int NW>
+struct PanelLds {
+  T part[2][NW][kNarrow];  // column sums by wavefront
+  T row[2][kNarrow];       // row K of the panel
+  T G[kNarrow][kNarrow];   // G[K][c] = v_c^T v_K, c < K
+  T tau[kNarrow];
+};
+
+// Reflector K: x = column K below its diagonal, sigma = x^T x, and for every
+// later column A_c -= tau (A_Kc + scale x^T A_c) [1; scale x] -- geqr2_panel's
+// dlarfg convention.  Row K leaves the registers (zero there) before the sums,
+// so sums over all rows are sums below the diagonal.  x stays unscaled in the
+// registers; lane K keeps the column's scale in `sc`.
+template <int K, typename T, int R, int NW>
+__device__ __forceinline__ void panel_step(T (&a)[R], T& sc, int t, int nb, T* __restrict__ A, int lda,
+                                           T* __restrict__ tau, PanelLds<T, NW>& L) {
+  constexpr int buf = K & 1;
+  asm volatile("" : "+v"(t));  // the lane masks below are made here, not kept over the steps
+  const int lane = t & 63, wave = t >> 6, c = lane & 15;
+  if (t < kNarrow) {
+    L.row[buf][c] = a[K] * sc;
+    a[K] = T(0);
+  }
+  T p0 = 0, p1 = 0, p2 = 0, p3 = 0;
+#pragma unroll
+  for (int r = 0; r < R; r += 4)
+    fmac_bcast4<K>(p0, p1, p2, p3, a[r], a[r + 1], a[r + 2], a[r + 3], a[r], a[r + 1], a[r + 2], a[r + 3]);
+  T p = (p0 + p1) + (p2 + p3);
+  p += __shfl_xor(p, 16);
+  p += __shfl_xor(p, 32);
+  if (lane < kNarrow) L.part[buf][wave][c] = p;
+  __syncthreads();
+  T tot = 0;
+#pragma unroll
+  for (int w = 0; w < NW; w++) tot += L.part[buf][w][c];
+  const T rk = L.row[buf][c];
+  const T sigma = row_bcast<K>(tot), alpha = row_bcast<K>(rk);
+  T beta = sqrt(alpha * alpha + sigma);
+  if (alpha > T(0)) beta = -beta;
+  const bool none = sigma == T(0);
+  const T tj = none ? T(0) : (beta - alpha) / beta;
+  const T scale = none ? T(0) : T(1) / (alpha - beta);
+  const T g = rk + scale * tot * sc;            // v_K^T A_c; for finished columns v_K^T v_c
+  const T f = c > K ? tj * g : T(0);
+  const T nfs = -(f * scale);
+  if (c == K && !none) sc = scale;
+  if (c >= K) {  // lane K, which the products read, is among them; its own is 0
+#pragma unroll
+    for (int r = 0; r < R; r += 4) fmac_self4<K>(a[r], a[r + 1], a[r + 2], a[r + 3], nfs);
+  }
+  if (t < kNarrow) {
+    if (c < K) L.G[K][c] = g;
+    // row K of the result: V left of the diagonal, R from it on
+    if (c < nb) A[(int64_t)K * lda + c] = c == K ? (none ? alpha : beta) : rk - f;
+    if (c == K) {
+      tau[K] = tj;
+      L.tau[K] = tj;
+    }
+  }
+}
+
+// T (16 x 16, row-major) by lanes 0..15 of a wavefront, lane r row r:
+// T_ii = tau_i, T[0:i, i] = -tau_i T[0:i, 0:i] (V^T v_i).
+template <typename T>
+__device__ __forceinline__ void narrow_t(int nb, const T (&G)[kNarrow][kNarrow], const T* tau, int r, T* out) {
+  T row[kNarrow];
+#pragma unroll
+  for (int i = 0; i < kNarrow; i++) {
+    T s = 0;
+#pragma unroll
+    for (int q = 0; q < i; q++) s += row[q] * G[i][q];  // row[q] = 0 left of the diagonal
+    const T ti = i < nb ? tau[i] : T(0);
+    row[i] = i >= nb || i < r ? T(0) : (i == r ? ti : -ti * s);
+  }
+#pragma unroll
+  for (int i = 0; i < kNarrow; i++) out[r * kNarrow + i] = row[i];
+}
+
+template <int K, typename T, int R, int NW>
+__device__ __forceinline__ void panel_steps(T (&a)[R], T& sc, int t, int nb, T* A, int lda, T* tau, PanelLds<T, NW>& L) {
+  if constexpr (K < kNarrow) {
+    if (K < nb) panel_step<K, T, R, NW>(a, sc, t, nb, A, lda, tau, L);  // uniform
+    panel_steps<K + 1, T, R, NW>(a, sc, t, nb, A, lda, tau, L);
+  }
+}
+
+// A: the panel's top left corner, rows x nb with rows <= 4 NW R.
+template <typename T, int R, int NW>
+__global__ void __launch_bounds__(64 * NW) geqr2_narrow_kernel(int rows, int nb, T* __restrict__ A, int lda,
+                                                               T* __restrict__ tau, T* __restrict__ Tout) {
+  __shared__ PanelLds<T, NW> L;
+  const int t = threadIdx.x, c = t & 15, row0 = (t >> 4) * R;
+  T a[R];
+  const T* src = A + (int64_t)row0 * lda + c;
+#pragma unroll
+  for (int r = 0; r < R; r++) a[r] = (row0 + r < rows) & (c < nb) ? src[(int64_t)r * lda] : T(0);
+  if (t < kNarrow)
+    for (int i = 0; i < kNarrow; i++) L.G[t][i] = T(0);
+  __syncthreads();  // and every load is done before row 0 is stored
+  T sc = T(1);  // a finished column's reflector is its x times this
+  panel_steps<0, T, R, NW>(a, sc, t, nb, A, lda, tau, L);
+  T* dst = A + (int64_t)row0 * lda + c;
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if ((row0 + r < rows) & (c < nb) & (row0 + r >= nb)) dst[(int64_t)r * lda] = a[r] * sc;
+  if (t < kNarrow) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    narrow_t<T>(nb, L.G, L.tau, t, Tout);
+  }
+}
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+// 16 x 16 += 16 x 4 by 4 x 16: operands by (lane % 16, lane / 16), output item e
+// of lane l in row acc_row(l, e), column l % 16
+__device__ __forceinline__ d4 mma16(double a, double b, d4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f4 mma16(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+template <typename T>
+__device__ __forceinline__ int acc_row(int lane, int e) {
+  return sizeof(T) == 8 ? (lane >> 4) + 4 * e : 4 * (lane >> 4) + e;
+}
+template <typename T>
+struct Acc16 {
+  typedef f4 type;
+};
+template <>
+struct Acc16<double> {
+  typedef d4 type;
+};
+
+// V[r][i] of a narrow panel at A (unit diagonal, zeros above it and past nb)
+template <typename T>
+__device__ __forceinline__ T narrow_v(const T* __restrict__ A, int lda, int rows, int nb, int r, int i) {
+  if (r < i || i >= nb || r >= rows) return T(0);
+  return r == i ? T(1) : A[(int64_t)r * lda + i];
+}
+
+// T of panels k = 0, 16.. of an already factored matrix, one workgroup each.
+template <typename T>
+__global__ void __launch_bounds__(kQrThreads) narrow_t_kernel(int m, int n, int block, const T* __restrict__ QR, int lda,
+                                                              const T* __restrict__ tau, T* __restrict__ Tout) {
+  __shared__ T part[kQrWaves][kNarrow][kNarrow];
+  __shared__ T G[kNarrow][kNarrow];
+  __shared__ T tl[kNarrow];
+  const int k = blockIdx.x * block, nb = min(block, n - k), rows = m - k;
+  const T* A = QR + (int64_t)k * lda + k;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  typename Acc16<T>::type acc = {0, 0, 0, 0};
+  for (int r0 = 16 * w; r0 < rows; r0 += 16 * kQrWaves) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const T v = narrow_v<T>(A, lda, rows, nb, r0 + acc_row<T>(lane, e), lane & 15);
+      acc = mma16(v, v, acc);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; e++) part[w][acc_row<T>(lane, e)][lane & 15] = acc[e];
+  if (t < kNarrow) tl[t] = t < nb ? tau[k + t] : T(0);
+  __syncthreads();
+  if (t < 256) {
+    T s = 0;
+    for (int q = 0; q < kQrWaves; q++) s += part[q][t >> 4][t & 15];
+    G[t >> 4][t & 15] = s;
+  }
+  __syncthreads();
+  if (t < kNarrow) narrow_t<T>(nb, G, tl, t, Tout + (int64_t)blockIdx.x * kNarrow * kNarrow);
+}
+
+// Tiles of 16 rows, wavefront w every 16th: the first and a last partial one
+// with every element's place looked at, the full ones below the unit triangle
+// four at a time, so that their loads are in flight together.
+template <typename F>
+__device__ __forceinline__ void walk_tiles(int rows, int w, F&& tile) {
+  int r0 = 16 * w;
+  if (r0 == 0) {
+    tile(0, false);
+    r0 = 16 * kQrWaves;
+  }
+#pragma unroll 4
+  for (; r0 + 16 <= rows; r0 += 16 * kQrWaves) tile(r0, true);
+  if (r0 < rows) tile(r0, false);
+}
+
+// C := (I - V op(T) V^T) C for a panel of at most 16 reflectors, 16 columns of
+// C a workgroup, in one launch: W = V^T C over all rows on MFMA (each wavefront
+// every 16th tile of 16 rows), the wavefronts' W summed in order through LDS,
+// Y = op(T) W by 256 threads, then C -= V Y on a second walk down the rows,
+// whose 16 columns are still in L2.  op(T) = T^T when `trans`.  The last
+// columns of the grid belong to a second matrix (lstsq's right-hand sides).
+// What bounds it is the latency of the two walks.  As three products of the
+// general GEMM the first one, one tile wide, ran 2500 rows deep on five
+// workgroups: 63 us against 30 us for this whole launch at 2500 x 284.
+template <typename T>
+__global__ void __launch_bounds__(kQrThreads) narrow_apply_kernel(int rows, int nb, const T* __restrict__ A, int lda,
+                                                                  const T* __restrict__ Tm, int trans, T* __restrict__ C1,
+                                                                  int ldc1, int width1, T* __restrict__ C2, int ldc2,
+                                                                  int width2) {
+  typedef typename Acc16<T>::type acc_t;
+  __shared__ T part[kQrWaves][kNarrow][kNarrow];
+  __shared__ T W[kNarrow][kNarrow], Y[kNarrow][kNarrow];
+  const int tiles1 = (width1 + 15) / 16;
+  const bool second = (int)blockIdx.x >= tiles1;
+  T* C = second ? C2 : C1;
+  const int ldc = second ? ldc2 : ldc1, width = second ? width2 : width1;
+  const int j0 = 16 * ((int)blockIdx.x - (second ? tiles1 : 0));
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int lc = lane & 15, lk = lane >> 4;
+  const bool in = j0 + lc < width;
+  C += j0 + (in ? lc : 0);
+  acc_t acc = {0, 0, 0, 0};
+  const int vc = min(lc, nb - 1);
+  walk_tiles(rows, w, [&](int r0, bool full) {
+    T v[4], cv[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int r = r0 + acc_row<T>(lane, e);
+      v[e] = full ? A[(int64_t)r * lda + vc] : narrow_v<T>(A, lda, rows, nb, r, lc);
+      cv[e] = full || r < rows ? C[(int64_t)r * ldc] : T(0);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc = mma16(lc < nb ? v[e] : T(0), cv[e], acc);
+  });
+#pragma unroll
+  for (int e = 0; e < 4; e++) part[w][acc_row<T>(lane, e)][lc] = acc[e];
+  __syncthreads();
+  if (t < 256) {
+    T s = 0;
+#pragma unroll
+    for (int q = 0; q < kQrWaves; q++) s += part[q][t >> 4][t & 15];
+    W[t >> 4][t & 15] = s;
+  }
+  __syncthreads();
+  if (t < 256) {
+    const int i = t >> 4, j = t & 15;
+    T s = 0;
+#pragma unroll
+    for (int q = 0; q < kNarrow; q++) s += (trans ? Tm[q * kNarrow + i] : Tm[i * kNarrow + q]) * W[q][j];
+    Y[i][j] = s;
+  }
+  __syncthreads();
+  T y[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) y[q] = Y[4 * lk + q][lc];
+  walk_tiles(rows, w, [&](int r0, bool full) {
+    T v[4], cv[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int i = 4 * lk + q;
+      v[q] = full ? A[(int64_t)(r0 + lc) * lda + min(i, nb - 1)] : narrow_v<T>(A, lda, rows, nb, r0 + lc, i);
+      if (i >= nb) v[q] = T(0);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int r = r0 + acc_row<T>(lane, e);
+      cv[e] = full || r < rows ? C[(int64_t)r * ldc] : T(0);
+    }
+    acc_t d = {0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 4; q++) d = mma16(v[q], y[q], d);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int r = r0 + acc_row<T>(lane, e);
+      if (in && (full || r < rows)) C[(int64_t)r * ldc] = cv[e] - d[e];
+    }
+  });
+}
+
+template <typename T>
+int narrow_apply(nmx_ctx* ctx, int rows, int nb, const T* A, int lda, const T* Tm, int trans, T* C1, int ldc1, int width1,
+                 T* C2, int ldc2, int width2) {
+  const int tiles = ceil_div(width1, 16) + ceil_div(width2, 16);
+  if (tiles <= 0) return NMX_OK;
+  ProfScope ps(ctx, K_GEMM, 4.0 * rows * nb * (double)(width1 + width2), 0.0);
+  narrow_apply_kernel<T><<<tiles, kQrThreads, 0, ctx->stream>>>(rows, nb, A, lda, Tm, trans, C1, ldc1, width1, C2, ldc2,
+                                                                width2);
+  NMX_HIP(ctx, hipGetLastError());
+  return NMX_OK;
+}
+
+// Factors the panel at A (rows x nb, nb <= 16) and leaves its T in Tm.  The
+// register kernels hold 4 NW R rows; the fewest that fit, since a step's sums
+// go with R and its LDS round with NW.  A taller panel streams through memory.
+template <typename T>
+int narrow_panel(nmx_ctx* ctx, int m, int k, int nb, T* A, int lda, T* tau, T* Tm) {
+  const int rows = m - k;
+  T* P = A + (int64_t)k * lda + k;
+  ProfScope ps(ctx, K_QR_PANEL, 4.0 * (double)rows * nb * nb, 2.0 * sizeof(T) * (double)rows * nb);
+  if (rows <= 256) geqr2_narrow_kernel<T, 16, 4><<<1, 256, 0, ctx->stream>>>(rows, nb, P, lda, tau + k, Tm);
+  else if (rows <= 1024) geqr2_narrow_kernel<T, 16, 16><<<1, 1024, 0, ctx->stream>>>(rows, nb, P, lda, tau + k, Tm);
+  else if (rows <= 2048) geqr2_narrow_kernel<T, 32, 16><<<1, 1024, 0, ctx->stream>>>(rows, nb, P, lda, tau + k, Tm);
+  else if (sizeof(T) == 4 && rows <= 4096) {
+    if constexpr (sizeof(T) == 4)
+      geqr2_narrow_kernel<T, 64, 16><<<1, 1024, 0, ctx->stream>>>(rows, nb, P, lda, tau + k, Tm);
+  } else {
+    geqr2_kernel<T><<<1, kQrThreads, 0, ctx->stream>>>(m, A, lda, tau, k, nb);
+    NMX_HIP(ctx, hipGetLastError());
+    narrow_t_kernel<T><<<1, kQrThreads, 0, ctx->stream>>>(rows, nb, nb, P, lda, tau + k, Tm);
+  }
+  NMX_HIP(ctx, hipGetLastError());
+  return NMX_OK;
+}
+
+// Blocked QR with panels of at most 16 columns; every panel's reflector also
+// reaches B (m x nrhs; nrhs 0: none), which leaves Q^T B there.
+template <typename T>
+int geqrf_narrow(nmx_ctx* ctx, int m, int n, T* A, int lda, T* tau, int block, T* B, int ldb, int nrhs) {
+  void* ws = nullptr;
+  NMX_TRY(nmx_workspace(ctx, kNarrow * kNarrow * sizeof(T), &ws));
+  for (int k = 0; k < n; k += block) {
+    const int nb = std::min(block, n - k), width = n - k - nb;
+    NMX_TRY(narrow_panel<T>(ctx, m, k, nb, A, lda, tau, (T*)ws));
+    const T* P = A + (int64_t)k * lda + k;
+    NMX_TRY(narrow_apply<T>(ctx, m - k, nb, P, lda, (const T*)ws, 1, A + (int64_t)k * lda + k + nb, lda, width,
+                            B + (int64_t)k * ldb, ldb, nrhs));
+  }
+  return NMX_OK;
+}
+
+// The Ts of all panels of a factored matrix, in the context workspace.
+template <typename T>
+int narrow_all_t(nmx_ctx* ctx, int m, int n, const T* QR, int lda, const T* tau, int block, const T** out) {
+  const int steps = ceil_div(n, block);
+  void* ws = nullptr;
+  NMX_TRY(nmx_workspace(ctx, (size_t)steps * kNarrow * kNarrow * sizeof(T), &ws));
+  narrow_t_kernel<T><<<steps, kQrThreads, 0, ctx->stream>>>(m, n, block, QR, lda, tau, (T*)ws);
+  NMX_HIP(ctx, hipGetLastError());
+  *out = (const T*)ws;
+  return NMX_OK;
+}
+
 template <typename T>
 int geqrf_impl(nmx_ctx* ctx, int m, int n, T* A, int lda, T* tau, int block) {
+  if (block <= kNarrow) return geqrf_narrow<T>(ctx, m, n, A, lda, tau, block, (T*)nullptr, 0, 0);
   void* ws = nullptr;
   NMX_TRY(nmx_workspace(ctx, reflector_bytes<T>(m, block, n), &ws));
   const Reflector<T> w = carve<T>(ws, m, block, n);
@@ -250,10 +650,20 @@ int geqrf_impl(nmx_ctx* ctx, int m, int n, T* A, int lda, T* tau, int block) {
 template <typename T>
 int ormqr_impl(nmx_ctx* ctx, int trans, int m, int n, int nrhs, const T* QR, int lda, const T* tau, T* B, int ldb,
                int block) {
+  const int steps = ceil_div(n, block);
+  if (block <= kNarrow) {
+    const T* Tm = nullptr;
+    NMX_TRY(narrow_all_t<T>(ctx, m, n, QR, lda, tau, block, &Tm));
+    for (int s = 0; s < steps; s++) {
+      const int p = trans ? s : steps - 1 - s, k = p * block;
+      NMX_TRY(narrow_apply<T>(ctx, m - k, std::min(block, n - k), QR + (int64_t)k * lda + k, lda,
+                              Tm + (size_t)p * kNarrow * kNarrow, trans, B + (int64_t)k * ldb, ldb, nrhs, (T*)nullptr, 0, 0));
+    }
+    return NMX_OK;
+  }
   void* ws = nullptr;
   NMX_TRY(nmx_workspace(ctx, reflector_bytes<T>(m, block, nrhs), &ws));
   const Reflector<T> w = carve<T>(ws, m, block, nrhs);
-  const int steps = ceil_div(n, block);
   for (int s = 0; s < steps; s++) {
     const int k = (trans ? s : steps - 1 - s) * block;
     const int nb = std::min(block, n - k);
@@ -313,6 +723,16 @@ int orgqr_api(nmx_ctx* ctx, int m, int n, const T* QR, int lda, const T* tau, T*
   identity_kernel<T><<<(unsigned)(((int64_t)m * n + 255) / 256), 256, 0, ctx->stream>>>(m, n, Q, ldq);
   NMX_HIP(ctx, hipGetLastError());
   // last panel first; columns left of the panel are unchanged (V^T e_j = 0)
+  if (block <= kNarrow) {
+    const T* Tm = nullptr;
+    NMX_TRY(narrow_all_t<T>(ctx, m, n, QR, lda, tau, block, &Tm));
+    for (int p = ceil_div(n, block) - 1; p >= 0; p--) {
+      const int k = p * block;
+      NMX_TRY(narrow_apply<T>(ctx, m - k, std::min(block, n - k), QR + (int64_t)k * lda + k, lda,
+                              Tm + (size_t)p * kNarrow * kNarrow, 0, Q + (int64_t)k * ldq + k, ldq, n - k, (T*)nullptr, 0, 0));
+    }
+    return NMX_OK;
+  }
   void* ws = nullptr;
   NMX_TRY(nmx_workspace(ctx, reflector_bytes<T>(m, block, n), &ws));
   const Reflector<T> w = carve<T>(ws, m, block, n);
@@ -353,8 +773,12 @@ int gels_api(nmx_ctx* ctx, int m, int n, int nrhs, T* A, int lda, T* tau, T* B, 
   if (!A) return -5;
   if (!tau) return -7;
   if (!B) return -8;
-  NMX_TRY(geqrf_impl<T>(ctx, m, n, A, lda, tau, block));
-  NMX_TRY(ormqr_impl<T>(ctx, 1, m, n, nrhs, A, lda, tau, B, ldb, block));
+  if (block <= kNarrow) {
+    NMX_TRY(geqrf_narrow<T>(ctx, m, n, A, lda, tau, block, B, ldb, nrhs));
+  } else {
+    NMX_TRY(geqrf_impl<T>(ctx, m, n, A, lda, tau, block));
+    NMX_TRY(ormqr_impl<T>(ctx, 1, m, n, nrhs, A, lda, tau, B, ldb, block));
+  }
   return trsm_left<T>(ctx, 1, 0, 0, n, nrhs, A, lda, B, ldb);
 }
 

@@ -161,3 +161,37 @@ def test_laswp_f32_is_exact():
     got = nl.laswp(b, ipiv).cpu().numpy()
     assert got.dtype == np.float32
     np.testing.assert_array_equal(got, oracle.laswp(b.astype(np.float64), ipiv).astype(np.float32))
+
+
+@pytest.mark.parametrize("m,n,block", [(16, 16, 16), (17, 3, 3), (255, 17, 16), (256, 16, 16), (257, 20, 7),
+                                       (1024, 33, 16), (1040, 19, 16), (2048, 18, 16), (2065, 17, 16), (4096, 20, 16),
+                                       (4113, 18, 16)])
+def test_narrow_panels_at_the_register_kernels_edges(m, n, block):
+    """Panels of at most 16 columns: the row limits of the register kernels
+    (256, 1024, 2048, FP32 4096), the streaming panel above them, panels and
+    trailing matrices that are no multiple of 16, a column that is zero below
+    its diagonal (tau 0) and untouched memory right of the matrix."""
+    import torch
+    for dtype, eps in ((np.float64, 2.3e-16), (np.float32, 1.2e-7)):
+        a = R.normal(m + 31 * n, (m, n)).astype(dtype)
+        a[1:, 0] = 0
+        f = nl.qr_factor(a, block=block)
+        qr_o, tau_o = oracle.geqrf(a.astype(np.float64), block=block)
+        qr, tau = f.factored.cpu().numpy().astype(np.float64), f.taus.cpu().numpy().astype(np.float64)
+        tol = 50 * np.sqrt(m) * n * eps  # columns of norm sqrt(m), n reflectors each rounding once
+        assert tau[0] == 0.0
+        np.testing.assert_allclose(tau, tau_o, atol=tol)
+        np.testing.assert_allclose(qr, qr_o, atol=tol * _scale(qr_o))
+        q = f.q().cpu().numpy().astype(np.float64)
+        np.testing.assert_allclose(q @ np.triu(qr[:n]), a, atol=tol * _scale(a))
+        b = R.normal(m + n, (m, 3)).astype(dtype)
+        x = nl.lstsq(a, b, block=block).cpu().numpy()
+        np.testing.assert_allclose(x, f.solve(b).cpu().numpy(), atol=tol * 10, rtol=tol * 10)
+        # a strided panel: the columns right of the matrix stay as they were
+        wide = torch.full((m, n + 5), 7.0, dtype=torch.float64 if dtype == np.float64 else torch.float32, device="cuda")
+        wide[:, :n] = torch.as_tensor(a, device="cuda")
+        taus = torch.zeros(n, dtype=wide.dtype, device="cuda")
+        from numax_amd import _lib
+        _lib.check(nl._fn("geqrf", wide.dtype)(nl._ctx(wide).handle, m, n, nl._ptr(wide), n + 5, nl._ptr(taus), block),
+                   "geqrf")
+        assert torch.equal(wide[:, :n], f.factored) and bool((wide[:, n:] == 7.0).all())
