@@ -68,7 +68,6 @@ NMX_API int nmx_ctx_create(int device, void* stream, nmx_ctx** out) {
   }
   if (hipMalloc(&c->err, 256) != hipSuccess) { nmx_ctx_destroy(c); return NMX_ERR_ALLOC; }
   if (hipMalloc(&c->mailbox, kMailboxBytes) != hipSuccess) { nmx_ctx_destroy(c); return NMX_ERR_ALLOC; }
-  if (hipMalloc(&c->tri_inv, 64 * 64 * sizeof(double)) != hipSuccess) { nmx_ctx_destroy(c); return NMX_ERR_ALLOC; }
   c->mailbox_bytes = kMailboxBytes;
   // an error another runtime user of this process left behind is not ours
   (void)hipGetLastError();
@@ -124,7 +123,6 @@ static void ctx_release(nmx_ctx* c) {
   if (c->ws) hipFree(c->ws);
   if (c->mailbox) hipFree(c->mailbox);
   if (c->err) hipFree(c->err);
-  if (c->tri_inv) hipFree(c->tri_inv);
   if (c->mp_cache && c->mp_cache_free) c->mp_cache_free(c->mp_cache);
   if (c->own_stream && c->stream) hipStreamDestroy(c->stream);
   delete c;

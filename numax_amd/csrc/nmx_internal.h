@@ -95,8 +95,6 @@ struct nmx_ctx {
   uint32_t epoch = 0;  // last epoch handed to a kernel (monotonic)
   // device error word (sticky): NMX_ERR_SYNC_TIMEOUT from bounded waits
   int* err = nullptr;
-  // 64 x 64 scratch for the inverse of a triangular base block (FP64-sized)
-  void* tri_inv = nullptr;
   // buffers of the mixed-precision factorization, kept across calls
   void* mp_cache = nullptr;
   void (*mp_cache_free)(void*) = nullptr;
@@ -156,6 +154,13 @@ int gemm_launch_splitk(nmx_ctx* ctx, int m, int n, int k, T alpha, const T* A, i
 // Left-side triangular solve op(T) X = B (vectors are columns of B).
 template <typename T>
 int trsm_left(nmx_ctx* ctx, int upper, int unit, int trans, int n, int nrhs, const T* Tm, int ldt, T* B, int ldb);
+
+// op(T) X = B in place for a triangle of at most kStripMax rows (one launch);
+// vec_rows: the vectors are B's rows (B is nvec x n), else its columns.
+constexpr int kStripMax = 256;
+template <typename T>
+int trsm_strip(nmx_ctx* ctx, int upper, int unit, int trans, int vec_rows, int n, int nvec, const T* Tm, int ldt, T* B,
+               int ldb);
 
 // Right-side X := X L^-T with L lower n x n; X is m x n (the Cholesky panel).
 template <typename T>

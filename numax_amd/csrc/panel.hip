@@ -626,168 +626,6 @@ __global__ void __launch_bounds__(256) gather_rows_kernel(int n, int ncols, cons
   out[(int64_t)i * ldo + c] = (To)in[(int64_t)perm[i] * ldi + c];
 }
 
-// Base triangular solve for n <= NB (32 or 64): one thread per vector, the
-// vector in registers, op(T) staged in LDS by columns.  Right-looking with
-// every index static: x_j is finished, then x_i -= op(T)[i][j] x_j for the
-// rows after it -- independent updates, so the substitution is throughput-
-// rather than latency-bound.  A lower solve takes each row's products in
-// ascending column order, as trsm_diag (panel.mojo:2221-2276): running
-// subtraction from the right-hand side, then the division unless `unit`; an
-// upper solve takes them in descending order.  VEC_ROWS picks where the
-// vectors live: the columns of B (left solves) or its rows (the Cholesky
-// panel X L^-T).
-template <typename T, int NB, int UPPER, int UNIT, int TRANS, int VEC_ROWS>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) trsm_base(int n, int nvec, const T* __restrict__ Tm, int ldt, T* __restrict__ B,
-                                                int ldb) {
-  __shared__ T Tc[NB][NB + 16 / sizeof(T)];  // Tc[j][i] = op(T)[i][j]
-  const int t = threadIdx.x;
-  const int v = blockIdx.x * 64 + t;
-  // padded to NB with the identity, so the sweeps below need no bounds; all
-  // NB^2/64 loads of a thread are issued before the first LDS store
-  {
-    constexpr int PER = NB * NB / 64;
-    const __amdgpu_buffer_rsrc_t rt = buf_rsrc(Tm);
-    T stg[PER];
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int idx = t + 64 * i, r = idx / NB, c = idx % NB;  // T[r][c], read along rows
-      const uint32_t off = (uint32_t)r * (uint32_t)ldt + (uint32_t)c;
-      stg[i] = buf_load<T>(rt, (r < n && c < n) ? off * (uint32_t)sizeof(T) : kBufOob);
-    }
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int idx = t + 64 * i, r = idx / NB, c = idx % NB;
-      const T val = (r < n && c < n) ? stg[i] : T(r == c ? 1 : 0);
-      if (TRANS) Tc[r][c] = val;  // op(T)[c][r]
-      else Tc[c][r] = val;        // op(T)[r][c]
-    }
-  }
-  __syncthreads();
-  // the block's 64 vectors through one descriptor (32-bit offsets, past-the-
-  // end lanes and rows read 0 and store nothing)
-  const int v0 = blockIdx.x * 64;
-  const __amdgpu_buffer_rsrc_t rb = buf_rsrc(VEC_ROWS ? B + (int64_t)v0 * ldb : B + v0);
-  const bool act = v < nvec;
-  T x[NB];
-#pragma unroll
-  for (int i = 0; i < NB; i++) {
-    const uint32_t off = VEC_ROWS ? (uint32_t)t * (uint32_t)ldb + (uint32_t)i : (uint32_t)i * (uint32_t)ldb + (uint32_t)t;
-    x[i] = buf_load<T>(rb, (act & (i < n)) ? (uint32_t)sizeof(T) * off : kBufOob);
-  }
-  // rows and columns past n are the identity and x is 0 there: they change
-  // nothing.  Each step's column is addressed through an index made opaque
-  // on a value of the step before, so the compiler cannot hoist the whole
-  // triangle into registers (NB^2/2 of them), and a scheduling barrier makes
-  // the step's LDS reads go out together: left to itself the compiler issues
-  // them one pair at a time between the products, a full LDS round trip per
-  // pair (2.3x slower at NB = 64).  FP32 reads step j's column during step
-  // j-1, right after the product that finishes x_j and before the rest, so
-  // the latency hides under those products; FP64 (twice the registers) reads
-  // it at the start of step j, which measured faster there.  Every x_i takes
-  // the same products in the same order as plain substitution.
-  constexpr bool kAhead = sizeof(T) == 4;
-  if (!UPPER && !kAhead) {
-#pragma unroll
-    for (int j = 0; j < NB; j++) {
-      const T xj = UNIT ? x[j] : x[j] / Tc[j][j];
-      x[j] = xj;
-      int jj = j;
-      asm volatile("" : "+s"(jj) : "v"(xj));
-      const T* col = Tc[jj];
-      T cv[NB];
-#pragma unroll
-      for (int i = j + 1; i < NB; i++) cv[i] = col[i];
-      __builtin_amdgcn_sched_barrier(0);  // the step's reads all go out before its products
-#pragma unroll
-      for (int i = j + 1; i < NB; i++) x[i] = x[i] - cv[i] * xj;
-    }
-  } else if (UPPER && !kAhead) {
-#pragma unroll
-    for (int j = NB - 1; j >= 0; j--) {
-      const T xj = UNIT ? x[j] : x[j] / Tc[j][j];
-      x[j] = xj;
-      int jj = j;
-      asm volatile("" : "+s"(jj) : "v"(xj));
-      const T* col = Tc[jj];
-      T cv[NB];
-#pragma unroll
-      for (int i = 0; i < j; i++) cv[i] = col[i];
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < j; i++) x[i] = x[i] - cv[i] * xj;
-    }
-  } else if (!UPPER) {
-    T cv[NB];  // the current step's column, read one step ahead
-    {
-      int jj = 0;
-      asm volatile("" : "+s"(jj));
-      const T* col = Tc[jj];
-#pragma unroll
-      for (int i = 1; i < NB; i++) cv[i] = col[i];
-    }
-#pragma unroll
-    for (int j = 0; j < NB; j++) {
-      const T xj = UNIT ? x[j] : x[j] / Tc[j][j];
-      x[j] = xj;
-      if (j + 1 < NB) {
-        __builtin_amdgcn_sched_barrier(0);
-        x[j + 1] = x[j + 1] - cv[j + 1] * xj;  // the next step's unknown first
-        T cn[NB];
-        int jj = j + 1;
-        asm volatile("" : "+s"(jj) : "v"(x[j + 1]));
-        const T* col = Tc[jj];
-#pragma unroll
-        for (int i = j + 2; i < NB; i++) cn[i] = col[i];
-        __builtin_amdgcn_sched_barrier(0);  // the reads go out before this step's products
-#pragma unroll
-        for (int i = j + 2; i < NB; i++) x[i] = x[i] - cv[i] * xj;
-#pragma unroll
-        for (int i = j + 2; i < NB; i++) cv[i] = cn[i];
-      }
-    }
-  } else {
-    T cv[NB];
-    {
-      int jj = NB - 1;
-      asm volatile("" : "+s"(jj));
-      const T* col = Tc[jj];
-#pragma unroll
-      for (int i = 0; i < NB - 1; i++) cv[i] = col[i];
-    }
-#pragma unroll
-    for (int j = NB - 1; j >= 0; j--) {
-      const T xj = UNIT ? x[j] : x[j] / Tc[j][j];
-      x[j] = xj;
-      if (j > 0) {
-        __builtin_amdgcn_sched_barrier(0);
-        x[j - 1] = x[j - 1] - cv[j - 1] * xj;
-        T cn[NB];
-        int jj = j - 1;
-        asm volatile("" : "+s"(jj) : "v"(x[j - 1]));
-        const T* col = Tc[jj];
-#pragma unroll
-        for (int i = 0; i < j - 1; i++) cn[i] = col[i];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < j - 1; i++) x[i] = x[i] - cv[i] * xj;
-#pragma unroll
-        for (int i = 0; i < j - 1; i++) cv[i] = cn[i];
-      }
-    }
-  }
-  // the store offsets are recomputed from an opaque lane index: shared with
-  // the loads' they would stay live (NB registers) through the sweep
-  int ts = t;
-  asm volatile("" : "+v"(ts));
-  const bool acts = ts + v0 < nvec;
-#pragma unroll
-  for (int i = 0; i < NB; i++) {
-    const uint32_t off =
-        VEC_ROWS ? (uint32_t)ts * (uint32_t)ldb + (uint32_t)i : (uint32_t)i * (uint32_t)ldb + (uint32_t)ts;
-    buf_store(rb, (acts & (i < n)) ? (uint32_t)sizeof(T) * off : kBufOob, x[i]);
-  }
-}
-
 // potrf_diag (panel.mojo:216-286) for nb <= 64, the block staged in LDS:
 // d <= 0 floored to 1e-30 with the first failure recorded 1-based, column
 // scaled by the root, then the lower triangle's rank-1 update.
@@ -868,129 +706,6 @@ __global__ void zero_i32(int32_t* p, int n) {
   if (i < n) p[i] = 0;
 }
 
-// inv(op(T)) for n <= 64 into a dense 64 x 64 (ld 64) block: one thread per
-// column of the inverse, substitution against the triangle staged in LDS.
-template <typename T, int UPPER, int UNIT, int TRANS>
-__global__ void __launch_bounds__(1024) tri_inv_small(int n, const T* __restrict__ Tm, int ldt, T* __restrict__ inv) {
-  // Gauss-Jordan sweep on [op(T) | I]: one pivot row per step, every other
-  // row updated in parallel (n <= 64 steps, each a barrier apart).
-  __shared__ T S[64][65];
-  __shared__ T X[64][65];
-  const int t = threadIdx.x;
-  for (int idx = t; idx < 64 * 64; idx += 1024) {
-    const int i = idx / 64, q = idx % 64;
-    S[i][q] = (i < n && q < n) ? (TRANS ? Tm[(int64_t)q * ldt + i] : Tm[(int64_t)i * ldt + q]) : T(0);
-    X[i][q] = (i == q) ? T(1) : T(0);
-  }
-  __syncthreads();
-  for (int s = 0; s < n; s++) {
-    const int j = UPPER ? n - 1 - s : s;
-    if (!UNIT) {
-      if (t < 64) X[j][t] = X[j][t] / S[j][j];
-      __syncthreads();
-    }
-    for (int idx = t; idx < 64 * 64; idx += 1024) {
-      const int r = idx / 64, c = idx % 64;
-      const bool below = UPPER ? (r < j) : (r > j && r < n);
-      if (below) X[r][c] = X[r][c] - S[r][j] * X[j][c];
-    }
-    __syncthreads();
-  }
-  for (int idx = t; idx < 64 * 64; idx += 1024) {
-    const int i = idx / 64, q = idx % 64;
-    inv[idx] = (i < n && q < n) ? X[i][q] : T(0);
-  }
-}
-
-// Apply a 64 x 64 (ld 64) inverse to 64 vectors per workgroup, in place:
-// each vector x of B becomes inv x.  Thread t owns vector t % 64 and 16 of
-// its n entries; the inverse and the vectors are staged in LDS.
-template <typename T, int VEC_ROWS>
-__global__ void __launch_bounds__(256) tri_apply_small(int n, int nvec, const T* __restrict__ inv,
-                                                       T* __restrict__ B, int ldb) {
-  __shared__ T Is[64][65];
-  __shared__ T Xs[64][65];
-  const int t = threadIdx.x;
-  const int v0 = blockIdx.x * 64;
-  for (int idx = t; idx < 64 * 64; idx += 256) Is[idx / 64][idx % 64] = inv[idx];
-  if (VEC_ROWS) {
-    for (int idx = t; idx < n * 64; idx += 256) {
-      int v = idx / n, i = idx % n;
-      if (v0 + v < nvec) Xs[i][v] = B[(int64_t)(v0 + v) * ldb + i];
-    }
-  } else {
-    for (int idx = t; idx < n * 64; idx += 256) {
-      int i = idx / 64, v = idx % 64;
-      if (v0 + v < nvec) Xs[i][v] = B[(int64_t)i * ldb + v0 + v];
-    }
-  }
-  __syncthreads();
-  const int v = t & 63, i0 = (t >> 6) * 16;
-  T y[16];
-#pragma unroll
-  for (int r = 0; r < 16; r++) y[r] = T(0);
-  for (int q = 0; q < n; q++) {
-    const T xq = Xs[q][v];
-#pragma unroll
-    for (int r = 0; r < 16; r++) y[r] += Is[i0 + r][q] * xq;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < 16; r++) Xs[i0 + r][v] = y[r];
-  __syncthreads();
-  if (VEC_ROWS) {
-    for (int idx = t; idx < n * 64; idx += 256) {
-      int vv = idx / n, i = idx % n;
-      if (v0 + vv < nvec) B[(int64_t)(v0 + vv) * ldb + i] = Xs[i][vv];
-    }
-  } else {
-    for (int idx = t; idx < n * 64; idx += 256) {
-      int i = idx / 64, vv = idx % 64;
-      if (v0 + vv < nvec) B[(int64_t)i * ldb + v0 + vv] = Xs[i][vv];
-    }
-  }
-}
-
-constexpr int kBaseInverseMinVec = 1 << 30;  // substitution for every width
-
-template <typename T, int UPPER, int UNIT, int TRANS, int VEC_ROWS>
-void launch_base(nmx_ctx* ctx, int n, int nvec, const T* Tm, int ldt, T* B, int ldb) {
-  // the explicit inverse only pays off for very wide right-hand sides: the
-  // register-resident substitution above runs 64 vectors per wavefront
-  if (nvec > kBaseInverseMinVec && ctx->tri_inv) {
-    T* inv = (T*)ctx->tri_inv;
-    ProfScope ps(ctx, K_TRSM, 2.0 * n * (double)n * nvec, sizeof(T) * (2.0 * n * nvec + 64.0 * 64));
-    tri_inv_small<T, UPPER, UNIT, TRANS><<<1, 1024, 0, ctx->stream>>>(n, Tm, ldt, inv);
-    tri_apply_small<T, VEC_ROWS><<<ceil_div(nvec, 64), 256, 0, ctx->stream>>>(n, nvec, inv, B, ldb);
-    return;
-  }
-  ProfScope ps(ctx, K_TRSM, (double)n * n * nvec, sizeof(T) * ((double)n * n + 2.0 * n * nvec));
-  if (n <= 32)
-    trsm_base<T, 32, UPPER, UNIT, TRANS, VEC_ROWS><<<ceil_div(nvec, 64), 64, 0, ctx->stream>>>(n, nvec, Tm, ldt, B,
-                                                                                             ldb);
-  else
-    trsm_base<T, 64, UPPER, UNIT, TRANS, VEC_ROWS><<<ceil_div(nvec, 64), 64, 0, ctx->stream>>>(n, nvec, Tm, ldt, B,
-                                                                                             ldb);
-}
-
-template <typename T, int VEC_ROWS>
-int base_dispatch(nmx_ctx* ctx, int upper, int unit, int trans, int n, int nvec, const T* Tm, int ldt, T* B,
-                  int ldb) {
-  int key = upper * 4 + unit * 2 + trans;
-  switch (key) {
-    case 0: launch_base<T, 0, 0, 0, VEC_ROWS>(ctx, n, nvec, Tm, ldt, B, ldb); break;
-    case 1: launch_base<T, 0, 0, 1, VEC_ROWS>(ctx, n, nvec, Tm, ldt, B, ldb); break;
-    case 2: launch_base<T, 0, 1, 0, VEC_ROWS>(ctx, n, nvec, Tm, ldt, B, ldb); break;
-    case 3: launch_base<T, 0, 1, 1, VEC_ROWS>(ctx, n, nvec, Tm, ldt, B, ldb); break;
-    case 4: launch_base<T, 1, 0, 0, VEC_ROWS>(ctx, n, nvec, Tm, ldt, B, ldb); break;
-    case 5: launch_base<T, 1, 0, 1, VEC_ROWS>(ctx, n, nvec, Tm, ldt, B, ldb); break;
-    case 6: launch_base<T, 1, 1, 0, VEC_ROWS>(ctx, n, nvec, Tm, ldt, B, ldb); break;
-    default: launch_base<T, 1, 1, 1, VEC_ROWS>(ctx, n, nvec, Tm, ldt, B, ldb); break;
-  }
-  NMX_HIP(ctx, hipGetLastError());
-  return NMX_OK;
-}
-
 // Recursive triangular solve: split op(T) in two, solve one diagonal block,
 // update the other half of the right-hand sides with the MFMA GEMM, solve the
 // other block.  VEC_ROWS = 0: the vectors are B's columns (B is n x nvec);
@@ -998,9 +713,15 @@ int base_dispatch(nmx_ctx* ctx, int upper, int unit, int trans, int n, int nvec,
 template <typename T, int VEC_ROWS>
 int trsm_rec(nmx_ctx* ctx, int upper, int unit, int trans, int n, int nvec, const T* Tm, int ldt, T* B, int ldb) {
   if (n <= 0 || nvec <= 0) return NMX_OK;
-  if (n <= 64) return base_dispatch<T, VEC_ROWS>(ctx, upper, unit, trans, n, nvec, Tm, ldt, B, ldb);
-  int n1 = ((n / 2 + 63) / 64) * 64;
-  if (n1 >= n) n1 = n - 64;
+  // a strip's offsets are 32-bit: rows of an operand more than 2 GiB apart
+  // (hundreds of thousands of columns) go through in lower strips
+  const int64_t span = (VEC_ROWS ? 32 : (int64_t)n) * ldb, tspan = (int64_t)n * ldt;
+  const bool fits = std::max(span, tspan) * (int64_t)sizeof(T) < 0x7FFFFFFF;
+  if (n <= kStripMax && (fits || n <= 16))
+    return trsm_strip<T>(ctx, upper, unit, trans, VEC_ROWS, n, nvec, Tm, ldt, B, ldb);
+  // whole strips but for the last block
+  const int unit_rows = n > kStripMax ? kStripMax : 16;
+  const int n1 = ((n / 2 + unit_rows - 1) / unit_rows) * unit_rows;
   const int n2 = n - n1;
   const T* T11 = Tm;
   const T* T22 = Tm + (int64_t)n1 * ldt + n1;

@@ -288,3 +288,57 @@ def test_cholesky_c2_scale():
     r = b - a @ x
     eta = (r.abs().max(0).values / (a.abs().sum(1).max() * x.abs().max(0).values)).max().item()
     assert eta < 10 * n * EPS
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 128, 129, 255, 256, 257, 530])
+def test_triangular_strip_edges(n, dtype):
+    """Every triangle, diagonal and transposition at the edges of the 16-row
+    steps and the 64 / 128 / 256-row kernels, one to 33 vectors, strided
+    operands, and the residual bound of substitution (n eps |T||x|, with a
+    factor for the inverted 16 x 16 blocks)."""
+    eps = torch.finfo(dtype).eps
+    rng = np.random.default_rng(n)
+    for upper, unit, trans, nrhs in ((0, 0, 0, 1), (0, 1, 0, 16), (1, 0, 0, 17), (1, 1, 0, 33), (0, 0, 1, 5),
+                                     (1, 0, 1, 2), (0, 1, 1, 1), (1, 1, 1, 20)):
+        t = rng.standard_normal((n, n + 3)) / np.sqrt(n)
+        t[:, :n] += 2.0 * np.eye(n)
+        T = torch.as_tensor(t, device="cuda").to(dtype)
+        B0 = torch.as_tensor(rng.standard_normal((n, nrhs + 2)), device="cuda").to(dtype)
+        B = B0.clone()
+        stored = T[:, :n].double().cpu().numpy()
+        stored = np.triu(stored) if upper else np.tril(stored)
+        if unit:
+            stored = stored - np.diag(np.diag(stored)) + np.eye(n)
+        op = stored.T if trans else stored
+        from numax_amd import _lib
+        _lib.check(nl._fn("trsm", dtype)(nl._ctx(T).handle, int(upper != trans), unit, trans, n, nrhs, nl._ptr(T), n + 3,
+                                         nl._ptr(B), nrhs + 2), "trsm")
+        x = B[:, :nrhs].double().cpu().numpy()
+        r = np.abs(op @ x - B0[:, :nrhs].double().cpu().numpy())
+        assert np.all(r <= 16 * (n + 16) * eps * (np.abs(op) @ np.abs(x) + 1)), (upper, unit, trans, nrhs)
+        assert torch.equal(B[:, nrhs:], B0[:, nrhs:])
+
+
+def test_triangular_strip_spreads_infinities_as_substitution_does():
+    n = 70
+    rng = np.random.default_rng(9)
+    t = np.tril(rng.standard_normal((n, n))) + 4 * np.eye(n)
+    b = rng.standard_normal((n, 3))
+    b[20, 1] = np.inf
+    t2 = t.copy()
+    t2[40, 40] = 0.0  # a zero on the diagonal divides
+    for m, upper in ((t, False), (t2, False), (t.T.copy(), True), (t2.T.copy(), True)):
+        x = _np(nl.solve_triangular(m, b, upper=upper))
+        order = range(n - 1, -1, -1) if upper else range(n)
+        xo = np.empty_like(b)
+        with np.errstate(all="ignore"):
+            w = b.copy()
+            for j in order:
+                xo[j] = w[j] / m[j, j]
+                rest = range(j) if upper else range(j + 1, n)
+                for i in rest:
+                    w[i] = w[i] - m[i, j] * xo[j]
+        np.testing.assert_array_equal(np.isfinite(x), np.isfinite(xo))
+        ok = np.isfinite(xo)
+        np.testing.assert_allclose(x[ok], xo[ok], rtol=1e-10, atol=1e-12)
