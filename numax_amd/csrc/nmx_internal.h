@@ -211,6 +211,14 @@ int tslu_panel_launch(nmx_ctx* ctx, void* scratch, size_t scratch_bytes, int n, 
 int tslu_swap_columns(nmx_ctx* ctx, void* scratch, float* A, int lda, int k, int nb, int c_lo, int c_hi,
                       int slot = 0);
 
+// Cholesky of the diagonal block at (k0, k0), nb <= chol_block_max columns, in
+// one workgroup (a block row of 16 x 16 tiles per wavefront: FP64 tiles of
+// 256 columns do not fit the registers).
+template <typename T>
+constexpr int chol_block_max() { return sizeof(T) == 8 ? 128 : 256; }
+template <typename T>
+int chol_block(nmx_ctx* ctx, T* A, int lda, int k0, int nb, int32_t* info);
+
 template <typename T>
 int potrf_impl(nmx_ctx* ctx, int n, T* A, int lda, int32_t* info, int block);
 

@@ -626,67 +626,6 @@ __global__ void __launch_bounds__(256) gather_rows_kernel(int n, int ncols, cons
   out[(int64_t)i * ldo + c] = (To)in[(int64_t)perm[i] * ldi + c];
 }
 
-// potrf_diag (panel.mojo:216-286) for nb <= 64, the block staged in LDS:
-// d <= 0 floored to 1e-30 with the first failure recorded 1-based, column
-// scaled by the root, then the lower triangle's rank-1 update.
-template <typename T>
-__global__ void __launch_bounds__(256) potrf_diag_kernel(T* __restrict__ A, int lda, int k0, int nb,
-                                                         int32_t* __restrict__ info) {
-  // thread t: row i = t % 64 of the block, columns 16 q .. 16 q + 15 in
-  // registers (q = t / 64, one wavefront per column quarter).  Column j's
-  // owner wavefront scales it and publishes it through LDS (two buffers by
-  // parity); one barrier per column, then every row updates its own columns.
-  __shared__ T col[2][64];
-  __shared__ int info_set;
-  const int t = threadIdx.x, i = t & 63, q = t >> 6;
-  T R[16];
-#pragma unroll
-  for (int cc = 0; cc < 16; cc++) {
-    const int c = 16 * q + cc;
-    R[cc] = (i < nb && c <= i) ? A[(int64_t)(k0 + i) * lda + k0 + c] : T(0);
-  }
-  if (t == 0) info_set = (*info != 0);
-  __syncthreads();
-  for (int qj = 0; qj < 4; qj++) {
-#pragma unroll
-    for (int cj = 0; cj < 16; cj++) {
-      const int j = 16 * qj + cj;
-      if (j >= nb) break;
-      T* cv = col[j & 1];
-      if (q == qj) {
-        const T d = __shfl(R[cj], j);  // the diagonal entry, from lane j
-        T dd = d;
-        if (dd <= T(0)) dd = T(kPivotFloor);
-        const T root = sqrt(dd);
-        if (i > j && i < nb) {
-          R[cj] = R[cj] / root;
-          cv[i] = R[cj];
-        } else if (i == j) {
-          R[cj] = root;
-          if (d <= T(0) && !info_set) {
-            *info = k0 + j + 1;
-            info_set = 1;
-          }
-        }
-      }
-      __syncthreads();
-      if (i > j && i < nb) {
-        const T lij = cv[i];
-#pragma unroll
-        for (int cc = 0; cc < 16; cc++) {
-          const int c = 16 * q + cc;
-          if (c > j && c <= i) R[cc] = R[cc] - lij * cv[c];
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int cc = 0; cc < 16; cc++) {
-    const int c = 16 * q + cc;
-    if (i < nb && c <= i) A[(int64_t)(k0 + i) * lda + k0 + c] = R[cc];
-  }
-}
-
 template <typename T>
 __global__ void diag_kernel(int n, const T* __restrict__ A, int lda, T* __restrict__ d) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -867,15 +806,6 @@ int zero_info(nmx_ctx* ctx, int32_t* info) {
 }
 
 template <typename T>
-int potrf_diag_launch(nmx_ctx* ctx, T* A, int lda, int k0, int nb, int32_t* info) {
-  if (nb > 64) return NMX_ERR_UNSUPPORTED;
-  ProfScope ps(ctx, K_POTRF_DIAG, (double)nb * nb * nb / 3.0, 2.0 * sizeof(T) * nb * nb);
-  potrf_diag_kernel<T><<<1, 256, 0, ctx->stream>>>(A, lda, k0, nb, info);
-  NMX_HIP(ctx, hipGetLastError());
-  return NMX_OK;
-}
-
-template <typename T>
 int tril_launch(nmx_ctx* ctx, int n, T* A, int lda) {
   int64_t total = (int64_t)n * n;
   if (total <= 0) return NMX_OK;
@@ -890,7 +820,6 @@ int tril_launch(nmx_ctx* ctx, int n, T* A, int lda) {
   template int laswp_launch<T>(nmx_ctx*, T*, int, int, int, int, int, const int32_t*, int, int);                   \
   template int getf2_leaf_launch<T>(nmx_ctx*, int, T*, int, int, int, int, int32_t*, int32_t*, int);               \
   template int diag_launch<T>(nmx_ctx*, int, const T*, int, T*);                                                   \
-  template int potrf_diag_launch<T>(nmx_ctx*, T*, int, int, int, int32_t*);                                        \
   template int tril_launch<T>(nmx_ctx*, int, T*, int);
 INST(double)
 INST(float)

@@ -27,71 +27,9 @@
 // non-finite inverse or solution solves its vectors again by plain
 // substitution, so that an infinity or NaN spreads as far as substitution
 // spreads it and no further.
-#include "nmx_internal.h"
+#include "tile16.h"
 
 namespace {
-
-typedef double d4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-template <typename T>
-struct Acc {
-  typedef f4 type;
-};
-template <>
-struct Acc<double> {
-  typedef d4 type;
-};
-__device__ __forceinline__ d4 mma(double a, double b, d4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ f4 mma(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-// row of output item e of lane l; also the contraction index of step e
-template <typename T>
-__device__ __forceinline__ int acc_row(int lane, int e) {
-  return sizeof(T) == 8 ? (lane >> 4) + 4 * e : 4 * (lane >> 4) + e;
-}
-
-template <int L>
-__device__ __forceinline__ float row_bcast(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + L, 0xF, 0xF, true));
-}
-template <int L>
-__device__ __forceinline__ double row_bcast(double v) {
-  const uint64_t b = (uint64_t)__double_as_longlong(v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, 0x150 + L, 0xF, 0xF, true);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), 0x150 + L, 0xF, 0xF, true);
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
-template <typename T>
-__device__ __forceinline__ bool finite(T v) {
-  return fabs(v) <= (sizeof(T) == 8 ? (T)1.7976931348623157e308 : (T)3.4028234663852886e38f);
-}
-
-// s += x(lane I of the 16-lane row) * y, the broadcast as the DPP operand of the
-// multiply-add.  s_nop 1: the two wait states between a vector write and a DPP
-// read of the same register.
-template <int I>
-__device__ __forceinline__ void fmac_bcast(float& s, float x, float y) {
-  asm volatile("s_nop 1\nv_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(s) : "v"(x), "v"(y), "n"(I));
-}
-template <int I>
-__device__ __forceinline__ void fmac_bcast(double& s, double x, double y) {
-  asm volatile("s_nop 1\nv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(s) : "v"(x), "v"(y), "n"(I));
-}
-
-// Row I of column c of the inverse of the lower triangular block whose rows
-// the 16 lanes hold (m: row `lane % 16`, rinv: the reciprocal of its diagonal);
-// ny is the inverse's column negated.
-template <int I, typename T>
-__device__ __forceinline__ void invert_rows(const T (&m)[16], T rinv, int c, T (&ny)[16]) {
-  if constexpr (I < 16) {
-    T s0 = I == c ? T(1) : T(0), s1 = T(0);
-#pragma unroll
-    for (int j = 0; j < I; j++) fmac_bcast<I>(j & 1 ? s1 : s0, m[j], ny[j]);
-    const T q = (s0 + s1) * row_bcast<I>(rinv);
-    ny[I] = I < c ? T(0) : -q;
-    invert_rows<I + 1, T>(m, rinv, c, ny);
-  }
-}
 
 struct StripArgs {
   int n, nvec;
@@ -259,8 +197,7 @@ trsm_strip_kernel(StripArgs a, const T* __restrict__ Tm, T* __restrict__ B) {
       L.inv[4 * lk + w][i][lc] = -ny[i];
     }
   }
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_order();
   T iv[NS][4];
 #pragma unroll
   for (int u = 0; u < NS; u++)

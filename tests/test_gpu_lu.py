@@ -342,3 +342,39 @@ def test_triangular_strip_spreads_infinities_as_substitution_does():
         np.testing.assert_array_equal(np.isfinite(x), np.isfinite(xo))
         ok = np.isfinite(xo)
         np.testing.assert_allclose(x[ok], xo[ok], rtol=1e-10, atol=1e-12)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 33, 63, 64, 65, 127, 128, 129, 200, 255, 256, 257, 385])
+def test_cholesky_block_edges(n, dtype):
+    """The one-workgroup block at the edges of its 16-column steps and of the
+    64 / 128 / 256-column workgroups, ill-conditioned and strided: the factor's
+    backward error |L L^T - A| <= n eps diag(A)^(1/2) diag(A)^(1/2)^T (Higham,
+    Theorem 10.3, with a factor of 4), and memory right of the matrix left alone."""
+    from numax_amd import _lib
+    rng = np.random.default_rng(n)
+    q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    kappa = 1e10 if dtype == torch.float64 else 1e4
+    a = (q * np.geomspace(1.0, 1.0 / kappa, n)) @ q.T
+    a = 0.5 * (a + a.T)
+    A = torch.full((n, n + 3), 5.0, dtype=dtype, device="cuda")
+    A[:, :n] = torch.as_tensor(a, device="cuda").to(dtype)
+    a = A[:, :n].double().cpu().numpy()
+    info = torch.zeros(1, dtype=torch.int32, device="cuda")
+    _lib.check(nl._fn("potrf", dtype)(nl._ctx(A).handle, n, nl._ptr(A), n + 3, nl._ptr(info), 0), "potrf")
+    assert int(info.item()) == 0
+    low = A[:, :n].double().cpu().numpy()
+    assert np.array_equal(low, np.tril(low)) and bool((A[:, n:] == 5.0).all())
+    d = np.sqrt(np.diag(a))
+    err = np.tril(np.abs(low @ low.T - a))
+    assert np.all(err <= 4 * (n + 1) * torch.finfo(dtype).eps * np.outer(d, d))
+
+
+@pytest.mark.parametrize("n,at", [(40, 0), (40, 17), (130, 127), (300, 16), (300, 299)])
+def test_cholesky_reports_the_first_bad_pivot(n, at):
+    a = R.spd_matrix(n, n)
+    a[at, at] = -1.0
+    if at + 1 < n:
+        a[n - 1, n - 1] = -2.0  # a later one is not reported
+    with pytest.raises(nl.NumaxError, match=f"at index {at}\\)"):
+        nl.cholesky(a)
