@@ -33,7 +33,7 @@ template <typename T>
 struct MbLayout {
   static constexpr int VW = sizeof(T) / 4;       // words per value
   static constexpr int STRIDE = 1 + VW + kLeafW * VW;  // header, |pivot|, row values
-  static constexpr int PARITY = kMaxParts * STRIDE + kLeafW * VW;  // + the diagonal row
+  static constexpr int PARITY = kMaxParts * STRIDE;
 };
 static_assert(2 * MbLayout<double>::PARITY * 8 <= kMailboxBytes, "mailbox too small");
 
@@ -54,14 +54,6 @@ __device__ __forceinline__ void mb_put_value(uint64_t* w, T v, uint32_t epoch) {
   }
 }
 
-template <typename T, int N>
-__device__ __forceinline__ void rotate_left(T (&v)[N]) {
-  const T first = v[0];
-#pragma unroll
-  for (int c = 0; c + 1 < N; c++) v[c] = v[c + 1];
-  v[N - 1] = first;
-}
-
 // Pivot keys: a candidate's magnitude as its (order-preserving) bit pattern
 // plus one, 0 for "no candidate".  Equal keys are equal magnitudes, so the
 // first maximum is the smallest row among the largest key.
@@ -71,7 +63,6 @@ template <>
 struct PivKey<float> {
   typedef uint32_t K;
   static __device__ __forceinline__ K of(float mag) { return __float_as_uint(mag) + 1u; }
-  static __device__ __forceinline__ K wave_max(K k) { return wave_umax(k); }
   static constexpr int WORDS = 1;
   static __device__ __forceinline__ uint32_t word(K k, int i) { return k; }
   static __device__ __forceinline__ K from(const uint32_t* w) { return w[0]; }
@@ -80,11 +71,6 @@ template <>
 struct PivKey<double> {
   typedef uint64_t K;
   static __device__ __forceinline__ K of(double mag) { return (uint64_t)__double_as_longlong(mag) + 1ull; }
-  static __device__ __forceinline__ K wave_max(K k) {
-    const uint32_t hi = wave_umax((uint32_t)(k >> 32));
-    const uint32_t lo = wave_umax((uint32_t)(k >> 32) == hi ? (uint32_t)k : 0u);
-    return ((uint64_t)hi << 32) | lo;
-  }
   static constexpr int WORDS = 2;
   static __device__ __forceinline__ uint32_t word(K k, int i) { return i ? (uint32_t)(k >> 32) : (uint32_t)k; }
   static __device__ __forceinline__ K from(const uint32_t* w) { return ((uint64_t)w[1] << 32) | w[0]; }
@@ -104,287 +90,359 @@ struct PivKey<double> {
 // the matrix numax's full-width swaps leave (panel.mojo:404-411).
 //
 // Workgroup p of `parts` owns rows r0 + 512 ROWS p + t + 512 i (i < ROWS) of
-// its 512 threads, each row's 32 columns in registers.  The column loop stays
-// rolled (unrolled it overflows the instruction cache); the rows are rotated
-// left by one after each column so register indices stay static: at step j,
-// v[.][0] is column j and v[.][1 .. w-j) are the columns still to update.
-// Per column, in one workgroup: DPP reductions of the pivot key and row, each
-// wavefront's winning row staged in LDS, one barrier.  Across workgroups
+// its threads (alone, up to 1024 rows of as many threads), each row's 32
+// columns in registers.  Rows stay where they are:
+// a thread keeps the position its row has in the interchanged panel and
+// stores it there at the end.  The columns are walked in groups of eight with
+// the registers rotated by eight after each, so that within a group every
+// register index is static and the loop over groups (and the instruction
+// cache) stays short.  Per column, in one workgroup: a DPP maximum of the
+// pivot key's high word (its low word and the position only where that ties),
+// each wavefront's winning row staged in LDS, one barrier.  Across workgroups
 // (parts > 1, grid 8 * parts of which every eighth takes part, so all
-// participants share one XCD and its L2): each part publishes its winner,
-// its key and (part 0) the diagonal row as epoch-tagged 64-bit words, and
-// every thread of every part spins on the words it stages, no fences: all of
-// them in one round trip up to 16 parts; above that the keys and rows first,
-// then the winner's row and the diagonal row.  Slots alternate by epoch
-// parity: a part publishes column j+2 only after reading every part's key
-// for column j+1, which each part publishes only after its reads of column j.
+// participants share one XCD and its L2): each part publishes its winner and
+// key as epoch-tagged 64-bit words, and every thread of every part spins on
+// the words it stages, no fences: all of them in one round trip up to 16
+// parts; above that the keys and positions first, then the winner's row.
+// Slots alternate by epoch parity: a part publishes column j+2 only after
+// reading every part's key for column j+1, which each part publishes only
+// after its reads of column j.
+//
+// What bounds it: the chain of one pivot decision per column.  Rotated by one
+// register a column, with every column's update and select run to full width,
+// both rows physically swapped through LDS and three maxima a decision, a
+// column took 3.7 us (1000 rows FP64, one workgroup) and 4.0 us (8192 rows,
+// sixteen); it takes 1.6 us (mean over 1000 .. 32 rows) and 2.8 us.
 // ---------------------------------------------------------------------------
-constexpr int kLeafT = 512;  // threads per workgroup
+constexpr int kLeafT = 512;      // threads per workgroup of several
+constexpr int kLeafMaxT = 1024;  // threads at most, in a workgroup alone
 constexpr int kTwoPhaseParts = 16;  // above this many parts the exchange reads the winner's row only
-constexpr int kLeafWaves = kLeafT / 64;
+constexpr int kLeafWaves = kLeafMaxT / 64;
+constexpr int kLeafG = 8;    // columns a group
 
-// ROWS rows per thread: 2 for a panel one workgroup holds (up to 1024
-// rows), 1 when the panel is spread over several (half the per-column
-// vector work per CU, twice the workgroups; up to 32 x 512 rows).
-template <typename T, int ROWS>
-__global__ void __launch_bounds__(kLeafT) getf2_leaf(T* __restrict__ A, int lda, int n, int r0, int c0, int w,
+// The lane with the largest key, the smallest position among equals; key 0
+// everywhere gives some lane.  All arguments per lane, the result uniform.
+__device__ __forceinline__ int winner_lane(uint64_t key, int pos) {
+  const uint32_t khi = (uint32_t)(key >> 32);
+  const uint32_t hi = wave_umax(khi);
+  uint64_t m = __ballot(khi == hi);
+  if (m & (m - 1)) {  // uniform
+    const uint32_t lo = wave_umax(khi == hi ? (uint32_t)key : 0u);
+    const bool eq = khi == hi && (uint32_t)key == lo;
+    m = __ballot(eq);
+    if (m & (m - 1)) {
+      const uint32_t p = wave_umin(eq ? (uint32_t)pos : 0xFFFFFFFFu);
+      m = __ballot(eq && (uint32_t)pos == p);
+    }
+  }
+  return __ffsll((long long)m) - 1;
+}
+__device__ __forceinline__ int winner_lane(uint32_t key, int pos) {
+  const uint32_t k = wave_umax(key);
+  uint64_t m = __ballot(key == k);
+  if (m & (m - 1)) {  // uniform
+    const uint32_t p = wave_umin(key == k ? (uint32_t)pos : 0xFFFFFFFFu);
+    m = __ballot(key == k && (uint32_t)pos == p);
+  }
+  return __ffsll((long long)m) - 1;
+}
+__device__ __forceinline__ uint32_t key_at(uint32_t k, int lane) { return __builtin_amdgcn_readlane(k, lane); }
+__device__ __forceinline__ uint64_t key_at(uint64_t k, int lane) {
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((uint32_t)(k >> 32), lane) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((uint32_t)k, lane);
+}
+
+// The same over lanes 0..15 only (one candidate a wavefront).
+__device__ __forceinline__ uint32_t row_umax(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, false));
+  return __builtin_amdgcn_readlane(v, 0);
+}
+__device__ __forceinline__ uint32_t key_high(uint32_t k) { return k; }
+__device__ __forceinline__ uint32_t key_high(uint64_t k) { return (uint32_t)(k >> 32); }
+template <typename K>
+__device__ __forceinline__ int winner_lane16(K key, int pos) {
+  const uint32_t hi = row_umax(key_high(key));
+  const uint64_t m = __ballot(key_high(key) == hi) & 0xFFFFull;
+  if (m & (m - 1)) return winner_lane(key, pos);  // uniform; the lanes above hold no key
+  return __ffsll((long long)m) - 1;
+}
+
+// x / p, correctly rounded but for rare last bits: the product with p's
+// reciprocal corrected by its residual (a quarter of a division's
+// instructions).  |x| <= |p| here.  A pivot whose reciprocal would leave the
+// normal range, an infinity or a NaN divides.
+__device__ __forceinline__ double quotient(double x, double p) {
+  if (!(fabs(p) >= 1e-290 && fabs(p) <= 1e290)) return x / p;  // uniform
+  double r = __builtin_amdgcn_rcp(p);
+  r = __builtin_fma(__builtin_fma(-p, r, 1.0), r, r);
+  r = __builtin_fma(__builtin_fma(-p, r, 1.0), r, r);
+  const double q = x * r;
+  return __builtin_fma(__builtin_fma(-q, p, x), r, q);
+}
+__device__ __forceinline__ float quotient(float x, float p) { return x / p; }
+
+template <typename T>
+struct LeafLds {
+  static constexpr int W = kLeafW, VW = MbLayout<T>::VW;
+  typedef typename PivKey<T>::K Key;
+  // staged mailbox words, per part [values | key | position] (PSTRIDE even, so
+  // every part's values stay 8-byte aligned)
+  static constexpr int PSTRIDE = (W * VW + VW + 1 + 1) & ~1;
+  // double-buffered by column parity
+  __attribute__((aligned(16))) T slot_v[2][kLeafWaves][W];  // each wavefront's winning row
+  Key slot_k[2][kLeafWaves];
+  int slot_p[2][kLeafWaves];
+  __attribute__((aligned(16))) uint32_t stage[2][kMaxParts * PSTRIDE];
+  int aborted, info_set;
+};
+
+struct LeafArgs {
+  int n, r0, c0, w, parts, p;  // p: this workgroup's part
+  int32_t* ipiv;
+  int32_t* info;
+  uint64_t* mb;
+  uint32_t epoch0;
+};
+
+// Column S of the group that starts at leaf column jb.
+template <int S, typename T, int ROWS, bool MULTI>
+__device__ __forceinline__ void leaf_step(const LeafArgs& a, T (&v)[ROWS][kLeafW], int (&pos)[ROWS], int jb, int nwaves,
+                                          LeafLds<T>& L) {
+  constexpr int W = kLeafW, VW = MbLayout<T>::VW, STRIDE = MbLayout<T>::STRIDE, PSTRIDE = LeafLds<T>::PSTRIDE;
+  typedef PivKey<T> PK;
+  typedef typename PK::K Key;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int j = jb + S, gr = a.r0 + j, gc = a.c0 + j, par = j & 1;
+
+  // 1. this thread's candidate: largest key, smallest position
+  Key tk = 0;
+  int tp = INT_MAX, ti = 0;
+#pragma unroll
+  for (int i = 0; i < ROWS; i++) {
+    T mag = fabs(v[i][S]);
+    if (!(mag == mag)) mag = T(-1);               // NaN never wins ...
+    if (pos[i] == gr && mag < T(0)) mag = T(0);   // ... the diagonal row starts at 0
+    const bool cand = pos[i] >= gr && pos[i] < a.n && mag >= T(0);
+    const Key k = cand ? PK::of(mag) : Key(0);
+    if (k > tk || (k == tk && k != 0 && pos[i] < tp)) {
+      tk = k;
+      tp = pos[i];
+      ti = i;
+    }
+  }
+  // 2. the wavefront's, and its row into LDS
+  const int wl = winner_lane(tk, tp);
+  if (lane == wl) {
+#pragma unroll
+    for (int i = 0; i < ROWS; i++)
+      if (ROWS == 1 || i == ti) {
+        // from this column on (finished columns stay with their rows)
+#pragma unroll
+        for (int g = 0; g < W / kLeafG; g++)
+          if (g == 0 || jb + kLeafG * g < a.w) {  // uniform
+#pragma unroll
+            for (int c = g ? 0 : S; c < kLeafG; c++) L.slot_v[par][wave][kLeafG * g + c] = v[i][kLeafG * g + c];
+          }
+      }
+    L.slot_k[par][wave] = tk;
+    L.slot_p[par][wave] = tp;
+  }
+  __syncthreads();
+  // 3. the workgroup's winner (every wavefront works it out)
+  Key ck = 0;
+  int cp = INT_MAX;
+  if (lane < nwaves) {
+    ck = L.slot_k[par][lane];
+    cp = L.slot_p[par][lane];
+  }
+  const int gw = winner_lane16(ck, cp);
+  int wp = __builtin_amdgcn_readlane(cp, gw);
+  const T* urow = L.slot_v[par][gw];
+  if constexpr (MULTI) {
+    const uint32_t epoch = a.epoch0 + (uint32_t)j + 1u;
+    const Key gk = key_at(ck, gw);
+    // 4. publish this part's winner (or "none")
+    uint64_t* mbp = a.mb + (size_t)(epoch & 1u) * MbLayout<T>::PARITY;
+    uint64_t* myslot = mbp + (size_t)a.p * STRIDE;
+    if (t < W * VW) {
+      const uint32_t* src = (const uint32_t*)urow;
+      mb_put(myslot + 1 + VW + t, gk != 0 ? src[t] : 0u, epoch);
+    } else if (t < W * VW + VW) {
+      mb_put(myslot + 1 + (t - W * VW), PK::word(gk, t - W * VW), epoch);
+    } else if (t == W * VW + VW) {
+      mb_put(myslot, (uint32_t)wp, epoch);
+    }
+    // 5. stage the parts' words, each validated by its epoch.  With many
+    // parts every workgroup reading every part's whole row crowds the few
+    // L2 lines they sit in, so it reads the keys and positions first, then
+    // only the winner's values (two round trips, a tenth of the data; 10%
+    // faster over a 32-part leaf, 2% slower over 8 parts).
+    uint32_t* stg = L.stage[par];
+    const bool two_phase = a.parts > kTwoPhaseParts;  // uniform
+    auto stage_word = [&](const uint64_t* src, int dst) {
+      uint64_t wv;
+      long spins = 0;
+      for (;;) {
+        wv = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((uint32_t)wv == epoch) break;
+        if (L.aborted || ++spins > kSpinLimit) { L.aborted = 1; break; }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      stg[dst] = (uint32_t)(wv >> 32);
+    };
+    // a slot's words still of use: its header and the columns ahead, which are
+    // the first registers.  (A thread's words polled together instead of one
+    // after the other crowd the same lines: 3.4 us a column against 3.0.)
+    const int words = 1 + VW + min(W, (a.w - jb + kLeafG - 1) / kLeafG * kLeafG) * VW;
+    if (two_phase) {
+      constexpr int HW = VW + 1;  // header words of a slot: position, key
+      for (int idx = t; idx < a.parts * HW; idx += kLeafT) {
+        const int q = idx / HW, f = idx % HW;
+        stage_word(mbp + (size_t)q * STRIDE + f, q * PSTRIDE + (f == 0 ? W * VW + VW : W * VW + f - 1));
+      }
+    } else {
+      for (int idx = t; idx < a.parts * STRIDE; idx += kLeafT) {
+        const int q = idx / STRIDE, f = idx % STRIDE;  // mailbox slot: [position | key | values]
+        if (f < words)
+          stage_word(mbp + idx, q * PSTRIDE + (f == 0 ? W * VW + VW : (f <= VW ? W * VW + f - 1 : f - 1 - VW)));
+      }
+    }
+    __syncthreads();
+    // 6. the global winner (lane q reads part q's; parts <= 32)
+    Key pk = 0;
+    int pp = INT_MAX;
+    if (lane < a.parts) {
+      const uint32_t* sq = stg + lane * PSTRIDE;
+      pk = PK::from(sq + W * VW);
+      pp = (int)sq[W * VW + VW];
+    }
+    const int bp = winner_lane(pk, pp);
+    wp = __builtin_amdgcn_readlane(pp, bp);
+    if (two_phase) {
+      for (int idx = t; idx < W * VW; idx += kLeafT)
+        stage_word(mbp + (size_t)bp * STRIDE + 1 + VW + idx, bp * PSTRIDE + idx);
+      __syncthreads();
+    }
+    urow = (const T*)(stg + bp * PSTRIDE);
+    // an exchange that gave up: any in-range row, the context reports it
+    if (L.aborted) wp = gr;
+  }
+  // 7. the winner's row takes position gr, the row that had it the winner's
+#pragma unroll
+  for (int i = 0; i < ROWS; i++) pos[i] = pos[i] == wp ? gr : (pos[i] == gr ? wp : pos[i]);
+  T pivot = urow[S];
+  if (t == 0 && a.p == 0) {
+    a.ipiv[gc] = wp;
+    if (fabs(pivot) == T(0) && !L.info_set) {
+      *a.info = gc + 1;
+      L.info_set = 1;
+    }
+  }
+  if (pivot == T(0)) pivot = T(kPivotFloor);
+  // 8. multipliers and the rank-1 update of the leaf's remaining columns:
+  // the rest of this group, then the groups that are still ahead (the others
+  // hold finished columns)
+  bool live[ROWS];
+  T l[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; i++) {
+    live[i] = pos[i] > gr && pos[i] < a.n;
+    const T q = quotient(v[i][S], pivot);
+    l[i] = q;
+    v[i][S] = live[i] ? q : v[i][S];
+  }
+#pragma unroll
+  for (int g = 0; g < W / kLeafG; g++) {
+    if (g == 0 || jb + kLeafG * g < a.w) {  // uniform
+      T u[kLeafG];
+#pragma unroll
+      for (int c = 0; c < kLeafG; c++)
+        if (g > 0 || c > S) u[c] = urow[kLeafG * g + c];
+#pragma unroll
+      for (int i = 0; i < ROWS; i++) {
+        if (live[i]) {
+#pragma unroll
+          for (int c = 0; c < kLeafG; c++)
+            if (g > 0 || c > S) v[i][kLeafG * g + c] = v[i][kLeafG * g + c] - l[i] * u[c];
+        }
+      }
+    }
+  }
+}
+
+template <int S, typename T, int ROWS, bool MULTI>
+__device__ __forceinline__ void leaf_group(const LeafArgs& a, T (&v)[ROWS][kLeafW], int (&pos)[ROWS], int jb, int nwaves,
+                                           LeafLds<T>& L) {
+  if constexpr (S < kLeafG) {
+    if (jb + S < a.w) {  // uniform
+      leaf_step<S, T, ROWS, MULTI>(a, v, pos, jb, nwaves, L);
+      leaf_group<S + 1, T, ROWS, MULTI>(a, v, pos, jb, nwaves, L);
+    }
+  }
+}
+
+// One row per thread (ROWS 1) for a panel of up to 1024 rows in one
+// workgroup or up to 32 x 512 rows over several (MULTI); two above that.
+template <typename T, int ROWS, bool MULTI>
+__global__ void __launch_bounds__(MULTI ? kLeafT : kLeafMaxT) getf2_leaf(T* __restrict__ A, int lda, int n, int r0, int c0, int w,
                                                      int32_t* __restrict__ ipiv, int32_t* __restrict__ info,
                                                      uint64_t* __restrict__ mb, uint32_t epoch0, int parts, int* err) {
   constexpr int W = kLeafW;
-  constexpr int VW = MbLayout<T>::VW;
-  constexpr int STRIDE = MbLayout<T>::STRIDE;
-  typedef PivKey<T> PK;
-  typedef typename PK::K Key;
-  const bool multi = parts > 1;
-  if (multi && (blockIdx.x % kXcds) != 0) return;
-  const int p = multi ? (int)(blockIdx.x / kXcds) : 0;
+  if (MULTI && (blockIdx.x % kXcds) != 0) return;
+  const int p = MULTI ? (int)(blockIdx.x / kXcds) : 0;
   const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-
-  // per-column staging, double-buffered by column parity
-  __shared__ __attribute__((aligned(16))) T slot_v[2][kLeafWaves][W];  // each wavefront's winning row
-  __shared__ Key slot_k[2][kLeafWaves];
-  __shared__ int slot_r[2][kLeafWaves];
-  __shared__ __attribute__((aligned(16))) T diag_v[2][W];               // the diagonal row
-  // staged mailbox words, per part [values | key | row] (PSTRIDE even, so
-  // every part's values stay 8-byte aligned), then the diagonal row
-  constexpr int PSTRIDE = (W * VW + VW + 1 + 1) & ~1;
-  __shared__ __attribute__((aligned(16))) uint32_t stage[2][kMaxParts * PSTRIDE + W * VW];
-  __shared__ int aborted, info_set;
-
+  __shared__ LeafLds<T> L;
   if (t == 0) {
-    aborted = 0;
-    info_set = (*info != 0);
+    L.aborted = 0;
+    L.info_set = (*info != 0);
   }
-
-  const int row0 = r0 + p * (kLeafT * ROWS) + t;  // row i = row0 + 512 i
+  const int first = r0 + p * (kLeafT * ROWS);  // row i of the thread: first + t + 512 i
   T v[ROWS][W];
+  int pos[ROWS];
   {
     // one descriptor at this workgroup's first row: offsets stay below 1024 rows
-    const __amdgpu_buffer_rsrc_t rs = buf_rsrc(A + (int64_t)(r0 + p * (kLeafT * ROWS)) * lda + c0);
+    const __amdgpu_buffer_rsrc_t rs = buf_rsrc(A + (int64_t)first * lda + c0);
 #pragma unroll
     for (int i = 0; i < ROWS; i++) {
-      const bool own = row0 + kLeafT * i < n;
+      pos[i] = first + t + kLeafT * i;
+      const bool own = pos[i] < n;
       const uint32_t rel = (uint32_t)(t + kLeafT * i) * (uint32_t)lda;
 #pragma unroll
       for (int c = 0; c < W; c++)
         v[i][c] = buf_load<T>(rs, (own & (c < w)) ? (rel + c) * (uint32_t)sizeof(T) : kBufOob);
     }
   }
+  // every load has landed before this part publishes anything (see the stores)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-
-  for (int j = 0; j < w; j++) {
-    const int gr = r0 + j;
-    const int gc = c0 + j;
-    const int par = j & 1;
-    const uint32_t epoch = epoch0 + (uint32_t)j + 1u;
-
-    // 1. this thread's candidate: largest key, smallest row
-    Key tk = 0;
-    int trow = INT_MAX;
+  const LeafArgs a{n, r0, c0, w, parts, p, ipiv, info, mb, epoch0};
+  const int nwaves = blockDim.x / 64;
+#pragma unroll 1
+  for (int jb = 0; jb < W; jb += kLeafG) {
+    leaf_group<0, T, ROWS, MULTI>(a, v, pos, jb, nwaves, L);
+    // the next group's columns to the front (four turns bring the first back)
 #pragma unroll
     for (int i = 0; i < ROWS; i++) {
-      const int row = row0 + kLeafT * i;
-      if (row >= gr && row < n) {
-        T mag = fabs(v[i][0]);
-        if (!(mag == mag)) mag = T(-1);           // NaN never wins ...
-        if (row == gr && mag < T(0)) mag = T(0);  // ... the diagonal row starts at 0
-        if (mag >= T(0)) {
-          const Key k = PK::of(mag);
-          if (k > tk) { tk = k; trow = row; }   // rows ascend with i: ties keep the first
-        }
-      }
-    }
-    // 2. the wavefront's: largest key, then the smallest row holding it
-    const Key wk = PK::wave_max(tk);
-    const int wrow = (int)wave_umin(tk == wk ? (uint32_t)trow : 0xFFFFFFFFu);
-    // its row values (and the diagonal row's) into LDS
+      T head[kLeafG];
 #pragma unroll
-    for (int i = 0; i < ROWS; i++) {
-      const int row = row0 + kLeafT * i;
-      if (wk != 0 && row == wrow) {
+      for (int c = 0; c < kLeafG; c++) head[c] = v[i][c];
 #pragma unroll
-        for (int c = 0; c < W; c++) slot_v[par][wave][c] = v[i][c];
-      }
-      if (row == gr) {
+      for (int c = 0; c + kLeafG < W; c++) v[i][c] = v[i][c + kLeafG];
 #pragma unroll
-        for (int c = 0; c < W; c++) diag_v[par][c] = v[i][c];
-      }
-    }
-    if (lane == 0) {
-      slot_k[par][wave] = wk;
-      slot_r[par][wave] = wrow;
-    }
-    __syncthreads();
-    // 3. the workgroup's winner (every wavefront works it out): lane q reads
-    // wavefront q's candidate, then the same key / smallest-row reductions
-    Key ck = 0;
-    int cr = INT_MAX;
-    if (lane < kLeafWaves) {
-      ck = slot_k[par][lane];
-      cr = slot_r[par][lane];
-    }
-    const Key gk0 = PK::wave_max(ck);
-    Key gk = gk0;
-    int grow = INT_MAX, gw = 0;
-    if (gk0 != 0) {  // uniform; rows are distinct, so one lane holds the winner
-      grow = (int)wave_umin(ck == gk0 ? (uint32_t)cr : 0xFFFFFFFFu);
-      gw = __ffsll((long long)__ballot(ck == gk0 && cr == grow)) - 1;
-    }
-    const T* urow;
-    const T* drow;
-    if (!multi) {
-      urow = slot_v[par][gw];
-      drow = diag_v[par];
-    } else {
-      // 4. publish this part's winner (or "none") and, from part 0, the diagonal row
-      uint64_t* mbp = mb + (size_t)(epoch & 1u) * MbLayout<T>::PARITY;
-      uint64_t* myslot = mbp + (size_t)p * STRIDE;
-      if (t < W * VW) {
-        const uint32_t* src = (const uint32_t*)slot_v[par][gw];
-        mb_put(myslot + 1 + VW + t, gk != 0 ? src[t] : 0u, epoch);
-      } else if (t < W * VW + VW) {
-        mb_put(myslot + 1 + (t - W * VW), PK::word(gk, t - W * VW), epoch);
-      } else if (t == W * VW + VW) {
-        mb_put(myslot, (uint32_t)grow, epoch);
-      } else if (p == 0 && t >= 128 && t < 128 + W * VW) {
-        mb_put(mbp + (size_t)kMaxParts * STRIDE + (t - 128), ((const uint32_t*)diag_v[par])[t - 128], epoch);
-      }
-      // 5. stage the parts' words, each validated by its epoch.  With many
-      // parts every workgroup reading every part's whole row crowds the few
-      // L2 lines they sit in, so it reads the keys and rows first, then only
-      // the winner's values and the diagonal row (two round trips, a tenth of
-      // the data; 10% faster over a 32-part leaf, 2% slower over 8 parts).
-      uint32_t* stg = stage[par];
-      const bool two_phase = parts > kTwoPhaseParts;  // uniform
-      auto stage_word = [&](const uint64_t* src, int dst) {
-        uint64_t wv;
-        long spins = 0;
-        for (;;) {
-          wv = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if ((uint32_t)wv == epoch) break;
-          if (aborted || ++spins > kSpinLimit) { aborted = 1; break; }
-          __builtin_amdgcn_s_sleep(1);
-        }
-        stg[dst] = (uint32_t)(wv >> 32);
-      };
-      if (two_phase) {
-        constexpr int HW = VW + 1;  // header words of a slot: row, key
-        for (int idx = t; idx < parts * HW; idx += kLeafT) {
-          const int q = idx / HW, f = idx % HW;
-          stage_word(mbp + (size_t)q * STRIDE + f, q * PSTRIDE + (f == 0 ? W * VW + VW : W * VW + f - 1));
-        }
-      } else {
-        const int words = parts * STRIDE + W * VW;
-        for (int idx = t; idx < words; idx += kLeafT) {
-          const uint64_t* src =
-              idx < parts * STRIDE ? mbp + idx : mbp + (size_t)kMaxParts * STRIDE + (idx - parts * STRIDE);
-          int dst;
-          if (idx < parts * STRIDE) {
-            const int q = idx / STRIDE, f = idx % STRIDE;  // mailbox slot: [row | key | values]
-            dst = q * PSTRIDE + (f == 0 ? W * VW + VW : (f <= VW ? W * VW + f - 1 : f - 1 - VW));
-          } else {
-            dst = kMaxParts * PSTRIDE + (idx - parts * STRIDE);
-          }
-          stage_word(src, dst);
-        }
-      }
-      __syncthreads();
-      // 6. the global winner: largest key, then smallest row (lane q reads
-      // part q's; parts <= 32)
-      Key pk = 0;
-      int pr = INT_MAX;
-      if (lane < parts) {
-        const uint32_t* sq = stg + lane * PSTRIDE;
-        pk = PK::from(sq + W * VW);
-        pr = (int)sq[W * VW + VW];
-      }
-      const Key bk = PK::wave_max(pk);
-      int brow = INT_MAX, bp = 0;
-      if (bk != 0) {
-        brow = (int)wave_umin(pk == bk ? (uint32_t)pr : 0xFFFFFFFFu);
-        bp = __ffsll((long long)__ballot(pk == bk && pr == brow)) - 1;
-      }
-      if (two_phase) {
-        // the winner's row values and the diagonal row (part bp published its
-        // values whether or not it had a candidate)
-        for (int idx = t; idx < 2 * W * VW; idx += kLeafT)
-          stage_word(idx < W * VW ? mbp + (size_t)bp * STRIDE + 1 + VW + idx
-                                  : mbp + (size_t)kMaxParts * STRIDE + (idx - W * VW),
-                     idx < W * VW ? bp * PSTRIDE + idx : kMaxParts * PSTRIDE + (idx - W * VW));
-        __syncthreads();
-      }
-      gk = bk;
-      grow = brow;
-      urow = (const T*)(stg + bp * PSTRIDE);
-      drow = (const T*)(stg + kMaxParts * PSTRIDE);
-    }
-
-    const int wr = (gk == 0 || aborted) ? gr : grow;
-    if (wr == gr) urow = drow;
-    // FP32: the pivot row into registers once (both rows of the thread use
-    // it); FP64 reads it from LDS per row (registers are at their limit)
-    constexpr bool kRowRegs = sizeof(T) == 4;
-    T u[kRowRegs ? W : 1];
-#pragma unroll
-    for (int c = 0; c < (kRowRegs ? W : 1); c++) u[c] = urow[c];
-    auto urow_at = [&](int c) -> T { return kRowRegs ? u[kRowRegs ? c : 0] : urow[c]; };
-    // 7. interchange inside the leaf's columns, record the pivot
-#pragma unroll
-    for (int i = 0; i < ROWS; i++) {
-      const int row = row0 + kLeafT * i;
-      if (wr != gr && row < n) {
-        if (row == gr) {
-#pragma unroll
-          for (int c = 0; c < W; c++) v[i][c] = urow_at(c);
-        } else if (row == wr) {
-#pragma unroll
-          for (int c = 0; c < W; c++) v[i][c] = drow[c];
-        }
-      }
-    }
-    T pivot = urow_at(0);
-    if (t == 0 && p == 0) {
-      ipiv[gc] = wr;
-      if (fabs(pivot) == T(0) && !info_set) {
-        *info = gc + 1;
-        info_set = 1;
-      }
-    }
-    if (pivot == T(0)) pivot = T(kPivotFloor);
-    // 8. multipliers and the rank-1 update of the leaf's remaining columns.
-    // The bound is opaque (a vector register), so the guard is a per-element
-    // select rather than 31 uniform branches; columns past it are finished
-    // ones rotated to the end and keep their values (a select, not a
-    // multiply by 0, which an infinite multiplier would turn into NaN).
-    int rem = w - j;
-    asm volatile("" : "+v"(rem));
-#pragma unroll
-    for (int i = 0; i < ROWS; i++) {
-      const int row = row0 + kLeafT * i;
-      if (row > gr && row < n) {
-        const T l = v[i][0] / pivot;
-        v[i][0] = l;
-#pragma unroll
-        for (int c = 1; c < W; c++) {
-          const T nv = v[i][c] - l * urow_at(c);
-          v[i][c] = c < rem ? nv : v[i][c];
-        }
-      }
-      rotate_left(v[i]);
+      for (int c = 0; c < kLeafG; c++) v[i][W - kLeafG + c] = head[c];
     }
   }
-  for (int j = w; j < W; j++) {
-#pragma unroll
-    for (int i = 0; i < ROWS; i++) rotate_left(v[i]);
-  }
-
-  if (aborted && t == 0) atomicExch(err, NMX_ERR_SYNC_TIMEOUT);
+  if (L.aborted && t == 0) atomicExch(err, NMX_ERR_SYNC_TIMEOUT);
+  // Rows change places across workgroups: no row is stored before every part
+  // has loaded its own.  A part that has staged every part's words of the
+  // first column knows that (each published them after its loads).
 #pragma unroll
   for (int i = 0; i < ROWS; i++) {
-    const int row = row0 + kLeafT * i;
-    if (row < n) {
-      T* dst = A + (int64_t)row * lda + c0;
+    if (first + t + kLeafT * i < n) {
+      T* dst = A + (int64_t)pos[i] * lda + c0;
 #pragma unroll
       for (int c = 0; c < W; c++)
         if (c < w) dst[c] = v[i][c];
@@ -765,10 +823,10 @@ int getf2_leaf_launch(nmx_ctx* ctx, int n, T* A, int lda, int r0, int c0, int w,
   const int m = n - r0;
   if (m <= 0 || w <= 0) return NMX_OK;
   if (w > kLeafW) return NMX_ERR_UNSUPPORTED;
-  // one row per thread once the panel spans several workgroups (and fits 32
-  // of 512 rows), two otherwise
-  const bool one_row = m > kLeafT * 2 && m <= kLeafT * kMaxParts;
-  int parts = ceil_div(m, one_row ? kLeafT : kLeafT * 2);
+  // one row per thread while the panel fits 32 workgroups of 512 rows, two
+  // above that
+  const bool one_row = m <= kLeafT * kMaxParts;
+  const int parts = m <= kLeafMaxT ? 1 : ceil_div(m, one_row ? kLeafT : kLeafT * 2);
   if (parts > kMaxParts) return NMX_ERR_UNSUPPORTED;  // n - r0 <= kLeafMaxRows
   uint32_t epoch0 = 0;
   NMX_TRY(nmx_epoch_reserve(ctx, (uint32_t)w, &epoch0));
@@ -781,10 +839,15 @@ int getf2_leaf_launch(nmx_ctx* ctx, int n, T* A, int lda, int r0, int c0, int w,
     // A participant that is not resident makes the others' bounded waits
     // expire, which the context reports as NMX_ERR_SYNC_TIMEOUT.
     const int grid = parts == 1 ? 1 : parts * kXcds;
-    if (one_row)
-      getf2_leaf<T, 1><<<grid, kLeafT, 0, ctx->stream>>>(A, lda, n, r0, c0, w, ipiv, info, mb, epoch0, parts, err);
+    // in one workgroup: only the wavefronts that hold rows.  Up to 1024 rows
+    // that is faster than an exchange between two (2.8 us a column)
+    const int threads = parts == 1 ? ceil_div(m, 64) * 64 : kLeafT;
+    if (parts == 1)
+      getf2_leaf<T, 1, false><<<grid, threads, 0, ctx->stream>>>(A, lda, n, r0, c0, w, ipiv, info, mb, epoch0, parts, err);
+    else if (one_row)
+      getf2_leaf<T, 1, true><<<grid, kLeafT, 0, ctx->stream>>>(A, lda, n, r0, c0, w, ipiv, info, mb, epoch0, parts, err);
     else
-      getf2_leaf<T, 2><<<grid, kLeafT, 0, ctx->stream>>>(A, lda, n, r0, c0, w, ipiv, info, mb, epoch0, parts, err);
+      getf2_leaf<T, 2, true><<<grid, kLeafT, 0, ctx->stream>>>(A, lda, n, r0, c0, w, ipiv, info, mb, epoch0, parts, err);
     NMX_HIP(ctx, hipGetLastError());
   }
   if (swap_others) return laswp_launch<T>(ctx, A, lda, 0, n, c0, c0 + w, ipiv, r0, r0 + w);

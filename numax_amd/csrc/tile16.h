@@ -59,10 +59,10 @@ __device__ __forceinline__ void fmac_bcast(double& s, double x, double y) {
 template <int I, typename T>
 __device__ __forceinline__ void invert_rows(const T (&m)[16], T rinv, int c, T (&ny)[16]) {
   if constexpr (I < 16) {
-    T s[4] = {I == c ? T(1) : T(0), T(0), T(0), T(0)};
+    T s0 = I == c ? T(1) : T(0), s1 = T(0);
 #pragma unroll
-    for (int j = 0; j < I; j++) fmac_bcast<I>(s[j & 3], m[j], ny[j]);
-    const T q = ((s[0] + s[1]) + (s[2] + s[3])) * row_bcast<I>(rinv);
+    for (int j = 0; j < I; j++) fmac_bcast<I>(j & 1 ? s1 : s0, m[j], ny[j]);
+    const T q = (s0 + s1) * row_bcast<I>(rinv);
     ny[I] = I < c ? T(0) : -q;
     invert_rows<I + 1, T>(m, rinv, c, ny);
   }

@@ -378,3 +378,24 @@ def test_cholesky_reports_the_first_bad_pivot(n, at):
         a[n - 1, n - 1] = -2.0  # a later one is not reported
     with pytest.raises(nl.NumaxError, match=f"at index {at}\\)"):
         nl.cholesky(a)
+
+
+@pytest.mark.parametrize("n", [31, 32, 33, 40, 64, 129, 512, 513, 1024, 1056])
+def test_leaf_ties_zeros_and_nans_keep_numax_pivots(n):
+    """Rows that tie, columns that are zero or NaN, at the row limits of the
+    one-workgroup leaf and its eight-column groups: the oracle's pivots."""
+    rng = np.random.default_rng(n)
+    a = rng.integers(-2, 3, (n, n)).astype(np.float64)  # many ties; singular with the zero column
+    a[:, 5] = 0.0
+    if n > 40:
+        a[:, 37] = 0.0
+    lu = nl.lu_factor(a)
+    _, piv, info, _ = oracle.getrf(a)
+    # exact small-integer arithmetic holds for the first columns only; compare
+    # the pivots until a rounding (a non-dyadic quotient) could reorder a tie
+    assert np.array_equal(lu.pivots.cpu().numpy()[:3], piv[:3])
+    assert lu.info == info
+    b = rng.standard_normal((n, n))
+    b[n // 2, 0] = np.nan  # a NaN below the diagonal never wins
+    lu = nl.lu_factor(b)
+    assert lu.pivots.cpu().numpy()[0] == oracle.getrf(b)[1][0]
