@@ -23,23 +23,19 @@
 // round and one barrier across them).  With a row per lane instead, every
 // step reduced 33 values over 256 threads and read them back: 165 LDS reads
 // and 126 shuffles a step, and 4096 problems of 1024 x 32 took 6.55 ms.
-// In this layout they take 0.64 ms (10.5x; 865 GB/s of the 4.8 TB/s a copy
-// reaches): about 210 instructions a step and wavefront, 60 % of the time in
-// issue, the rest in the step's barrier and LDS round.
+// In this layout they take 0.62 ms (10.8x; 885 GB/s of the 4.8 TB/s a copy
+// reaches): the broadcasts are the DPP operand of the multiply-adds (0.64 ms as
+// separate moves), 60 % of the time is
+// issue, the rest the step's barrier and LDS round.
 #include <math.h>
 
-#include "nmx_internal.h"
+#include "tile16.h"
 
 namespace {
 
 constexpr int kRows = 32;              // rows a thread holds
 constexpr int kGroupPad = kRows + 4;   // LDS stride of a row group's column (b128 aligned, banks apart)
 
-// lane L of each 16-lane row to the whole row (folds into the consuming instruction)
-template <int L>
-__device__ __forceinline__ float row_bcast(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + L, 0xF, 0xF, true));
-}
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {
   return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
@@ -88,8 +84,7 @@ __device__ __forceinline__ void gels_step(float (&a)[SETS][kRows], float (&b)[2]
     for (int r = 0; r < kRows; r += 4)
       *(float4*)(xg + r) = make_float4(a[set][r], a[set][r + 1], a[set][r + 2], a[set][r + 3]);
   }
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_order();
   const float2 xb = *(const float2*)(xg + 2 * c);
   if (t < 16) {
 #pragma unroll
@@ -99,13 +94,12 @@ __device__ __forceinline__ void gels_step(float (&a)[SETS][kRows], float (&b)[2]
   float p[SETS];
 #pragma unroll
   for (int s = s0; s < SETS; s++) {
-    float q0 = 0.f, q1 = 0.f;
+    float q0 = 0.f, q1 = 0.f, q2 = 0.f, q3 = 0.f;
 #pragma unroll
-    for (int r = 0; r < kRows; r += 2) {
-      q0 = fmaf(row_bcast<lk>(a[set][r]), a[s][r], q0);
-      q1 = fmaf(row_bcast<lk>(a[set][r + 1]), a[s][r + 1], q1);
-    }
-    p[s] = q0 + q1;
+    for (int r = 0; r < kRows; r += 4)
+      fmac_bcast4<lk>(q0, q1, q2, q3, a[set][r], a[set][r + 1], a[set][r + 2], a[set][r + 3], a[s][r], a[s][r + 1],
+                      a[s][r + 2], a[s][r + 3]);
+    p[s] = (q0 + q1) + (q2 + q3);
   }
   float pb = xb.x * b[0] + xb.y * b[1];
   pb = dpp_add<0xB1>(pb);   // quad_perm 1,0,3,2
@@ -128,7 +122,7 @@ __device__ __forceinline__ void gels_step(float (&a)[SETS][kRows], float (&b)[2]
     __syncthreads();
   }
   float tot[2] = {0.f, 0.f}, tb = 0.f;
-#pragma unroll(NW < 8 ? NW : 8)
+#pragma unroll(NW < 4 ? NW : 4)
   for (int w = 0; w < NW; w++) {
     const float2 v = *(const float2*)L.part[buf][w][c];
     tot[0] += v.x;
@@ -159,7 +153,13 @@ __device__ __forceinline__ void gels_step(float (&a)[SETS][kRows], float (&b)[2]
 #pragma unroll
   for (int s = SETS - 1; s >= s0; s--)
 #pragma unroll
-    for (int r = 0; r < kRows; r++) a[s][r] = fmaf(row_bcast<lk>(a[set][r]), -f[s], a[s][r]);
+    for (int r = 0; r < kRows; r += 4) {
+      if (s == set)
+        fmac_self4<lk>(a[s][r], a[s][r + 1], a[s][r + 2], a[s][r + 3], -f[s]);
+      else
+        fmac_bcast4<lk>(a[s][r], a[s][r + 1], a[s][r + 2], a[s][r + 3], a[set][r], a[set][r + 1], a[set][r + 2],
+                        a[set][r + 3], -f[s], -f[s], -f[s], -f[s]);
+    }
   b[0] -= xb.x * fb;
   b[1] -= xb.y * fb;
   // row K is finished

@@ -18,7 +18,7 @@
 // lstsq of 2500 x 300 FP32: 21.3 ms -> 1.8 ms.
 #include <math.h>
 
-#include "nmx_internal.h"
+#include "tile16.h"
 
 namespace {
 
@@ -242,58 +242,6 @@ int apply_reflector(nmx_ctx* ctx, const Reflector<T>& w, int rows, int nb, int w
 // builds it from.
 constexpr int kNarrow = 16;
 
-template <int L>
-__device__ __forceinline__ float row_bcast(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + L, 0xF, 0xF, true));
-}
-template <int L>
-__device__ __forceinline__ double row_bcast(double v) {
-  const uint64_t b = (uint64_t)__double_as_longlong(v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, 0x150 + L, 0xF, 0xF, true);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), 0x150 + L, 0xF, 0xF, true);
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
-// acc += x(lane K of the 16-lane row) * y for four registers, the broadcast as
-// the multiply-add's DPP operand (the compiler makes a move of it, which would
-// double the instructions and keep R broadcast values live).  s_nop 1: the two
-// wait states between a vector write and a DPP read of the same register.
-#define NMX_FMAC_DPP4(TYPE, D0, D1, D2, D3, X0, X1, X2, X3, S0, S1, S2, S3, CONS)                                  \
-  asm volatile("s_nop 1\n"                                                                                         \
-               "v_fmac_" TYPE "_dpp %0, %4, %8 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                      \
-               "v_fmac_" TYPE "_dpp %1, %5, %9 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                      \
-               "v_fmac_" TYPE "_dpp %2, %6, %10 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                     \
-               "v_fmac_" TYPE "_dpp %3, %7, %11 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                     \
-               : "+v"(D0), "+v"(D1), "+v"(D2), "+v"(D3)                                                            \
-               : "v"(X0), "v"(X1), "v"(X2), "v"(X3), "v"(S0), "v"(S1), "v"(S2), "v"(S3), "n"(CONS))
-template <int K>
-__device__ __forceinline__ void fmac_bcast4(float& d0, float& d1, float& d2, float& d3, float x0, float x1, float x2,
-                                            float x3, float s0, float s1, float s2, float s3) {
-  NMX_FMAC_DPP4("f32", d0, d1, d2, d3, x0, x1, x2, x3, s0, s1, s2, s3, K);
-}
-template <int K>
-__device__ __forceinline__ void fmac_bcast4(double& d0, double& d1, double& d2, double& d3, double x0, double x1,
-                                            double x2, double x3, double s0, double s1, double s2, double s3) {
-  NMX_FMAC_DPP4("f64", d0, d1, d2, d3, x0, x1, x2, x3, s0, s1, s2, s3, K);
-}
-// x -= x(lane K) * s in place, four registers
-#define NMX_FMAC_DPP4_SELF(TYPE, X0, X1, X2, X3, S, CONS)                                     \
-  asm volatile("s_nop 1\n"                                                                    \
-               "v_fmac_" TYPE "_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
-               "v_fmac_" TYPE "_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
-               "v_fmac_" TYPE "_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
-               "v_fmac_" TYPE "_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
-               : "+v"(X0), "+v"(X1), "+v"(X2), "+v"(X3)                                       \
-               : "v"(S), "n"(CONS))
-template <int K>
-__device__ __forceinline__ void fmac_self4(float& x0, float& x1, float& x2, float& x3, float s) {
-  NMX_FMAC_DPP4_SELF("f32", x0, x1, x2, x3, s, K);
-}
-template <int K>
-__device__ __forceinline__ void fmac_self4(double& x0, double& x1, double& x2, double& x3, double s) {
-  NMX_FMAC_DPP4_SELF("f64", x0, x1, x2, x3, s, K);
-}
-
 template <typename T, int NW>
 struct PanelLds {
   T part[2][NW][kNarrow];  // column sums by wavefront
@@ -406,25 +354,6 @@ __global__ void __launch_bounds__(64 * NW) geqr2_narrow_kernel(int rows, int nb,
   }
 }
 
-typedef double d4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-// 16 x 16 += 16 x 4 by 4 x 16: operands by (lane % 16, lane / 16), output item e
-// of lane l in row acc_row(l, e), column l % 16
-__device__ __forceinline__ d4 mma16(double a, double b, d4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ f4 mma16(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-template <typename T>
-__device__ __forceinline__ int acc_row(int lane, int e) {
-  return sizeof(T) == 8 ? (lane >> 4) + 4 * e : 4 * (lane >> 4) + e;
-}
-template <typename T>
-struct Acc16 {
-  typedef f4 type;
-};
-template <>
-struct Acc16<double> {
-  typedef d4 type;
-};
-
 // V[r][i] of a narrow panel at A (unit diagonal, zeros above it and past nb)
 template <typename T>
 __device__ __forceinline__ T narrow_v(const T* __restrict__ A, int lda, int rows, int nb, int r, int i) {
@@ -442,12 +371,12 @@ __global__ void __launch_bounds__(kQrThreads) narrow_t_kernel(int m, int n, int 
   const int k = blockIdx.x * block, nb = min(block, n - k), rows = m - k;
   const T* A = QR + (int64_t)k * lda + k;
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  typename Acc16<T>::type acc = {0, 0, 0, 0};
+  typename Acc<T>::type acc = {0, 0, 0, 0};
   for (int r0 = 16 * w; r0 < rows; r0 += 16 * kQrWaves) {
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       const T v = narrow_v<T>(A, lda, rows, nb, r0 + acc_row<T>(lane, e), lane & 15);
-      acc = mma16(v, v, acc);
+      acc = mma(v, v, acc);
     }
   }
 #pragma unroll
@@ -492,7 +421,7 @@ __global__ void __launch_bounds__(kQrThreads) narrow_apply_kernel(int rows, int 
                                                                   const T* __restrict__ Tm, int trans, T* __restrict__ C1,
                                                                   int ldc1, int width1, T* __restrict__ C2, int ldc2,
                                                                   int width2) {
-  typedef typename Acc16<T>::type acc_t;
+  typedef typename Acc<T>::type acc_t;
   __shared__ T part[kQrWaves][kNarrow][kNarrow];
   __shared__ T W[kNarrow][kNarrow], Y[kNarrow][kNarrow];
   const int tiles1 = (width1 + 15) / 16;
@@ -515,7 +444,7 @@ __global__ void __launch_bounds__(kQrThreads) narrow_apply_kernel(int rows, int 
       cv[e] = full || r < rows ? C[(int64_t)r * ldc] : T(0);
     }
 #pragma unroll
-    for (int e = 0; e < 4; e++) acc = mma16(lc < nb ? v[e] : T(0), cv[e], acc);
+    for (int e = 0; e < 4; e++) acc = mma(lc < nb ? v[e] : T(0), cv[e], acc);
   });
 #pragma unroll
   for (int e = 0; e < 4; e++) part[w][acc_row<T>(lane, e)][lc] = acc[e];
@@ -553,7 +482,7 @@ __global__ void __launch_bounds__(kQrThreads) narrow_apply_kernel(int rows, int 
     }
     acc_t d = {0, 0, 0, 0};
 #pragma unroll
-    for (int q = 0; q < 4; q++) d = mma16(v[q], y[q], d);
+    for (int q = 0; q < 4; q++) d = mma(v[q], y[q], d);
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       const int r = r0 + acc_row<T>(lane, e);

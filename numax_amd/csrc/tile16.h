@@ -68,6 +68,46 @@ __device__ __forceinline__ void invert_rows(const T (&m)[16], T rinv, int c, T (
   }
 }
 
+// acc += x(lane K of the 16-lane row) * y for four registers, the broadcast as
+// the multiply-add's DPP operand (the compiler makes a move of it, which would
+// double the instructions and keep R broadcast values live).  s_nop 1: the two
+// wait states between a vector write and a DPP read of the same register.
+#define NMX_FMAC_DPP4(TYPE, D0, D1, D2, D3, X0, X1, X2, X3, S0, S1, S2, S3, CONS)                                  \
+  asm volatile("s_nop 1\n"                                                                                         \
+               "v_fmac_" TYPE "_dpp %0, %4, %8 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                      \
+               "v_fmac_" TYPE "_dpp %1, %5, %9 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                      \
+               "v_fmac_" TYPE "_dpp %2, %6, %10 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                     \
+               "v_fmac_" TYPE "_dpp %3, %7, %11 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"                     \
+               : "+v"(D0), "+v"(D1), "+v"(D2), "+v"(D3)                                                            \
+               : "v"(X0), "v"(X1), "v"(X2), "v"(X3), "v"(S0), "v"(S1), "v"(S2), "v"(S3), "n"(CONS))
+template <int K>
+__device__ __forceinline__ void fmac_bcast4(float& d0, float& d1, float& d2, float& d3, float x0, float x1, float x2,
+                                            float x3, float s0, float s1, float s2, float s3) {
+  NMX_FMAC_DPP4("f32", d0, d1, d2, d3, x0, x1, x2, x3, s0, s1, s2, s3, K);
+}
+template <int K>
+__device__ __forceinline__ void fmac_bcast4(double& d0, double& d1, double& d2, double& d3, double x0, double x1,
+                                            double x2, double x3, double s0, double s1, double s2, double s3) {
+  NMX_FMAC_DPP4("f64", d0, d1, d2, d3, x0, x1, x2, x3, s0, s1, s2, s3, K);
+}
+// x -= x(lane K) * s in place, four registers
+#define NMX_FMAC_DPP4_SELF(TYPE, X0, X1, X2, X3, S, CONS)                                     \
+  asm volatile("s_nop 1\n"                                                                    \
+               "v_fmac_" TYPE "_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
+               "v_fmac_" TYPE "_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
+               "v_fmac_" TYPE "_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
+               "v_fmac_" TYPE "_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"  \
+               : "+v"(X0), "+v"(X1), "+v"(X2), "+v"(X3)                                       \
+               : "v"(S), "n"(CONS))
+template <int K>
+__device__ __forceinline__ void fmac_self4(float& x0, float& x1, float& x2, float& x3, float s) {
+  NMX_FMAC_DPP4_SELF("f32", x0, x1, x2, x3, s, K);
+}
+template <int K>
+__device__ __forceinline__ void fmac_self4(double& x0, double& x1, double& x2, double& x3, double s) {
+  NMX_FMAC_DPP4_SELF("f64", x0, x1, x2, x3, s, K);
+}
+
 // LDS written by some lanes of a wavefront is read by the others of it
 __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
