@@ -16,34 +16,9 @@
 // Tile order is XCD-aware: workgroup b runs on XCD b % 8, so each XCD is
 // given a contiguous run of tiles (grouped 8 tile-rows at a time) and the
 // A row-panels and B column-panels it reads stay in that XCD's L2.
-#include "nmx_internal.h"
+#include "tile16.h"
 
 namespace {
-
-typedef double d4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-
-template <typename T>
-struct Mfma;
-
-template <>
-struct Mfma<double> {
-  typedef d4 acc_t;
-  static __device__ __forceinline__ acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  // Output item i of lane l sits at row l/16 + 4 i (measured on gfx950).
-  static __device__ __forceinline__ int row(int lane, int i) { return (lane >> 4) + 4 * i; }
-};
-
-template <>
-struct Mfma<float> {
-  typedef f4 acc_t;
-  static __device__ __forceinline__ acc_t mma(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lane, int i) { return 4 * (lane >> 4) + i; }
-};
 
 constexpr int BM = 128, BK = 16, PAD = 4;  // the large tile, K slab, LDS row pad
 
@@ -56,7 +31,7 @@ template <typename T, int TA, int TB, int TILE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 gemm_kernel(int M, int N, int K, T alpha, const T* __restrict__ A, int lda, const T* __restrict__ B, int ldb, T beta,
             T* __restrict__ C, int ldc, int tilesM, int tilesN, int lower_only, int ksplit, int kchunk, int64_t csplit) {
-  typedef typename Mfma<T>::acc_t acc_t;
+  typedef typename Acc<T>::type acc_t;
   // TILE x TILE of C per workgroup; each wavefront owns WT x WT = FR x FR
   // MFMA tiles; each thread stages LPT elements of each K slab
   constexpr int TM = TILE, TN = TILE, WT = TILE / 2, FR = WT / 16, LPT = TILE * BK / 256;
@@ -203,7 +178,7 @@ gemm_kernel(int M, int N, int K, T alpha, const T* __restrict__ A, int lda, cons
 #pragma unroll
       for (int i = 0; i < FR; i++)
 #pragma unroll
-        for (int j = 0; j < FR; j++) acc[i][j] = Mfma<T>::mma(af[cur][i], bf[cur][j], acc[i][j]);
+        for (int j = 0; j < FR; j++) acc[i][j] = mma(af[cur][i], bf[cur][j], acc[i][j]);
     }
     if (s + 1 < ksteps) {
       store_tiles(buf ^ 1);
@@ -223,7 +198,7 @@ gemm_kernel(int M, int N, int K, T alpha, const T* __restrict__ A, int lda, cons
       for (int j = 0; j < FR; j++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          const int lr = wm * WT + i * 16 + Mfma<T>::row(lane, e);
+          const int lr = wm * WT + i * 16 + acc_row<T>(lane, e);
           const int lc = wn * WT + j * 16 + (lane & 15);
           const uint32_t off =
               ((m0 + lr < M) & (n0 + lc < N)) ? ((uint32_t)lr * (uint32_t)ldc + (uint32_t)lc) * E : kBufOob;
@@ -237,12 +212,108 @@ gemm_kernel(int M, int N, int K, T alpha, const T* __restrict__ A, int lda, cons
       const int col = n0 + wn * WT + j * 16 + (lane & 15);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        const int row = m0 + wm * WT + i * 16 + Mfma<T>::row(lane, e);
+        const int row = m0 + wm * WT + i * 16 + acc_row<T>(lane, e);
         T v = alpha * acc[i][j][e];
         if (use_c) v += beta * cv[i][j][e];
         if ((row < M) & (col < N)) C[(int64_t)row * ldc + col] = v;
       }
     }
+}
+
+// Products too small for a tile per CU: a workgroup owns 16 x (16 NF) of C
+// and its wavefronts take every NW-th 16-deep slab of K, operands straight
+// from memory into MFMA registers (a lane's four contraction indices are
+// neighbours, so A's rows are read 16 B at a time), the partial tiles added
+// in LDS.  What bounds these is not the matrix cores but the chain of K
+// slabs one workgroup walks -- 64 x 64 tiles of a 256 x 16 x 256 update run
+// 16 slabs in turn, three quarters of each for columns that are not there --
+// and here that chain is K / (16 NW) slabs, four of them in flight.  Cholesky
+// and solve of order 8192 with 16 vectors: 14.6 -> 11.5 ms, LU 45.5 -> 43.4,
+// FP32 Cholesky of order 1301 1.21 -> 0.94.
+template <typename T, int TA, int TB, int NF>
+__global__ void __launch_bounds__(512)
+gemm_thin(int M, int N, int K, T alpha, const T* __restrict__ A, int lda, const T* __restrict__ B, int ldb, T beta,
+          T* __restrict__ C, int ldc, int lower_only) {
+  typedef typename Acc<T>::type acc_t;
+  constexpr int SL = 4 / NF < 2 ? 2 : 4 / NF;  // slabs in flight
+  __shared__ T part[8][16][16 * NF + 1];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = blockDim.x >> 6;
+  const int m0 = blockIdx.x * 16, n0 = blockIdx.y * 16 * NF;
+  const int c = lane & 15, k4 = 4 * (lane >> 4);
+  if (lower_only && n0 > m0 + 15) return;
+  // rows and columns past the edge read the last one and are not stored
+  const int row = min(m0 + c, M - 1);
+  const T* a = TA ? A + row : A + (int64_t)row * lda;
+  const T* b[NF];
+#pragma unroll
+  for (int f = 0; f < NF; f++) {
+    const int col = min(n0 + 16 * f + c, N - 1);
+    b[f] = TB ? B + (int64_t)col * ldb : B + col;
+  }
+  acc_t acc[NF];
+#pragma unroll
+  for (int f = 0; f < NF; f++) acc[f] = acc_t{0, 0, 0, 0};
+  auto quad = [&](auto trans, const T* p, int ld, int k, T(&r)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) r[e] = trans ? p[(int64_t)(k + e) * ld] : p[k + e];
+  };
+  const std::integral_constant<bool, TA != 0> ta{};
+  const std::integral_constant<bool, TB == 0> tb{};
+  const int full = K / 16;
+  int s = wave;
+  for (; s + (SL - 1) * nw < full; s += SL * nw) {
+    T ra[SL][4], rb[SL][NF][4];
+#pragma unroll
+    for (int u = 0; u < SL; u++) {
+      const int k = 16 * (s + u * nw) + k4;
+      quad(ta, a, lda, k, ra[u]);
+#pragma unroll
+      for (int f = 0; f < NF; f++) quad(tb, b[f], ldb, k, rb[u][f]);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // all slabs' loads go out before the first is waited for
+#pragma unroll
+    for (int u = 0; u < SL; u++)
+#pragma unroll
+      for (int f = 0; f < NF; f++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[f] = mma(ra[u][e], rb[u][f][e], acc[f]);
+  }
+  for (; 16 * s < K; s += nw) {
+    const int k = 16 * s + k4;
+    T ra[4], rb[NF][4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      // past K both factors are zero (a zero against an infinity would be NaN)
+      const bool in = k + e < K;
+      const int ke = in ? k + e : K - 1;
+      const T va = TA ? a[(int64_t)ke * lda] : a[ke];
+      ra[e] = in ? va : T(0);
+#pragma unroll
+      for (int f = 0; f < NF; f++) {
+        const T vb = TB ? b[f][ke] : b[f][(int64_t)ke * ldb];
+        rb[f][e] = in ? vb : T(0);
+      }
+    }
+#pragma unroll
+    for (int f = 0; f < NF; f++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[f] = mma(ra[e], rb[f][e], acc[f]);
+  }
+#pragma unroll
+  for (int f = 0; f < NF; f++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) part[wave][acc_row<T>(lane, e)][16 * f + c] = acc[f][e];
+  __syncthreads();
+  for (int i = t; i < 256 * NF; i += blockDim.x) {
+    const int r = i / (16 * NF), q = i % (16 * NF);
+    if (m0 + r >= M || n0 + q >= N) continue;
+    T v = 0;
+    for (int w = 0; w < nw; w++) v += part[w][r][q];
+    T* p = C + (int64_t)(m0 + r) * ldc + n0 + q;
+    v *= alpha;
+    if (beta != T(0)) v += beta * *p;
+    *p = v;
+  }
 }
 
 template <typename T>
@@ -256,9 +327,13 @@ __global__ void scale_kernel(int M, int N, T beta, T* C, int ldc) {
 
 }  // namespace
 
+// The tiled product: every element's K is summed in one order whatever the
+// shape.  The public gemm promises that; the mixed-precision factors keep it
+// too, because whether a BF16 or an unpivoted one refines at all can hang on
+// their rounding.  The drivers' large updates run here as well.
 template <typename T>
-int gemm_launch(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alpha, const T* A, int lda, const T* B,
-                int ldb, T beta, T* C, int ldc, int lower_only) {
+int gemm_tiles(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alpha, const T* A, int lda, const T* B,
+               int ldb, T beta, T* C, int ldc, int lower_only) {
   if (m <= 0 || n <= 0) return NMX_OK;
   if (k <= 0 || alpha == T(0)) {
     if (beta == T(1)) return NMX_OK;
@@ -268,6 +343,8 @@ int gemm_launch(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alp
     return NMX_OK;
   }
   if (lower_only && m != n) return NMX_ERR_UNSUPPORTED;
+  const double flops = 2.0 * m * (double)n * k * (lower_only ? 0.5 : 1.0);
+  ProfScope ps(ctx, K_GEMM, flops, (double)sizeof(T) * ((double)m * k + (double)k * n + 2.0 * m * n));
   // 128x128 tiles unless they would leave the device under-filled (fewer
   // than two per CU, the in-panel and late trailing updates): 64x64 tiles
   // then quadruple the workgroups and quarter each one's MFMA chain.  The
@@ -280,8 +357,6 @@ int gemm_launch(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alp
   const int tilesM = ceil_div(m, tile), tilesN = ceil_div(n, tile);
   const int grid = ceil_div(tiles(tile), kXcds) * kXcds;
   dim3 g(grid), blk(256);
-  const double flops = 2.0 * m * (double)n * k * (lower_only ? 0.5 : 1.0);
-  ProfScope ps(ctx, K_GEMM, flops, (double)sizeof(T) * ((double)m * k + (double)k * n + 2.0 * m * n));
   auto run = [&](auto tile_tag) {
     constexpr int TL = decltype(tile_tag)::value;
     if (!transa && !transb)
@@ -301,6 +376,39 @@ int gemm_launch(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alp
     run(std::integral_constant<int, 64>());
   else
     run(std::integral_constant<int, BM>());
+  NMX_HIP(ctx, hipGetLastError());
+  return NMX_OK;
+}
+
+// The drivers' product (alpha != 0).
+template <typename T>
+int gemm_launch(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alpha, const T* A, int lda, const T* B,
+                int ldb, T beta, T* C, int ldc, int lower_only) {
+  // Up to four workgroups per CU of 16-row tiles: there K's chain decides
+  // (FP64, us, 64 x 64 tiles / thin: 256 x 16 x 256 18 / 6.6, 4096 x 16 x 4096
+  // 244 / 32, 4096 x 64 x 4096 245 / 71, 1000 x 96 x 96 9.1 / 5.9, 1024 x 512
+  // x 512 35 / 20).  With more of them a tile's reuse of its operands does
+  // (1024 x 1024 x 192 17 / 20, 8192 x 96 x 96 10 / 12, 16384 x 64 x 64 8.3 / 10).
+  const int nf = n <= 16 ? 1 : 2;
+  const int64_t thin_tiles = (int64_t)ceil_div(m, 16) * ceil_div(n, 16 * nf) / (lower_only ? 2 : 1);
+  if (thin_tiles > 4 * ctx->num_cus || (transa && transb) || m <= 0 || n <= 0 || k <= 0 || (lower_only && m != n))
+    return gemm_tiles<T>(ctx, transa, transb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_only);
+  const double flops = 2.0 * m * (double)n * k * (lower_only ? 0.5 : 1.0);
+  ProfScope ps(ctx, K_GEMM, flops, (double)sizeof(T) * ((double)m * k + (double)k * n + 2.0 * m * n));
+  auto thin = [&](auto nf_tag) {
+    constexpr int NF = decltype(nf_tag)::value;
+    const dim3 tg(ceil_div(m, 16), ceil_div(n, 16 * NF)), tb(64 * std::min(8, ceil_div(k, 16)));
+    if (!transa && !transb)
+      gemm_thin<T, 0, 0, NF><<<tg, tb, 0, ctx->stream>>>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_only);
+    else if (!transa && transb)
+      gemm_thin<T, 0, 1, NF><<<tg, tb, 0, ctx->stream>>>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_only);
+    else
+      gemm_thin<T, 1, 0, NF><<<tg, tb, 0, ctx->stream>>>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_only);
+  };
+  if (nf == 1)
+    thin(std::integral_constant<int, 1>());
+  else
+    thin(std::integral_constant<int, 2>());
   NMX_HIP(ctx, hipGetLastError());
   return NMX_OK;
 }
@@ -328,6 +436,8 @@ int gemm_launch_splitk(nmx_ctx* ctx, int m, int n, int k, T alpha, const T* A, i
 template int gemm_launch_splitk<double>(nmx_ctx*, int, int, int, double, const double*, int, const double*, int,
                                         double*, int, int, int64_t);
 
+template int gemm_tiles<float>(nmx_ctx*, int, int, int, int, int, float, const float*, int, const float*, int, float,
+                               float*, int, int);
 template int gemm_launch<double>(nmx_ctx*, int, int, int, int, int, double, const double*, int, const double*, int,
                                  double, double*, int, int);
 template int gemm_launch<float>(nmx_ctx*, int, int, int, int, int, float, const float*, int, const float*, int, float,
@@ -343,7 +453,7 @@ static int gemm_api(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T
   if (lda < (transa ? m : k) || lda < 1) return -9;
   if (ldb < (transb ? k : n) || ldb < 1) return -11;
   if (ldc < n || ldc < 1) return -14;
-  return gemm_launch<T>(ctx, transa, transb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, 0);
+  return gemm_tiles<T>(ctx, transa, transb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, 0);
 }
 
 NMX_API int nmx_gemm_f64(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, double alpha, const double* A,

@@ -24,9 +24,9 @@
 // step reduced 33 values over 256 threads and read them back: 165 LDS reads
 // and 126 shuffles a step, and 4096 problems of 1024 x 32 took 6.55 ms.
 // In this layout they take 0.62 ms (10.8x; 885 GB/s of the 4.8 TB/s a copy
-// reaches): the broadcasts are the DPP operand of the multiply-adds (0.64 ms as
-// separate moves), 60 % of the time is
-// issue, the rest the step's barrier and LDS round.
+// reaches): the broadcasts are the DPP operand of the multiply-adds (0.64 ms
+// as separate moves), 60 % of the time is issue, the rest the step's barrier
+// and LDS round.
 #include <math.h>
 
 #include "tile16.h"

@@ -320,6 +320,32 @@ def test_triangular_strip_edges(n, dtype):
         assert torch.equal(B[:, nrhs:], B0[:, nrhs:])
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n,nrhs", [(1100, 1), (1100, 17), (793, 16), (2050, 33)])
+def test_triangular_thin_updates(n, nrhs, dtype):
+    """Updates of a few vectors with long, ragged contractions: several slabs a
+    wavefront, a remainder of 1 to 15, a partial last row and column tile.
+    Residual bound of substitution as at the strip edges."""
+    eps = torch.finfo(dtype).eps
+    rng = np.random.default_rng(n + nrhs)
+    from numax_amd import _lib
+    for upper, trans in ((0, 0), (1, 0), (0, 1), (1, 1)):
+        t = rng.standard_normal((n, n + 1)) / np.sqrt(n)
+        t[:, :n] += 2.0 * np.eye(n)
+        T = torch.as_tensor(t, device="cuda").to(dtype)
+        B0 = torch.as_tensor(rng.standard_normal((n, nrhs + 1)), device="cuda").to(dtype)
+        B = B0.clone()
+        stored = T[:, :n].double().cpu().numpy()
+        stored = np.triu(stored) if upper else np.tril(stored)
+        op = stored.T if trans else stored
+        _lib.check(nl._fn("trsm", dtype)(nl._ctx(T).handle, int(upper != trans), 0, trans, n, nrhs, nl._ptr(T), n + 1,
+                                         nl._ptr(B), nrhs + 1), "trsm")
+        x = B[:, :nrhs].double().cpu().numpy()
+        r = np.abs(op @ x - B0[:, :nrhs].double().cpu().numpy())
+        assert np.all(r <= 16 * (n + 16) * eps * (np.abs(op) @ np.abs(x) + 1)), (upper, trans)
+        assert torch.equal(B[:, nrhs:], B0[:, nrhs:])
+
+
 def test_triangular_strip_spreads_infinities_as_substitution_does():
     n = 70
     rng = np.random.default_rng(9)
