@@ -212,17 +212,21 @@ __global__ void __launch_bounds__(64 * NB16) chol_block_kernel(T* __restrict__ A
     }
     __syncthreads();
     if (w > s && w < steps) {
+      // products from zero, one addition each: summed onto the tile every term
+      // would round at the tile's size (256 columns FP32: 2.4x the error)
       const acc_t x = c[0];
+      acc_t d = {0, 0, 0, 0};
 #pragma unroll
-      for (int q = 0; q < 4; q++) dg = mma(L.x[w][q][lane], x[q], dg);
+      for (int q = 0; q < 4; q++) d = mma(L.x[w][q][lane], x[q], d);
+      dg += d;
       // tile j of the row moves to place j - 1 with the product
 #pragma unroll
       for (int j = 1; j < NB16 - 1; j++)
         if (j < w - s) {  // uniform
-          acc_t v = c[j];
+          acc_t v = {0, 0, 0, 0};
 #pragma unroll
           for (int q = 0; q < 4; q++) v = mma(L.x[s + j][q][lane], x[q], v);
-          c[j - 1] = v;
+          c[j - 1] = c[j] + v;
         }
     }
     // the next step's X is published after its first barrier, which every

@@ -229,7 +229,7 @@ gemm_kernel(int M, int N, int K, T alpha, const T* __restrict__ A, int lda, cons
 // 16 slabs in turn, three quarters of each for columns that are not there --
 // and here that chain is K / (16 NW) slabs, four of them in flight.  Cholesky
 // and solve of order 8192 with 16 vectors: 14.6 -> 11.5 ms, LU 45.5 -> 43.4,
-// FP32 Cholesky of order 1301 1.21 -> 0.94.
+// FP32 Cholesky of order 1301 1.21 -> 0.94 ms.
 template <typename T, int TA, int TB, int NF>
 __global__ void __launch_bounds__(512)
 gemm_thin(int M, int N, int K, T alpha, const T* __restrict__ A, int lda, const T* __restrict__ B, int ldb, T beta,
@@ -328,9 +328,9 @@ __global__ void scale_kernel(int M, int N, T beta, T* C, int ldc) {
 }  // namespace
 
 // The tiled product: every element's K is summed in one order whatever the
-// shape.  The public gemm promises that; the mixed-precision factors keep it
-// too, because whether a BF16 or an unpivoted one refines at all can hang on
-// their rounding.  The drivers' large updates run here as well.
+// shape.  The public gemm promises that; the unpivoted mixed-precision factor
+// keeps it too, because whether one refines at all can hang on its rounding.
+// The drivers' large updates run here as well.
 template <typename T>
 int gemm_tiles(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alpha, const T* A, int lda, const T* B,
                int ldb, T beta, T* C, int ldc, int lower_only) {

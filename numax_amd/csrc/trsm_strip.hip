@@ -112,8 +112,12 @@ __device__ __forceinline__ void strip_steps(int n, __amdgpu_buffer_rsrc_t rt, co
 #pragma unroll
           for (int v = u; v < NS; v++)
             if (v > u || w > owner) {  // uniform
+              // the product from zero, then one addition: summed onto r each
+              // of its terms would round at r's size (256 rows: 1.8x the error)
+              typename Acc<T>::type d = {0, 0, 0, 0};
 #pragma unroll
-              for (int q = 0; q < 4; q++) r[v][g] = mma(tl[buf][v][q], xb[q], r[v][g]);
+              for (int q = 0; q < 4; q++) d = mma(tl[buf][v][q], xb[q], d);
+              r[v][g] += d;
             }
         }
       }
