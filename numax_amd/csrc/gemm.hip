@@ -228,7 +228,7 @@ gemm_kernel(int M, int N, int K, T alpha, const T* __restrict__ A, int lda, cons
 // slabs one workgroup walks -- 64 x 64 tiles of a 256 x 16 x 256 update run
 // 16 slabs in turn, three quarters of each for columns that are not there --
 // and here that chain is K / (16 NW) slabs, four of them in flight.  Cholesky
-// and solve of order 8192 with 16 vectors: 14.6 -> 11.5 ms, LU 45.5 -> 43.4,
+// and solve of order 8192 with 16 vectors: 14.6 -> 11.5 ms, LU 45.5 -> 43.4 ms,
 // FP32 Cholesky of order 1301 1.21 -> 0.94 ms.
 template <typename T, int TA, int TB, int NF>
 __global__ void __launch_bounds__(512)

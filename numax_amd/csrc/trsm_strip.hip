@@ -9,8 +9,8 @@
 // s % 4, and a block's right-hand sides stay in the owner's registers in the
 // MFMA output layout.  Step s: the owner multiplies its block by the inverse
 // of the 16 x 16 diagonal block, corrects that by its residual, and passes
-// X_s on through LDS; one barrier;
-// every wavefront subtracts its blocks' products with X_s.  The products run
+// X_s on through LDS; one barrier; every wavefront subtracts its blocks'
+// products with X_s.  The products run
 // on 16x16x4 MFMA with the contraction index permuted to the output layout's
 // row order, so an output is the next product's operand as it is.  The tiles
 // of T do not depend on X and are read a step ahead.
@@ -19,8 +19,9 @@
 // round and a barrier each).  64 rows a launch by substitution, a column per
 // thread, took 15 us (FP64 or FP32, 64 rows) and a GEMM launch between every
 // two: 256 rows by 7936 columns FP64 were 4 such launches and 3 GEMMs.
-// Now 256 rows by 16 columns FP64 are one launch of 23 us, 64 rows 6 us, and
-// FP64 Cholesky + 16-column solve of order 8192 takes 21.2 ms (31.7 before).
+// Now 256 rows by 16 columns FP64 are one launch of 23 us, 64 rows 6 us: FP64
+// Cholesky + 16-column solve of order 8192 31.7 -> 21.2 ms (11.8 with the
+// Cholesky blocks and thin products since).
 //
 // The inverses are of 16 x 16 blocks only and made per workgroup (a column
 // per lane, the block's rows by DPP broadcast).  A workgroup that meets a

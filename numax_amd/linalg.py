@@ -156,9 +156,9 @@ def lu_factor(a, block: int = 16, base: int = 16) -> LU:
 
     ``block`` is the panel width and ``base`` the recursive panel's leaf width
     (the reference's parameters of the same names, with its device defaults
-    16 / 16, lu.mojo:454-459); the pivots do not depend on them, the speed
-    does: 256 / 32 is the fastest shape on MI355X at large n.  A singular
-    matrix is not reported as an error (see ``LU.singular``).
+    16 / 16, lu.mojo:454-459); the pivots do not depend on them, and panels
+    narrower than 192 / 32 run at that width, the fastest shape on MI355X.  A
+    singular matrix is not reported as an error (see ``LU.singular``).
     """
     work = _device_tensor(a).clone()
     n = _square(work, "lu_factor")
@@ -281,8 +281,8 @@ def cholesky(a, block: int = 32) -> torch.Tensor:
     """Lower ``L`` with ``L L^T = a`` (cholesky.mojo:233-396).  Reads only the
     lower triangle; raises naming the 0-based index of the first non-positive
     pivot, after the whole factorization has run.  ``block`` defaults to
-    numax's device default (32, cholesky.mojo:233-237); 256 is the fastest
-    panel width on MI355X at large n."""
+    numax's device default (32, cholesky.mojo:233-237); a panel is at least
+    what one workgroup factors whole (128 columns in FP64, 256 in FP32)."""
     work = _device_tensor(a).clone()
     n = _square(work, "cholesky")
     info = torch.zeros(1, dtype=torch.int32, device=work.device)
