@@ -74,8 +74,8 @@ const char* nmx_kernel_name(int kind);
  * in-place P A = L U, unit L below the diagonal, first-maximum pivots, full
  * row interchanges, an exact-zero pivot divided as 1e-30 and recorded in
  * `info` (not an error).  `block` is the panel width, `base` the recursive
- * panel's leaf width (0 picks the defaults 256 / 32; narrower ones run as
- * 192 / 32, the pivots depending on neither).  n is at most 32768
+ * panel's leaf width (0 picks the defaults 256 / 32; a leaf is at most 32).
+ * n is at most 32768
  * (the rows the cooperative pivoting leaf holds); a larger n returns
  * NMX_ERR_UNSUPPORTED before any work is queued. */
 int nmx_getrf_f64(nmx_ctx* ctx, int n, double* A, int lda, int32_t* ipiv, int32_t* info, int block, int base);

@@ -53,15 +53,6 @@ int getrf_impl_ex(nmx_ctx* ctx, int n, T* A, int lda, int32_t* ipiv, int32_t* in
                   TrailingUpdate update, void* user, PanelHook panel_hook) {
   if (block <= 0) block = 256;
   if (base <= 0 || base > kLeafW) base = kLeafW;
-  if (!panel_hook) {
-    // The pivots do not depend on either width.  A narrower leaf (numax's
-    // device default is 16 / 16) costs the same a column, and each leaf an
-    // interchange, a triangular solve and an update launch besides: order
-    // 1000 FP64 takes 3.1 ms with 16 / 16 and 2.7 to 2.9 ms with leaves of 32
-    // in panels of any width from 32 to 512.
-    block = std::max(block, 192);
-    base = kLeafW;
-  }
   NMX_TRY(zero_info(ctx, info));
   for (int k = 0; k < n; k += block) {
     const int nb = block < n - k ? block : n - k;

@@ -1385,6 +1385,7 @@ template <int BF, int SPLIT>
 static int mp_convert(nmx_ctx* ctx, MpFactor& f, int k, int nb, int m) {
   typedef typename Lo<BF>::t lt;
   const int n = f.n;
+  if (nb > f.block) return NMX_ERR_UNSUPPORTED;  // lo_buf holds panels of f.block columns
   const float* L21 = f.F + (int64_t)(k + nb) * n + k;  // m x nb, ld n
   const float* U12 = f.F + (int64_t)k * n + k + nb;    // nb x m, ld n
   lt* base = (lt*)f.lo_buf;

@@ -156,9 +156,9 @@ def lu_factor(a, block: int = 16, base: int = 16) -> LU:
 
     ``block`` is the panel width and ``base`` the recursive panel's leaf width
     (the reference's parameters of the same names, with its device defaults
-    16 / 16, lu.mojo:454-459); the pivots do not depend on them, and panels
-    narrower than 192 / 32 run at that width, the fastest shape on MI355X.  A
-    singular matrix is not reported as an error (see ``LU.singular``).
+    16 / 16, lu.mojo:454-459); the pivots do not depend on them, the speed
+    does: 256 / 32 is the fastest shape on MI355X at large n.  A singular
+    matrix is not reported as an error (see ``LU.singular``).
     """
     work = _device_tensor(a).clone()
     n = _square(work, "lu_factor")

@@ -163,6 +163,22 @@ def test_mpir_block_of_right_hand_sides(nrhs, kappa, pivot):
     assert max(r["backward_error"] for r in reps) <= 1e-15
 
 
+@pytest.mark.parametrize("precision", ["fp16", "bf16", "fp16s", "fp32"])
+@pytest.mark.parametrize("n,block", [(347, 64), (700, 64), (700, 128), (1801, 128), (1000, 192), (1000, 512)])
+def test_partial_pivoting_in_panels_of_every_width(n, block, precision, monkeypatch):
+    """The update's operand buffers hold panels of the caller's width: in a
+    context of their own, where no wider call has grown them, every panel is
+    that width (a wider one is refused on the host)."""
+    from numax_amd import _lib
+    monkeypatch.setattr(_lib, "_contexts", {})
+    a = svd_matrix(n, 1e2, seed=n + block)
+    b = R.normal(n, (n,))
+    x, rep = nl.solve_mpir(a, b, precision=precision, pivot="partial", block=block)
+    eta = oracle.backward_error(a, x.cpu().numpy(), b)
+    assert rep["converged"] and eta <= 1e-15, (rep, eta)
+    _lib._contexts[0].close()
+
+
 def test_autotuners_pick_from_their_candidates(tmp_path, monkeypatch):
     from numax_amd import autotune
     monkeypatch.setenv("NUMAX_AMD_TUNE_CACHE", str(tmp_path / "tune.json"))
