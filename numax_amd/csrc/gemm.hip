@@ -220,100 +220,93 @@ gemm_kernel(int M, int N, int K, T alpha, const T* __restrict__ A, int lda, cons
     }
 }
 
-// Products too small for a tile per CU: a workgroup owns 16 x (16 NF) of C
-// and its wavefronts take every NW-th 16-deep slab of K, operands straight
-// from memory into MFMA registers (a lane's four contraction indices are
-// neighbours, so A's rows are read 16 B at a time), the partial tiles added
-// in LDS.  What bounds these is not the matrix cores but the chain of K
-// slabs one workgroup walks -- 64 x 64 tiles of a 256 x 16 x 256 update run
-// 16 slabs in turn, three quarters of each for columns that are not there --
-// and here that chain is K / (16 NW) slabs, four of them in flight.  Cholesky
-// and solve of order 8192 with 16 vectors: 14.6 -> 11.5 ms, LU 45.5 -> 43.4 ms,
-// FP32 Cholesky of order 1301 1.21 -> 0.94 ms.
-template <typename T, int TA, int TB, int NF>
-__global__ void __launch_bounds__(512)
-gemm_thin(int M, int N, int K, T alpha, const T* __restrict__ A, int lda, const T* __restrict__ B, int ldb, T beta,
-          T* __restrict__ C, int ldc, int lower_only) {
-  typedef typename Acc<T>::type acc_t;
-  constexpr int SL = 4 / NF < 2 ? 2 : 4 / NF;  // slabs in flight
-  __shared__ T part[8][16][16 * NF + 1];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = blockDim.x >> 6;
-  const int m0 = blockIdx.x * 16, n0 = blockIdx.y * 16 * NF;
-  const int c = lane & 15, k4 = 4 * (lane >> 4);
-  if (lower_only && n0 > m0 + 15) return;
-  // rows and columns past the edge read the last one and are not stored
-  const int row = min(m0 + c, M - 1);
-  const T* a = TA ? A + row : A + (int64_t)row * lda;
-  const T* b[NF];
-#pragma unroll
-  for (int f = 0; f < NF; f++) {
-    const int col = min(n0 + 16 * f + c, N - 1);
-    b[f] = TB ? B + (int64_t)col * ldb : B + col;
-  }
-  acc_t acc[NF];
-#pragma unroll
-  for (int f = 0; f < NF; f++) acc[f] = acc_t{0, 0, 0, 0};
-  auto quad = [&](auto trans, const T* p, int ld, int k, T(&r)[4]) {
-#pragma unroll
-    for (int e = 0; e < 4; e++) r[e] = trans ? p[(int64_t)(k + e) * ld] : p[k + e];
-  };
-  const std::integral_constant<bool, TA != 0> ta{};
-  const std::integral_constant<bool, TB == 0> tb{};
-  const int full = K / 16;
-  int s = wave;
-  for (; s + (SL - 1) * nw < full; s += SL * nw) {
-    T ra[SL][4], rb[SL][NF][4];
-#pragma unroll
-    for (int u = 0; u < SL; u++) {
-      const int k = 16 * (s + u * nw) + k4;
-      quad(ta, a, lda, k, ra[u]);
-#pragma unroll
-      for (int f = 0; f < NF; f++) quad(tb, b[f], ldb, k, rb[u][f]);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // all slabs' loads go out before the first is waited for
+// Products too small for a tile per CU: a wavefront owns 16 x (16 NF) of C and
+// walks K from its start, the order of the tiles above, operands straight from
+// memory into MFMA registers with SL 16-deep slabs of them in flight while the
+// SL before are multiplied.  What bounds these is not the matrix cores but the
+// chain of K slabs -- 64 x 64 tiles of a 256 x 16 x 256 update run
+// 16 slabs in turn, each with a round trip to memory and three quarters of it
+// for columns that are not there.
+template <typename T, int TA, int TB, int NF, int SL>
+struct ThinSlabs {
+  T a[SL][4], b[SL][NF][4];
+  // Slabs SL g .. of operands whose lane offsets at k = 0 are oa and ob.  Past
+  // K both factors are zero, by offsets out of the descriptor's range: no
+  // branches, which would wait for the loads where they meet.
+  __device__ __forceinline__ void load(const T* A, int lda, uint32_t oa, const T* B, int ldb, const uint32_t (&ob)[NF], int g,
+                                       int lk, int K) {
+    constexpr uint32_t E = sizeof(T);
+    const int k0 = 16 * SL * g;
+    const __amdgpu_buffer_rsrc_t ra = buf_rsrc(A + (TA ? (int64_t)k0 * lda : k0));
+    const __amdgpu_buffer_rsrc_t rb = buf_rsrc(B + (TB ? k0 : (int64_t)k0 * ldb));
 #pragma unroll
     for (int u = 0; u < SL; u++)
 #pragma unroll
-      for (int f = 0; f < NF; f++)
+      for (int e = 0; e < 4; e++) {
+        const uint32_t kk = 16 * u + 4 * e;
+        const bool in = k0 + (int)kk + lk < K;
+        a[u][e] = buf_load<T>(ra, in ? oa + kk * (TA ? (uint32_t)lda : 1u) * E : kBufOob);
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[f] = mma(ra[u][e], rb[u][f][e], acc[f]);
-  }
-  for (; 16 * s < K; s += nw) {
-    const int k = 16 * s + k4;
-    T ra[4], rb[NF][4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      // past K both factors are zero (a zero against an infinity would be NaN)
-      const bool in = k + e < K;
-      const int ke = in ? k + e : K - 1;
-      const T va = TA ? a[(int64_t)ke * lda] : a[ke];
-      ra[e] = in ? va : T(0);
-#pragma unroll
-      for (int f = 0; f < NF; f++) {
-        const T vb = TB ? b[f][ke] : b[f][(int64_t)ke * ldb];
-        rb[f][e] = in ? vb : T(0);
+        for (int f = 0; f < NF; f++) b[u][f][e] = buf_load<T>(rb, in ? ob[f] + kk * (TB ? 1u : (uint32_t)ldb) * E : kBufOob);
       }
+  }
+  __device__ __forceinline__ void multiply(typename Acc<T>::type (&acc)[NF], int g, int K) const {
+#pragma unroll
+    for (int u = 0; u < SL; u++) {
+      if (16 * (SL * g + u) >= K) break;  // uniform
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int f = 0; f < NF; f++) acc[f] = mma(a[u][e], b[u][f][e], acc[f]);
     }
+  }
+};
+
+template <typename T, int TA, int TB, int NF>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1)))
+gemm_thin(int M, int N, int K, T alpha, const T* __restrict__ A, int lda, const T* __restrict__ B, int ldb, T beta,
+          T* __restrict__ C, int ldc, int lower_only) {
+  typedef typename Acc<T>::type acc_t;
+  constexpr uint32_t E = sizeof(T);
+  constexpr int SL = NF == 1 ? 4 : 3;  // slabs a buffer: a wavefront has at most 63 loads in flight
+  const int lane = threadIdx.x, lc = lane & 15, lk = lane >> 4;
+  const int m0 = blockIdx.x * 16, n0 = blockIdx.y * 16 * NF;
+  if (lower_only && n0 > m0 + 15) return;
+  A += TA ? m0 : (int64_t)m0 * lda;
+  B += TB ? (int64_t)n0 * ldb : n0;
+  // rows and columns past the edge read the last one and are not stored
+  const uint32_t r = min(lc, M - 1 - m0);
+  const uint32_t oa = (TA ? (uint32_t)lk * (uint32_t)lda + r : r * (uint32_t)lda + (uint32_t)lk) * E;
+  uint32_t ob[NF];
+  acc_t acc[NF];
 #pragma unroll
-    for (int f = 0; f < NF; f++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) acc[f] = mma(ra[e], rb[f][e], acc[f]);
+  for (int f = 0; f < NF; f++) {
+    const uint32_t q = min(16 * f + lc, N - 1 - n0);
+    ob[f] = (TB ? q * (uint32_t)ldb + (uint32_t)lk : (uint32_t)lk * (uint32_t)ldb + q) * E;
+    acc[f] = acc_t{0, 0, 0, 0};
+  }
+  const int groups = (K + 16 * SL - 1) / (16 * SL);
+  ThinSlabs<T, TA, TB, NF, SL> one, two;
+  one.load(A, lda, oa, B, ldb, ob, 0, lk, K);
+  for (int g = 0; g < groups; g += 2) {
+    two.load(A, lda, oa, B, ldb, ob, g + 1, lk, K);
+    __builtin_amdgcn_sched_barrier(0);
+    one.multiply(acc, g, K);
+    one.load(A, lda, oa, B, ldb, ob, g + 2, lk, K);
+    __builtin_amdgcn_sched_barrier(0);
+    two.multiply(acc, g + 1, K);
   }
 #pragma unroll
   for (int f = 0; f < NF; f++)
 #pragma unroll
-    for (int e = 0; e < 4; e++) part[wave][acc_row<T>(lane, e)][16 * f + c] = acc[f][e];
-  __syncthreads();
-  for (int i = t; i < 256 * NF; i += blockDim.x) {
-    const int r = i / (16 * NF), q = i % (16 * NF);
-    if (m0 + r >= M || n0 + q >= N) continue;
-    T v = 0;
-    for (int w = 0; w < nw; w++) v += part[w][r][q];
-    T* p = C + (int64_t)(m0 + r) * ldc + n0 + q;
-    v *= alpha;
-    if (beta != T(0)) v += beta * *p;
-    *p = v;
-  }
+    for (int e = 0; e < 4; e++) {
+      const int r = m0 + acc_row<T>(lane, e), q = n0 + 16 * f + lc;
+      if (r >= M || q >= N) continue;
+      T* p = C + (int64_t)r * ldc + q;
+      T v = alpha * acc[f][e];
+      if (beta != T(0)) v += beta * *p;
+      *p = v;
+    }
 }
 
 template <typename T>
@@ -327,13 +320,10 @@ __global__ void scale_kernel(int M, int N, T beta, T* C, int ldc) {
 
 }  // namespace
 
-// The tiled product: every element's K is summed in one order whatever the
-// shape.  The public gemm promises that; the unpivoted mixed-precision factor
-// keeps it too, because whether one refines at all can hang on its rounding.
-// The drivers' large updates run here as well.
+// Every element's K is summed in one ascending order whatever the shape.
 template <typename T>
-int gemm_tiles(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alpha, const T* A, int lda, const T* B,
-               int ldb, T beta, T* C, int ldc, int lower_only) {
+int gemm_launch(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alpha, const T* A, int lda, const T* B,
+                int ldb, T beta, T* C, int ldc, int lower_only) {
   if (m <= 0 || n <= 0) return NMX_OK;
   if (k <= 0 || alpha == T(0)) {
     if (beta == T(1)) return NMX_OK;
@@ -345,6 +335,31 @@ int gemm_tiles(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alph
   if (lower_only && m != n) return NMX_ERR_UNSUPPORTED;
   const double flops = 2.0 * m * (double)n * k * (lower_only ? 0.5 : 1.0);
   ProfScope ps(ctx, K_GEMM, flops, (double)sizeof(T) * ((double)m * k + (double)k * n + 2.0 * m * n));
+  // A wavefront a 16-row tile while the device has a few CUs' worth of them:
+  // there K's chain decides (FP64, us, 64 x 64 tiles / thin: 256 x 16 x 256
+  // 18.8 / 6.0, 4096 x 16 x 4096 239 / 51, 4096 x 64 x 4096 240 / 95, 1000 x
+  // 96 x 96 10.1 / 5.8, 512 x 512 x 16 6.2 / 5.9).  Of up to four a CU a short
+  // chain loses to the reuse of operands (1024 x 512 x 32 7.3 / 8.7, x 192 17.1
+  // / 15.0, 4096 x 128 x 128 12.6 / 12.6), of more any (1024 x 1024 x 192 17 /
+  // 24).  The order of every sum is the same.
+  const int nf = n <= 16 ? 1 : 2;
+  const int64_t thin_tiles = (int64_t)ceil_div(m, 16) * ceil_div(n, 16 * nf) / (lower_only ? 2 : 1);
+  if (thin_tiles <= (k < 128 ? 2 : 4) * ctx->num_cus && !(transa && transb)) {
+    auto thin = [&](auto nf_tag) {
+      constexpr int NF = decltype(nf_tag)::value;
+      const dim3 tg(ceil_div(m, 16), ceil_div(n, 16 * NF));
+      if (!transa && !transb)
+        gemm_thin<T, 0, 0, NF><<<tg, 64, 0, ctx->stream>>>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_only);
+      else if (!transa && transb)
+        gemm_thin<T, 0, 1, NF><<<tg, 64, 0, ctx->stream>>>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_only);
+      else
+        gemm_thin<T, 1, 0, NF><<<tg, 64, 0, ctx->stream>>>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_only);
+    };
+    if (nf == 1) thin(std::integral_constant<int, 1>());
+    else thin(std::integral_constant<int, 2>());
+    NMX_HIP(ctx, hipGetLastError());
+    return NMX_OK;
+  }
   // 128x128 tiles unless they would leave the device under-filled (fewer
   // than two per CU, the in-panel and late trailing updates): 64x64 tiles
   // then quadruple the workgroups and quarter each one's MFMA chain.  The
@@ -380,39 +395,6 @@ int gemm_tiles(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alph
   return NMX_OK;
 }
 
-// The drivers' product (alpha != 0).
-template <typename T>
-int gemm_launch(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alpha, const T* A, int lda, const T* B,
-                int ldb, T beta, T* C, int ldc, int lower_only) {
-  // Up to four workgroups per CU of 16-row tiles: there K's chain decides
-  // (FP64, us, 64 x 64 tiles / thin: 256 x 16 x 256 18 / 6.6, 4096 x 16 x 4096
-  // 244 / 32, 4096 x 64 x 4096 245 / 71, 1000 x 96 x 96 9.1 / 5.9, 1024 x 512
-  // x 512 35 / 20).  With more of them a tile's reuse of its operands does
-  // (1024 x 1024 x 192 17 / 20, 8192 x 96 x 96 10 / 12, 16384 x 64 x 64 8.3 / 10).
-  const int nf = n <= 16 ? 1 : 2;
-  const int64_t thin_tiles = (int64_t)ceil_div(m, 16) * ceil_div(n, 16 * nf) / (lower_only ? 2 : 1);
-  if (thin_tiles > 4 * ctx->num_cus || (transa && transb) || m <= 0 || n <= 0 || k <= 0 || (lower_only && m != n))
-    return gemm_tiles<T>(ctx, transa, transb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_only);
-  const double flops = 2.0 * m * (double)n * k * (lower_only ? 0.5 : 1.0);
-  ProfScope ps(ctx, K_GEMM, flops, (double)sizeof(T) * ((double)m * k + (double)k * n + 2.0 * m * n));
-  auto thin = [&](auto nf_tag) {
-    constexpr int NF = decltype(nf_tag)::value;
-    const dim3 tg(ceil_div(m, 16), ceil_div(n, 16 * NF)), tb(64 * std::min(8, ceil_div(k, 16)));
-    if (!transa && !transb)
-      gemm_thin<T, 0, 0, NF><<<tg, tb, 0, ctx->stream>>>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_only);
-    else if (!transa && transb)
-      gemm_thin<T, 0, 1, NF><<<tg, tb, 0, ctx->stream>>>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_only);
-    else
-      gemm_thin<T, 1, 0, NF><<<tg, tb, 0, ctx->stream>>>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_only);
-  };
-  if (nf == 1)
-    thin(std::integral_constant<int, 1>());
-  else
-    thin(std::integral_constant<int, 2>());
-  NMX_HIP(ctx, hipGetLastError());
-  return NMX_OK;
-}
-
 // C_q = alpha A[:, K_q] B[K_q, :] for the ksplit K slices K_q of length
 // kchunk = round_up(ceil(k / ksplit), 16) (C_q at C + q csplit, no beta):
 // one launch with ksplit times the workgroups, for products whose output
@@ -436,8 +418,6 @@ int gemm_launch_splitk(nmx_ctx* ctx, int m, int n, int k, T alpha, const T* A, i
 template int gemm_launch_splitk<double>(nmx_ctx*, int, int, int, double, const double*, int, const double*, int,
                                         double*, int, int, int64_t);
 
-template int gemm_tiles<float>(nmx_ctx*, int, int, int, int, int, float, const float*, int, const float*, int, float,
-                               float*, int, int);
 template int gemm_launch<double>(nmx_ctx*, int, int, int, int, int, double, const double*, int, const double*, int,
                                  double, double*, int, int);
 template int gemm_launch<float>(nmx_ctx*, int, int, int, int, int, float, const float*, int, const float*, int, float,
@@ -453,7 +433,7 @@ static int gemm_api(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T
   if (lda < (transa ? m : k) || lda < 1) return -9;
   if (ldb < (transb ? k : n) || ldb < 1) return -11;
   if (ldc < n || ldc < 1) return -14;
-  return gemm_tiles<T>(ctx, transa, transb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, 0);
+  return gemm_launch<T>(ctx, transa, transb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, 0);
 }
 
 NMX_API int nmx_gemm_f64(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, double alpha, const double* A,

@@ -1497,8 +1497,8 @@ static int nopiv_diag(nmx_ctx* ctx, MpFactor& f, int k, int nb) {
   NMX_TRY(trsm_left<float>(ctx, 0, 1, 0, half, rest, A11, n, F + (int64_t)k * n + k + half, n));
   // L21 := A21 U11^-1 (rows solve U11^T x^T = a^T)
   NMX_TRY(trsm_rec_rows_upper(ctx, rest, half, A11, n, F + (int64_t)(k + half) * n + k, n));
-  NMX_TRY(gemm_tiles<float>(ctx, 0, 0, rest, rest, half, -1.0f, F + (int64_t)(k + half) * n + k, n,
-                            F + (int64_t)k * n + k + half, n, 1.0f, F + (int64_t)(k + half) * n + k + half, n, 0));
+  NMX_TRY(gemm_launch<float>(ctx, 0, 0, rest, rest, half, -1.0f, F + (int64_t)(k + half) * n + k, n,
+                             F + (int64_t)k * n + k + half, n, 1.0f, F + (int64_t)(k + half) * n + k + half, n, 0));
   return nopiv_diag(ctx, f, k + half, rest);
 }
 
@@ -1574,8 +1574,8 @@ static int mp_factor(nmx_ctx* ctx, MpFactor& f, const double* A, int lda, uint64
       case 1: NMX_TRY((mp_update<1, 0>(ctx, f, k, nb, m))); break;
       case 2: NMX_TRY((mp_update<0, 1>(ctx, f, k, nb, m))); break;
       default:
-        NMX_TRY(gemm_tiles<float>(ctx, 0, 0, m, m, nb, -1.0f, f.F + (int64_t)(k + nb) * n + k, n,
-                                  f.F + (int64_t)k * n + k + nb, n, 1.0f, f.F + (int64_t)(k + nb) * n + k + nb, n, 0));
+        NMX_TRY(gemm_launch<float>(ctx, 0, 0, m, m, nb, -1.0f, f.F + (int64_t)(k + nb) * n + k, n,
+                                   f.F + (int64_t)k * n + k + nb, n, 1.0f, f.F + (int64_t)(k + nb) * n + k + nb, n, 0));
     }
   }
   const int nblk = ceil_div(n, TB);

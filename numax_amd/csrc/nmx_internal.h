@@ -146,10 +146,6 @@ int nmx_epoch_reserve(nmx_ctx* ctx, uint32_t columns, uint32_t* base);
 template <typename T>
 int gemm_launch(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alpha, const T* A, int lda, const T* B,
                 int ldb, T beta, T* C, int ldc, int lower_only = 0);
-// the same, every element's K summed in one order whatever the shape
-template <typename T>
-int gemm_tiles(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alpha, const T* A, int lda, const T* B,
-               int ldb, T beta, T* C, int ldc, int lower_only = 0);
 // ksplit K slices of A B (no transposes) into ksplit outputs C + q csplit
 template <typename T>
 int gemm_launch_splitk(nmx_ctx* ctx, int m, int n, int k, T alpha, const T* A, int lda, const T* B, int ldb, T* C,
@@ -162,6 +158,8 @@ int trsm_left(nmx_ctx* ctx, int upper, int unit, int trans, int n, int nrhs, con
 // op(T) X = B in place for a triangle of at most kStripMax rows (one launch);
 // vec_rows: the vectors are B's rows (B is nvec x n), else its columns.
 constexpr int kStripMax = 256;
+// Where a triangle of n > 64 rows splits in two.
+inline int trsm_split(int n) { return ((n / 2 + 63) / 64) * 64; }
 template <typename T>
 int trsm_strip(nmx_ctx* ctx, int upper, int unit, int trans, int vec_rows, int n, int nvec, const T* Tm, int ldt, T* B,
                int ldb);

@@ -718,9 +718,7 @@ int trsm_rec(nmx_ctx* ctx, int upper, int unit, int trans, int n, int nvec, cons
   const bool fits = std::max(span, tspan) * (int64_t)sizeof(T) < 0x7FFFFFFF;
   if (n <= kStripMax && (fits || n <= 16))
     return trsm_strip<T>(ctx, upper, unit, trans, VEC_ROWS, n, nvec, Tm, ldt, B, ldb);
-  // whole strips but for the last block
-  const int unit_rows = n > kStripMax ? kStripMax : 16;
-  const int n1 = ((n / 2 + unit_rows - 1) / unit_rows) * unit_rows;
+  const int n1 = n > 64 ? trsm_split(n) : ((n / 2 + 15) / 16) * 16;
   const int n2 = n - n1;
   const T* T11 = Tm;
   const T* T22 = Tm + (int64_t)n1 * ldt + n1;

@@ -53,6 +53,49 @@ __device__ __forceinline__ void fmac_bcast(double& s, double x, double y) {
   asm volatile("s_nop 1\nv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(s) : "v"(x), "v"(y), "n"(I));
 }
 
+// d0 .. d3 += x(lanes I .. I + 3 of the 16-lane row) * y, as above
+#define NMX_FMAC_LANES4(TYPE, D0, D1, D2, D3, X, Y, I)                                     \
+  asm volatile("s_nop 1\n"                                                                 \
+               "v_fmac_" TYPE "_dpp %0, %4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n" \
+               "v_fmac_" TYPE "_dpp %1, %4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n" \
+               "v_fmac_" TYPE "_dpp %2, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n" \
+               "v_fmac_" TYPE "_dpp %3, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n" \
+               : "+v"(D0), "+v"(D1), "+v"(D2), "+v"(D3)                                    \
+               : "v"(X), "v"(Y), "n"(I), "n"((I) + 1), "n"((I) + 2), "n"((I) + 3))
+template <int I>
+__device__ __forceinline__ void fmac_lanes4(float& d0, float& d1, float& d2, float& d3, float x, float y) {
+  NMX_FMAC_LANES4("f32", d0, d1, d2, d3, x, y, I);
+}
+template <int I>
+__device__ __forceinline__ void fmac_lanes4(double& d0, double& d1, double& d2, double& d3, double x, double y) {
+  NMX_FMAC_LANES4("f64", d0, d1, d2, d3, x, y, I);
+}
+
+// x / d, correctly rounded, from r = 1 / d correctly rounded: two corrections
+// of the product by its residual (Markstein; the first leaves it within an ulp,
+// the second rounds).  For operands whose quotient and residuals stay normal:
+// d and x in the ranges below.  A quarter of a division's instructions.
+template <typename T>
+__device__ __forceinline__ T plain_quotient(T x, T d, T r) {
+  T q = x * r;
+  q = __builtin_elementwise_fma(__builtin_elementwise_fma(-q, d, x), r, q);
+  return __builtin_elementwise_fma(__builtin_elementwise_fma(-q, d, x), r, q);
+}
+// and zeros (with their sign), infinities and NaNs
+__device__ __forceinline__ double quotient(double x, double d, double r) {
+  return __builtin_amdgcn_div_fixup(plain_quotient(x, d, r), d, x);
+}
+__device__ __forceinline__ float quotient(float x, float d, float r) {
+  return __builtin_amdgcn_div_fixupf(plain_quotient(x, d, r), d, x);
+}
+__device__ __forceinline__ bool plain_divisor(double d) { return fabs(d) >= 1e-90 && fabs(d) <= 1e90; }
+__device__ __forceinline__ bool plain_divisor(float d) { return fabsf(d) >= 1e-9f && fabsf(d) <= 1e9f; }
+// a dividend's magnitude as an exponent; 0 for zeros, infinities and NaNs
+__device__ __forceinline__ int magnitude(double x) { return __builtin_amdgcn_frexp_exp(x); }
+__device__ __forceinline__ int magnitude(float x) { return __builtin_amdgcn_frexp_expf(x); }
+template <typename T>
+constexpr int plain_magnitude() { return sizeof(T) == 8 ? 600 : 90; }  // dividends of 2^-this .. 2^this
+
 // Row I of column c of the inverse of the lower triangular block whose rows
 // the 16 lanes hold (m: row `lane % 16`, rinv: the reciprocal of its diagonal);
 // ny is the inverse's column negated.

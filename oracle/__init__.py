@@ -67,6 +67,10 @@ def _load() -> ctypes.CDLL:
         "orc_array_slogdet_cholesky": (ctypes.c_double, [_i, _dp]),
         "orc_array_eigh": (None, [_i, _dp, _dp, _dp, _i]),
         "orc_array_lstsq": (None, [_i, _i, _dp, _dp, _dp]),
+        "orc_dev_trsm_f64": (None, [_i, _i, _i, _i, _i, _vp, _i, _vp, _i]),
+        "orc_dev_trsm_f32": (None, [_i, _i, _i, _i, _i, _vp, _i, _vp, _i]),
+        "orc_dev_getrf_f64": (_i, [_i, _vp, _i, _vp, _i, _i]),
+        "orc_dev_getrf_f32": (_i, [_i, _vp, _i, _vp, _i, _i]),
         "orc_backward_error": (ctypes.c_double, [_i, _i, _dp, _i, _dp, _i, _dp, _i]),
     }
     for name, (res, args) in sig.items():
@@ -352,6 +356,25 @@ def array_lstsq_batch(a, b):
     x = np.zeros((count, n), dtype=np.float64)
     _lib.orc_array_lstsq_batch(count, m, n, _a(aa), _a(bb), _a(x))
     return x
+
+
+def device_order_trsm(a, b, upper: bool, unit: bool = False, trans: bool = False):
+    """``op(a) x = b`` for a lower (or upper) ``op(a)`` in the device's order of
+    operations, in the arrays' own type (float64 or float32)."""
+    aa = np.array(a, order="C", copy=True)
+    x = np.array(b, dtype=aa.dtype, order="C", copy=True)
+    fn = _lib.orc_dev_trsm_f64 if aa.dtype == np.float64 else _lib.orc_dev_trsm_f32
+    fn(int(upper), int(unit), int(trans), aa.shape[0], x.shape[1], _a(aa), aa.shape[1], _a(x), x.shape[1])
+    return x
+
+
+def device_order_getrf(a, block: int, base: int):
+    """``(lu, ipiv, info)`` of the blocked LU in the device's order of operations."""
+    lu = np.array(a, order="C", copy=True)
+    ipiv = np.zeros(lu.shape[0], dtype=np.int32)
+    fn = _lib.orc_dev_getrf_f64 if lu.dtype == np.float64 else _lib.orc_dev_getrf_f32
+    info = fn(lu.shape[0], _a(lu), lu.shape[0], _a(ipiv), block, base)
+    return lu, ipiv, int(info)
 
 
 def backward_error(a, x, b) -> float:

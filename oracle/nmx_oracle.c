@@ -1040,6 +1040,114 @@ void orc_array_lstsq_batch(int count, int m, int n, const double* a, const doubl
 }
 
 /* ------------------------------------------------------------------------ */
+/* The device's order of operations                                         */
+/* ------------------------------------------------------------------------ */
+
+/* The order that the device's triangular solves and LU promise, so that their
+ * results can be compared bit for bit.  Every multiply-add is fused.  A triangle
+ * of more than 64 rows splits in two at a multiple of 64; the solved half's
+ * product is summed from zero in ascending stored order and subtracted once; up
+ * to 64 rows are substituted column by column.  LU is the recursive panel of
+ * getrf2 below with its leaves of `base` columns and, for the blocks right of a
+ * panel, these solves and products. */
+#define DEVICE_ORDER(T, FMA, SUF)                                                                                    \
+  static void dev_product_##SUF(int m, int n, int k, const T* a, int64_t ars, int64_t acs, const T* b, int ldb,     \
+                                T* c, int ldc) {                                                                     \
+    T* acc = (T*)malloc(sizeof(T) * (size_t)(n > 0 ? n : 1));                                                        \
+    for (int i = 0; i < m; i++) {                                                                                    \
+      for (int j = 0; j < n; j++) acc[j] = 0;                                                                        \
+      for (int q = 0; q < k; q++) {                                                                                  \
+        const T l = a[i * ars + q * acs];                                                                            \
+        for (int j = 0; j < n; j++) acc[j] = FMA(l, AT(b, ldb, q, j), acc[j]);                                       \
+      }                                                                                                              \
+      for (int j = 0; j < n; j++) AT(c, ldc, i, j) -= acc[j];                                                        \
+    }                                                                                                                \
+    free(acc);                                                                                                       \
+  }                                                                                                                  \
+  static void dev_trsm_##SUF(int upper, int unit, int n, int nrhs, const T* a, int64_t rs, int64_t cs, T* b,         \
+                             int ldb) {                                                                              \
+    if (n <= 64) {                                                                                                   \
+      for (int s = 0; s < n; s++) {                                                                                  \
+        const int j = upper ? n - 1 - s : s;                                                                         \
+        for (int r = 0; r < nrhs && !unit; r++) AT(b, ldb, j, r) /= a[j * rs + j * cs];                              \
+        for (int i = upper ? 0 : j + 1; i < (upper ? j : n); i++) {                                                  \
+          const T l = -a[i * rs + j * cs];                                                                           \
+          for (int r = 0; r < nrhs; r++) AT(b, ldb, i, r) = FMA(l, AT(b, ldb, j, r), AT(b, ldb, i, r));              \
+        }                                                                                                            \
+      }                                                                                                              \
+      return;                                                                                                        \
+    }                                                                                                                \
+    const int n1 = (n / 2 + 63) / 64 * 64, n2 = n - n1;                                                              \
+    T* const b2 = b + (int64_t)n1 * ldb;                                                                             \
+    if (!upper) {                                                                                                    \
+      dev_trsm_##SUF(upper, unit, n1, nrhs, a, rs, cs, b, ldb);                                                      \
+      dev_product_##SUF(n2, nrhs, n1, a + n1 * rs, rs, cs, b, ldb, b2, ldb);                                         \
+      dev_trsm_##SUF(upper, unit, n2, nrhs, a + n1 * (rs + cs), rs, cs, b2, ldb);                                    \
+    } else {                                                                                                         \
+      dev_trsm_##SUF(upper, unit, n2, nrhs, a + n1 * (rs + cs), rs, cs, b2, ldb);                                    \
+      dev_product_##SUF(n1, nrhs, n2, a + n1 * cs, rs, cs, b2, ldb, b, ldb);                                         \
+      dev_trsm_##SUF(upper, unit, n1, nrhs, a, rs, cs, b, ldb);                                                      \
+    }                                                                                                                \
+  }                                                                                                                  \
+  static void dev_leaf_##SUF(int n, T* a, int lda, int32_t* ipiv, int32_t* info, int k, int w) {                     \
+    for (int j = k; j < k + w; j++) {                                                                                \
+      int best = j;                                                                                                  \
+      T mag = AT(a, lda, j, j) < 0 ? -AT(a, lda, j, j) : AT(a, lda, j, j);                                           \
+      if (!(mag == mag)) mag = 0;                                                                                    \
+      for (int i = j + 1; i < n; i++) {                                                                              \
+        const T v = AT(a, lda, i, j) < 0 ? -AT(a, lda, i, j) : AT(a, lda, i, j);                                     \
+        if (v > mag) mag = v, best = i;                                                                              \
+      }                                                                                                              \
+      ipiv[j] = best;                                                                                                \
+      for (int c = 0; best != j && c < n; c++) {                                                                     \
+        const T v = AT(a, lda, j, c);                                                                                \
+        AT(a, lda, j, c) = AT(a, lda, best, c);                                                                      \
+        AT(a, lda, best, c) = v;                                                                                     \
+      }                                                                                                              \
+      T p = AT(a, lda, j, j);                                                                                        \
+      if (p == 0) {                                                                                                  \
+        if (!*info) *info = j + 1;                                                                                   \
+        p = (T)PIVOT_FLOOR;                                                                                          \
+      }                                                                                                              \
+      for (int i = j + 1; i < n; i++) {                                                                              \
+        const T l = AT(a, lda, i, j) / p;                                                                            \
+        AT(a, lda, i, j) = l;                                                                                        \
+        for (int c = j + 1; c < k + w; c++) AT(a, lda, i, c) = FMA(-l, AT(a, lda, j, c), AT(a, lda, i, c));          \
+      }                                                                                                              \
+    }                                                                                                                \
+  }                                                                                                                  \
+  static void dev_panel_##SUF(int n, T* a, int lda, int32_t* ipiv, int32_t* info, int k, int nb, int base) {         \
+    if (nb <= base) {                                                                                                \
+      dev_leaf_##SUF(n, a, lda, ipiv, info, k, nb);                                                                  \
+      return;                                                                                                        \
+    }                                                                                                                \
+    int half = nb / 2;                                                                                               \
+    if (half > base) half = half / base * base;                                                                      \
+    const int m = k + half;                                                                                          \
+    dev_panel_##SUF(n, a, lda, ipiv, info, k, half, base);                                                           \
+    dev_trsm_##SUF(0, 1, half, nb - half, &AT(a, lda, k, k), lda, 1, &AT(a, lda, k, m), lda);                        \
+    dev_product_##SUF(n - m, nb - half, half, &AT(a, lda, m, k), lda, 1, &AT(a, lda, k, m), lda, &AT(a, lda, m, m),  \
+                      lda);                                                                                          \
+    dev_panel_##SUF(n, a, lda, ipiv, info, m, nb - half, base);                                                      \
+  }                                                                                                                  \
+  void orc_dev_trsm_##SUF(int upper, int unit, int trans, int n, int nrhs, const T* a, int lda, T* b, int ldb) {     \
+    dev_trsm_##SUF(upper, unit, n, nrhs, a, trans ? 1 : lda, trans ? lda : 1, b, ldb);                               \
+  }                                                                                                                  \
+  int orc_dev_getrf_##SUF(int n, T* a, int lda, int32_t* ipiv, int block, int base) {                                \
+    int32_t info = 0;                                                                                                \
+    for (int k = 0; k < n; k += block) {                                                                             \
+      const int nb = block < n - k ? block : n - k, e = k + nb, m = n - e;                                           \
+      dev_panel_##SUF(n, a, lda, ipiv, &info, k, nb, base);                                                          \
+      if (m <= 0) break;                                                                                             \
+      dev_trsm_##SUF(0, 1, nb, m, &AT(a, lda, k, k), lda, 1, &AT(a, lda, k, e), lda);                                \
+      dev_product_##SUF(m, m, nb, &AT(a, lda, e, k), lda, 1, &AT(a, lda, k, e), lda, &AT(a, lda, e, e), lda);        \
+    }                                                                                                                \
+    return info;                                                                                                     \
+  }
+DEVICE_ORDER(double, __builtin_fma, f64)
+DEVICE_ORDER(float, __builtin_fmaf, f32)
+
+/* ------------------------------------------------------------------------ */
 /* Checks                                                                   */
 /* ------------------------------------------------------------------------ */
 
