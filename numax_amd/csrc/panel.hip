@@ -10,7 +10,7 @@
 // pivot search is one exchange through a mailbox in device memory.
 #include <limits.h>
 
-#include "nmx_internal.h"
+#include "tile16.h"
 
 namespace {
 
@@ -84,10 +84,11 @@ struct PivKey<double> {
 // (ties to the lower row; the diagonal row counts as magnitude >= 0, so an
 // all-zero or all-NaN column keeps its diagonal; NaN never wins),
 // interchange, an exact-zero pivot divided as 1e-30 with `info` recording the
-// first, true division for the multipliers and the rank-1 update of the
-// panel's own columns.  The leaf's interchanges are then replayed over every
-// other column of the matrix right after (laswp_gather_kernel), which leaves
-// the matrix numax's full-width swaps leave (panel.mojo:404-411).
+// first, correctly rounded quotients for the multipliers and the rank-1
+// update of the panel's own columns, every multiply-add fused.  The leaf's
+// interchanges are then replayed over every other column of the matrix right
+// after (laswp_gather_kernel), which leaves the matrix numax's full-width
+// swaps leave (panel.mojo:404-411).
 //
 // Workgroup p of `parts` owns rows r0 + 512 ROWS p + t + 512 i (i < ROWS) of
 // its threads (alone, up to 1024 rows of as many threads), each row's 32
@@ -112,7 +113,11 @@ struct PivKey<double> {
 // register a column, with every column's update and select run to full width,
 // both rows physically swapped through LDS and three maxima a decision, a
 // column took 3.7 us (1000 rows FP64, one workgroup) and 4.0 us (8192 rows,
-// sixteen); it takes 1.6 us (mean over 1000 .. 32 rows) and 2.8 us.
+// sixteen); it takes 1.6 us (mean over 1000 .. 32 rows) and 2.9 us.
+// An FP64 quotient is the product with the pivot's reciprocal and two
+// corrections: one correction leaves rare last bits wrong, which a system of
+// condition 1e6 carries into x, and saves 1.4 of a 32-column leaf's 91.6 us
+// (order 8192, mean over its panels).
 // ---------------------------------------------------------------------------
 constexpr int kLeafT = 512;      // threads per workgroup of several
 constexpr int kLeafMaxT = 1024;  // threads at most, in a workgroup alone
@@ -169,20 +174,6 @@ __device__ __forceinline__ int winner_lane16(K key, int pos) {
   if (m & (m - 1)) return winner_lane(key, pos);  // uniform; the lanes above hold no key
   return __ffsll((long long)m) - 1;
 }
-
-// x / p, correctly rounded but for rare last bits: the product with p's
-// reciprocal corrected by its residual (a quarter of a division's
-// instructions).  |x| <= |p| here.  A pivot whose reciprocal would leave the
-// normal range, an infinity or a NaN divides.
-__device__ __forceinline__ double quotient(double x, double p) {
-  if (!(fabs(p) >= 1e-290 && fabs(p) <= 1e290)) return x / p;  // uniform
-  double r = __builtin_amdgcn_rcp(p);
-  r = __builtin_fma(__builtin_fma(-p, r, 1.0), r, r);
-  r = __builtin_fma(__builtin_fma(-p, r, 1.0), r, r);
-  const double q = x * r;
-  return __builtin_fma(__builtin_fma(-q, p, x), r, q);
-}
-__device__ __forceinline__ float quotient(float x, float p) { return x / p; }
 
 template <typename T>
 struct LeafLds {
@@ -347,13 +338,30 @@ __device__ __forceinline__ void leaf_step(const LeafArgs& a, T (&v)[ROWS][kLeafW
   // hold finished columns)
   bool live[ROWS];
   T l[ROWS];
+  // FP32 divides; FP64 too where an operand is out of the plain range
+  bool divide = sizeof(T) == 4 || !plain_divisor(pivot);  // uniform
+  if constexpr (sizeof(T) == 8) {
+    const T rinv = reciprocal(pivot);
+    bool odd = false;
 #pragma unroll
-  for (int i = 0; i < ROWS; i++) {
-    live[i] = pos[i] > gr && pos[i] < a.n;
-    const T q = quotient(v[i][S], pivot);
-    l[i] = q;
-    v[i][S] = live[i] ? q : v[i][S];
+    for (int i = 0; i < ROWS; i++) {
+      live[i] = pos[i] > gr && pos[i] < a.n;
+      const T x = v[i][S];
+      odd = odd || (live[i] && !plain_dividend(x));
+      const T q = plain_quotient(x, pivot, rinv);
+      l[i] = x == T(0) ? x * rinv : q;  // a zero keeps its sign
+    }
+    divide = divide || __ballot(odd) != 0;
   }
+  if (divide) {
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) {
+      live[i] = pos[i] > gr && pos[i] < a.n;
+      l[i] = v[i][S] / pivot;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < ROWS; i++) v[i][S] = live[i] ? l[i] : v[i][S];
 #pragma unroll
   for (int g = 0; g < W / kLeafG; g++) {
     if (g == 0 || jb + kLeafG * g < a.w) {  // uniform

@@ -88,8 +88,16 @@ __device__ __forceinline__ double quotient(double x, double d, double r) {
 __device__ __forceinline__ float quotient(float x, float d, float r) {
   return __builtin_amdgcn_div_fixupf(plain_quotient(x, d, r), d, x);
 }
+// 1 / d, correctly rounded unless d's significand is all ones (Markstein):
+// Newton's step from a value within an ulp.  d in the range below.
+__device__ __forceinline__ double reciprocal(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+}
 __device__ __forceinline__ bool plain_divisor(double d) { return fabs(d) >= 1e-90 && fabs(d) <= 1e90; }
 __device__ __forceinline__ bool plain_divisor(float d) { return fabsf(d) >= 1e-9f && fabsf(d) <= 1e9f; }
+__device__ __forceinline__ bool plain_dividend(double x) { return (fabs(x) >= 1e-180 && fabs(x) <= 1e180) || x == 0; }
 // a dividend's magnitude as an exponent; 0 for zeros, infinities and NaNs
 __device__ __forceinline__ int magnitude(double x) { return __builtin_amdgcn_frexp_exp(x); }
 __device__ __forceinline__ int magnitude(float x) { return __builtin_amdgcn_frexp_expf(x); }

@@ -474,3 +474,62 @@ def test_triangular_solves_keep_substitutions_order(n, nrhs, dtype):
         _trsm(T, B, upper, unit, trans, n, nrhs)
         with np.errstate(all="ignore"):
             _same_bits(_np(B), oracle.device_order_trsm(t, b, bool(upper), bool(unit), bool(trans)))
+
+
+def _lu_input(n, kind, npd):
+    """Matrices on which a leaf's decisions and quotients can go wrong: 1, small
+    integers (rows that tie in every column, zero pivots) with zero columns; 2,
+    columns and rows out of the quotients' plain range; 3, NaNs and infinities."""
+    rng = np.random.default_rng(100 * n + kind)
+    a = rng.standard_normal((n, n))
+    far = 200 if npd is np.float64 else 30
+    if kind == 1:
+        a = rng.integers(-2, 3, (n, n)).astype(np.float64)
+        a[:, [j for j in (5, 8, 31, 32, 37) if j < n]] = 0.0
+    elif kind == 2:
+        a[:, n // 2] *= 10.0 ** -far
+        a[n // 3] *= 10.0 ** (far - 10)
+        a[n // 5:, 9 % n] = 0.0
+    elif kind == 3:
+        a[n // 2, 0] = np.nan  # below the diagonal: never wins
+        a[n - 1, min(n - 1, 20)] = np.inf
+        if n > 9:
+            a[8, 8] = np.nan
+    return a.astype(npd)
+
+
+def _lu_bits(n, block, base, dtype, kinds):
+    npd = np.float64 if dtype == torch.float64 else np.float32
+    for kind in kinds:
+        a = _lu_input(n, kind, npd)
+        f = nl.lu_factor(torch.as_tensor(a, device="cuda"), block=block, base=base)
+        with np.errstate(all="ignore"):
+            lu, piv, info = oracle.device_order_getrf(a, block, base)
+        assert np.array_equal(_np(f.pivots), piv), kind
+        assert f.info == info, kind
+        _same_bits(_np(f.factored), lu)
+        if kind == 0:
+            b = np.random.default_rng(n).standard_normal((n, 3)).astype(npd)
+            w = oracle.laswp(b, piv).astype(npd)
+            x = oracle.device_order_trsm(lu, oracle.device_order_trsm(lu, w, False, True), True)
+            _same_bits(_np(f.solve(torch.as_tensor(b, device="cuda"))), x)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n", [1, 5, 31, 33, 40, 64, 129, 257, 512, 513, 1024, 1056, 1700])
+def test_lu_is_the_blocked_elimination_bit_for_bit(n, dtype):
+    """Factor, every pivot, ``info`` and solution equal the oracle's blocked
+    elimination in the device's order: correctly rounded quotients, ties, zeros
+    and NaNs in every eight-column group and leaf, one workgroup and several.
+    (Gaussian systems of order 8192 reach condition 1e6: x kept to 1e-9 of the
+    former x takes the same rounding, not only as good a one.)"""
+    _lu_bits(n, 256, 32, dtype, (0, 1, 2, 3))
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("block,base", [(16, 16), (32, 8), (64, 32), (100, 25), (33, 7), (192, 32), (512, 16)])
+@pytest.mark.parametrize("n", [17, 200, 600])
+def test_lu_runs_the_panels_it_is_given(n, block, base, dtype):
+    """Panels and leaves of the caller's widths: the same blocked elimination
+    with those widths, bit for bit."""
+    _lu_bits(n, block, base, dtype, (0, 1))
