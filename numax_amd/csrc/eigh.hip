@@ -206,15 +206,19 @@ __device__ __forceinline__ void jacobi_step(float (&a)[NP], float (&v)[NP], floa
     }
   }
   wave_lds_order();
-  // columns of A and V (with the exchange): new = alpha own + beta partner's
-  const float alpha = isP ? s : (isQ ? -s : 1.f);
-  const float beta = (isP || isQ) ? c : 0.f;
+  // columns of A and V (with the exchange): new = alpha own + beta partner's.
+  // Lanes without a pair sit out: beside one may be another matrix's lane, and
+  // a zero coefficient does not keep its infinities and NaNs out.  (What a
+  // neighbour reads of a lane that sits out is 0.)
+  const float alpha = isP ? s : -s;
   const float beta_next = isP ? c : 0.f, beta_prev = isQ ? c : 0.f;
+  if (OFF == 0 || isP || isQ) {
 #pragma unroll
-  for (int i = 0; i < NP; i += 4)
-    rotate_col4<OFF>(a[i], a[i + 1], a[i + 2], a[i + 3], alpha, beta, beta_next, beta_prev);
-  // V's rows past the matrix's order are never read
-  rotate_rows<NP, OFF, 0>(v, nmax, alpha, beta, beta_next, beta_prev);
+    for (int i = 0; i < NP; i += 4)
+      rotate_col4<OFF>(a[i], a[i + 1], a[i + 2], a[i + 3], alpha, c, beta_next, beta_prev);
+    // V's rows past the matrix's order are never read
+    rotate_rows<NP, OFF, 0>(v, nmax, alpha, c, beta_next, beta_prev);
+  }
   d = d_new;
   const int player_o = __float_as_int(other<OFF>(__int_as_float(player), isP));
   player = isP || isQ ? player_o : player;

@@ -150,3 +150,30 @@ def test_lstsq_shape_errors():
         nl.lstsq_batched(np.zeros((2, 8, 4), np.float32), np.zeros((2, 7), np.float32))
     with pytest.raises(ValueError):
         nl.lstsq_batched(np.zeros((1, 8, 40), np.float32), np.zeros((1, 8), np.float32))
+
+
+@pytest.mark.parametrize("sizes", [(31, 32), (5, 17, 32), (1, 2, 24), (33, 48, 64)])
+def test_eigh_batched_keeps_non_finite_matrices_to_themselves(sizes):
+    """A matrix with a NaN or an infinity beside every valid one: orders up to
+    32 share a wavefront in pairs.  The valid ones come out as in a batch that
+    holds no other, bit for bit."""
+    rng = np.random.default_rng(sum(sizes))
+    n = np.resize(np.array(sizes, dtype=np.int32), 240)
+    mats = []
+    for k in n:
+        m = rng.standard_normal((k, k)).astype(np.float32)
+        mats.append(m + m.T)
+    offa, offw = np.zeros(len(n), dtype=np.int64), np.zeros(len(n), dtype=np.int64)
+    offa[1:] = np.cumsum(n.astype(np.int64) ** 2)[:-1]
+    offw[1:] = np.cumsum(n.astype(np.int64))[:-1]
+    w0, v0 = (t.cpu().numpy() for t in nl.eigh_batched(np.concatenate([m.ravel() for m in mats]), n, offa, offw))
+    bad = [p for p in range(len(n)) if p % 7 in (1, 3, 4)]
+    for p in bad:
+        i, j = rng.integers(0, n[p], 2)
+        mats[p][i, j] = mats[p][j, i] = (np.nan, np.inf, -np.inf)[p % 3]
+    w1, v1 = (t.cpu().numpy() for t in nl.eigh_batched(np.concatenate([m.ravel() for m in mats]), n, offa, offw))
+    for p in range(len(n)):
+        if p in bad:
+            continue
+        np.testing.assert_array_equal(w1[offw[p]:offw[p] + n[p]], w0[offw[p]:offw[p] + n[p]], err_msg=f"matrix {p}")
+        np.testing.assert_array_equal(v1[offa[p]:offa[p] + n[p] ** 2], v0[offa[p]:offa[p] + n[p] ** 2], err_msg=f"matrix {p}")
