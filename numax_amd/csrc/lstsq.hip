@@ -6,8 +6,7 @@
 // (qr.mojo:470-534), then the upper-triangular solve with R
 // (qr.mojo:536-612).  Here the n reflectors are applied one column at a time
 // to [A | b] held whole in registers, and x comes from R and the first n
-// entries of Q^T b; R can differ from numax's in the sign of a row whose
-// column is already zero below the diagonal, x does not.
+// entries of Q^T b.
 //
 // What bounds it: not HBM (each problem is read once) but the chain of n
 // dependent reflectors per problem -- a sum over all rows, a square root and
@@ -23,7 +22,7 @@
 // round and one barrier across them).  With a row per lane instead, every
 // step reduced 33 values over 256 threads and read them back: 165 LDS reads
 // and 126 shuffles a step, and 4096 problems of 1024 x 32 took 6.55 ms.
-// In this layout they take 0.62 ms (10.8x; 885 GB/s of the 4.8 TB/s a copy
+// In this layout they take 0.65 ms (10.4x; 850 GB/s of the 4.8 TB/s a copy
 // reaches): the broadcasts are the DPP operand of the multiply-adds (0.64 ms
 // as separate moves), 60 % of the time is issue, the rest the step's barrier
 // and LDS round.
@@ -61,12 +60,11 @@ struct GelsLds {
   float y[32];
 };
 
-// Reflector K.  Rows 0 .. K-1 have left the registers (they are zero there
-// and their R is in LDS), so sums over all rows are sums over rows >= K:
-// S = |x|^2 with x the column including row K, beta = -sign(alpha) sqrt(S),
-// and with w = x - beta e_K the reflector is I - w w^T / (beta (beta - alpha));
-// w^T A_j = x^T A_j - beta A_Kj needs only the sums.  beta - alpha has no
-// cancellation.  S = 0 leaves the column (f = 0).
+// Reflector K.  Rows 0 .. K have left the registers (they are zero there; the
+// finished ones' R is in LDS), so sums over all rows are sums below the diagonal:
+// sigma = x^T x, beta = -sign(alpha) sqrt(alpha^2 + sigma), v = [1; x / (alpha -
+// beta)], tau = (beta - alpha) / beta, and a column that is zero below its
+// diagonal stays as it is (geqr2_panel's dlarfg convention).
 template <int K, int NW, int SETS>
 __device__ __forceinline__ void gels_step(float (&a)[SETS][kRows], float (&b)[2], int t, GelsLds<NW>& L) {
   constexpr int set = K >> 4, lk = K & 15;
@@ -77,6 +75,17 @@ __device__ __forceinline__ void gels_step(float (&a)[SETS][kRows], float (&b)[2]
   asm volatile("" : "+v"(t));
   const int lane = t & 63, wave = NW == 1 ? 0 : t >> 6;
   const int c = lane & 15, g = lane >> 4;
+  if (t < 16) {
+#pragma unroll
+    for (int s = s0; s < SETS; s++) {
+      L.row[buf][2 * c + s] = a[s][K];
+      a[s][K] = 0.f;
+    }
+  }
+  if (t == K / 2) {
+    L.row[buf][32] = b[K & 1];
+    b[K & 1] = 0.f;
+  }
   // b is held two rows a lane: it meets the column through LDS (own wavefront, in order)
   float* xg = L.x[wave][g];
   if (c == lk) {
@@ -86,11 +95,6 @@ __device__ __forceinline__ void gels_step(float (&a)[SETS][kRows], float (&b)[2]
   }
   wave_lds_order();
   const float2 xb = *(const float2*)(xg + 2 * c);
-  if (t < 16) {
-#pragma unroll
-    for (int s = s0; s < SETS; s++) L.row[buf][2 * c + s] = a[s][K];
-  }
-  if (t == K / 2) L.row[buf][32] = b[K & 1];
   float p[SETS];
 #pragma unroll
   for (int s = s0; s < SETS; s++) {
@@ -131,24 +135,25 @@ __device__ __forceinline__ void gels_step(float (&a)[SETS][kRows], float (&b)[2]
   }
   const float2 rk = *(const float2*)&L.row[buf][2 * c];
   const float bk = L.row[buf][32];
-  const float S = row_bcast<lk>(tot[set]);
+  const float sigma = row_bcast<lk>(tot[set]);
   const float alpha = row_bcast<lk>(set ? rk.y : rk.x);
-  const float beta = -copysignf(sqrtf(S), alpha);
-  const float i0 = S == 0.f ? 0.f : 1.f / beta, i1 = S == 0.f ? 0.f : 1.f / (beta - alpha);
-  const float wk = alpha - beta;
+  const bool none = sigma == 0.f;
+  const float beta = none ? alpha : -copysignf(sqrtf(fmaf(alpha, alpha, sigma)), alpha);
+  const float tau = (beta - alpha) / beta, scale = 1.f / (alpha - beta);
   float f[SETS];
 #pragma unroll
   for (int s = s0; s < SETS; s++) {
     const float rks = s ? rk.y : rk.x;
-    const float fs = (tot[s] - beta * rks) * i0 * i1;
-    f[s] = 16 * s + c > K ? fs : 0.f;  // finished columns and K itself stay
+    // finished columns, K itself and every column of a reflector that is none stay
+    const float fs = 16 * s + c > K && !none ? tau * (rks + scale * tot[s]) : 0.f;
     if (t < 16) {
       const int col = 16 * s + c;
-      if (col >= K) L.R[K][col] = col == K ? beta : rks - f[s] * wk;
+      if (col >= K) L.R[K][col] = col == K ? beta : rks - fs;
     }
+    f[s] = none ? 0.f : fs * scale;
   }
-  const float fb = (tb - beta * bk) * i0 * i1;
-  if (t == 0) L.y[K] = bk - fb * wk;
+  const float fy = none ? 0.f : tau * (bk + scale * tb), fb = none ? 0.f : fy * scale;
+  if (t == 0) L.y[K] = bk - fy;
   // the other sets first: x is read from its own set's registers
 #pragma unroll
   for (int s = SETS - 1; s >= s0; s--)
@@ -162,12 +167,6 @@ __device__ __forceinline__ void gels_step(float (&a)[SETS][kRows], float (&b)[2]
     }
   b[0] -= xb.x * fb;
   b[1] -= xb.y * fb;
-  // row K is finished
-  if (t < 16) {
-#pragma unroll
-    for (int s = s0; s < SETS; s++) a[s][K] = 0.f;
-  }
-  if (t == K / 2) b[K & 1] = 0.f;
 }
 
 template <int K, int NW, int SETS>
@@ -233,7 +232,8 @@ gels_kernel(int count, int m, int n, const float* __restrict__ A, const float* _
     }
     // R x = (Q^T b)[0:n] in wavefront 0, a row per lane; the reciprocals of
     // the diagonal once for all lanes, each quotient corrected by its residual
-    // (a division inside the chain costs four times as much)
+    // (a division inside the chain costs four times as much; it is taken where
+    // an entry of the diagonal has no finite reciprocal)
     if (t < 64) {
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -246,12 +246,14 @@ gels_kernel(int count, int m, int n, const float* __restrict__ A, const float* _
       float acc = live ? L.y[i] : 0.f;
       const float diag = live ? L.R[i][i] : 1.f;
       const float inv = 1.f / diag;
+      const bool divide = __ballot(!(fabsf(diag) >= 1e-37f)) != 0;
 #pragma unroll
       for (int q = 16 * SETS - 1; q >= 0; q--) {
         if (q < n) {  // uniform
           float v = acc * inv;
           const float v2 = fmaf(fmaf(-v, diag, acc), inv, v);
-          v = v2 == v2 ? v2 : v;  // a zero diagonal keeps its infinity
+          v = v2 == v2 ? v2 : v;  // an infinity stays one
+          if (divide) v = acc / diag;  // uniform
           const float xq = readlane_f(v, q);
           if (i == q) acc = xq;
           else if (i < q) acc -= rr[q] * xq;

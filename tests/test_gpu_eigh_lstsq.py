@@ -177,3 +177,36 @@ def test_eigh_batched_keeps_non_finite_matrices_to_themselves(sizes):
             continue
         np.testing.assert_array_equal(w1[offw[p]:offw[p] + n[p]], w0[offw[p]:offw[p] + n[p]], err_msg=f"matrix {p}")
         np.testing.assert_array_equal(v1[offa[p]:offa[p] + n[p] ** 2], v0[offa[p]:offa[p] + n[p] ** 2], err_msg=f"matrix {p}")
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 16, 17, 32])
+@pytest.mark.parametrize("extra", [0, 1, 130, 2100])
+def test_lstsq_batched_leaves_columns_that_are_zero_below_the_diagonal(n, extra):
+    """Upper triangles over `extra` zero rows, as the last column of every square
+    problem is one: no reflector squares the diagonal, so entries whose square
+    under- or overflows solve like any other, a subnormal one too, and an
+    infinity right of the diagonal reaches the unknowns above it only.  The
+    solution is back substitution's, each unknown within n + 2 roundings of the
+    terms it sums."""
+    rng = np.random.default_rng(40 * n + extra)
+    m, scales = n + extra, [1.0, 3e-30, 2e-23, 4e19, 2e37]
+    a = np.zeros((len(scales) + 2, m, n), dtype=np.float32)
+    b = rng.standard_normal((len(a), m)).astype(np.float32)
+    for p, s in enumerate(scales + [1.0, 1.0]):
+        a[p, :n] = (s * (np.triu(rng.uniform(-0.5, 0.5, (n, n)) / n, 1) + np.diag(rng.uniform(1.0, 2.0, n)))).astype(np.float32)
+        b[p] *= np.float32(s)
+    a[-1, n - 1, n - 1], b[-1, n - 1] = 3e-39, 1e-39
+    if n > 2:
+        a[-2, 0, n - 1] = np.inf
+    x = nl.lstsq_batched(a, b).cpu().numpy().astype(np.float64)
+    eps = np.finfo(np.float32).eps
+    for p in range(len(a)):
+        u, y = a[p, :n].astype(np.float64), b[p, :n].astype(np.float64)
+        for i in range(n - 1, -1, -1):
+            if not np.isfinite(u[i]).all():
+                assert not np.isfinite(x[p, i])
+                continue
+            # against the unknowns that the kernel found, so that roundings do not add up
+            terms = u[i, i + 1:] * x[p, i + 1:]
+            bound = (n + 2) * eps * (np.abs(terms).sum() + abs(y[i])) / abs(u[i, i])
+            assert abs(x[p, i] - (y[i] - terms.sum()) / u[i, i]) <= bound, (p, i)
