@@ -18,7 +18,8 @@
 // Goldschmidt iteration on v_rsq with residual corrections, and a column's
 // quotients are products corrected by their residuals; a pivot out
 // of their range (negative, zero, tiny, huge, NaN) sends the tile through the
-// plain square roots and divisions.  64 columns a launch with a
+// plain square roots and divisions, and a tile of X that is not finite through
+// plain substitution.  64 columns a launch with a
 // barrier per column took 55 us FP64 (27 us for 32 columns FP32), and a 128
 // column block two of them, a triangular solve and a product.
 // 128 columns FP64: 36 us; 256 columns FP32: 75 us.  FP64 Cholesky + solve of
@@ -113,6 +114,31 @@ __device__ __forceinline__ void chol_tile_general(T (*D)[17], int lane, int cols
   }
 }
 
+// x = c L_ss^-T by plain substitution, a row per lane 0..15, in the wavefront's
+// own LDS tile: where a quotient is not finite, so that an infinity or NaN
+// spreads to the columns right of it and no others, and an infinite pivot
+// gives zeros.
+template <typename T>
+__device__ __forceinline__ void chol_substitute(const T (*D)[17], T (*tile)[64], int lane, const typename Acc<T>::type& c,
+                                                typename Acc<T>::type& x) {
+#pragma unroll
+  for (int e = 0; e < 4; e++) tile[e][lane] = c[e];
+  wave_lds_order();
+  if (lane < 16) {
+    auto at = [&](int j) -> T& { return sizeof(T) == 8 ? tile[j >> 2][16 * (j & 3) + lane] : tile[j & 3][16 * (j >> 2) + lane]; };
+#pragma unroll 1
+    for (int j = 0; j < 16; j++) {
+      const T l = at(j) / D[j][j];
+      at(j) = l;
+#pragma unroll 1
+      for (int i = j + 1; i < 16; i++) at(i) = at(i) - l * D[i][j];
+    }
+  }
+  wave_lds_order();
+#pragma unroll
+  for (int e = 0; e < 4; e++) x[e] = tile[e][lane];
+}
+
 template <typename T, int NB16>
 struct CholLds {
   T D[16][17];         // the step's factored diagonal tile, row-major
@@ -197,6 +223,10 @@ __global__ void __launch_bounds__(64 * NB16) chol_block_kernel(T* __restrict__ A
       for (int q = 0; q < 4; q++) res = mma(ld[q], -x[q], res);
 #pragma unroll
       for (int q = 0; q < 4; q++) x = mma(iv[q], res[q], x);
+      bool bad = false;
+#pragma unroll
+      for (int e = 0; e < 4; e++) bad = bad || !finite(x[e]);
+      if (__ballot(bad)) chol_substitute<T>(L.D, L.x[w], lane, c[0], x);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         L.x[w][e][lane] = -x[e];

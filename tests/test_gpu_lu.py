@@ -396,6 +396,33 @@ def test_cholesky_block_edges(n, dtype):
     assert np.all(err <= 4 * (n + 1) * torch.finfo(dtype).eps * np.outer(d, d))
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n,i,j,value", [(40, 30, 5, np.nan), (128, 100, 20, np.nan), (128, 127, 111, np.inf),
+                                         (256, 200, 190, np.nan), (60, 7, 7, np.inf), (128, 70, 70, np.inf),
+                                         (300, 290, 17, -np.inf), (256, 129, 129, np.nan)])
+def test_cholesky_spreads_infinities_as_column_elimination_does(n, i, j, value, dtype):
+    """One entry that is not finite: entries that the plain column loop leaves
+    finite are finite and right, the others are its infinities and NaNs.  An
+    infinite pivot gives a column of zeros."""
+    npd = np.float64 if dtype == torch.float64 else np.float32
+    a = R.spd_matrix(n + i, n).astype(npd)
+    a[i, j] = value
+    low = _np(nl.cholesky(torch.as_tensor(a, device="cuda")))
+    ref = np.tril(a.astype(np.float64))
+    with np.errstate(all="ignore"):
+        for k in range(n):
+            ref[k, k] = np.sqrt(ref[k, k])
+            ref[k + 1:, k] /= ref[k, k]
+            ref[k + 1:, k + 1:] -= np.tril(np.outer(ref[k + 1:, k], ref[k + 1:, k]))
+    ref = np.tril(ref)
+    np.testing.assert_array_equal(np.isnan(low), np.isnan(ref))
+    np.testing.assert_array_equal(np.isinf(low), np.isinf(ref))
+    ok = np.isfinite(ref)
+    # each entry: the elimination's n roundings of terms bounded by the diagonal's root
+    tol = 8 * (n + 1) * np.finfo(npd).eps * np.sqrt(np.max(np.diag(a)[np.isfinite(np.diag(a))]))
+    assert np.all(np.abs(low[ok] - ref[ok]) <= tol)
+
+
 @pytest.mark.parametrize("n,at", [(40, 0), (40, 17), (130, 127), (300, 16), (300, 299)])
 def test_cholesky_reports_the_first_bad_pivot(n, at):
     a = R.spd_matrix(n, n)
