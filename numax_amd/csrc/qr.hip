@@ -284,8 +284,10 @@ __device__ __forceinline__ void panel_step(T (&a)[R], T& sc, int t, int nb, T* _
   const bool none = sigma == T(0);
   const T tj = none ? T(0) : (beta - alpha) / beta;
   const T scale = none ? T(0) : T(1) / (alpha - beta);
-  const T g = rk + scale * tot * sc;            // v_K^T A_c; for finished columns v_K^T v_c
-  const T f = c > K ? tj * g : T(0);
+  // v_K^T A_c; for finished columns v_K^T v_c.  Of a column that is zero below
+  // its diagonal v_K is a unit vector: nothing below it counts, infinities included
+  const T g = none ? rk : rk + scale * tot * sc;
+  const T f = c > K && !none ? tj * g : T(0);
   const T nfs = -(f * scale);
   if (c == K && !none) sc = scale;
   if (c >= K) {  // lane K, which the products read, is among them; its own is 0

@@ -195,3 +195,19 @@ def test_narrow_panels_at_the_register_kernels_edges(m, n, block):
         _lib.check(nl._fn("geqrf", wide.dtype)(nl._ctx(wide).handle, m, n, nl._ptr(wide), n + 5, nl._ptr(taus), block),
                    "geqrf")
         assert torch.equal(wide[:, :n], f.factored) and bool((wide[:, n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("m,n", [(20, 5), (300, 16), (1500, 20), (3000, 16)])
+def test_narrow_panels_skip_columns_that_are_zero_below_the_diagonal(m, n):
+    """Such a column has no reflector (tau 0): it leaves its row of R as the
+    matrix has it, also left of an infinity further down in a later column."""
+    for dtype in (np.float64, np.float32):
+        a = R.normal(m + n, (m, n)).astype(dtype)
+        a[1:, 0] = 0
+        a[2:, 1] = 0
+        a[m - 1, n - 1] = np.inf
+        f = nl.qr_factor(a)
+        qr, tau = f.factored.cpu().numpy(), f.taus.cpu().numpy()
+        assert tau[0] == 0 and tau[1] == 0
+        np.testing.assert_array_equal(qr[:2, :16], a[:2, :16])
+        assert np.isfinite(qr[:, :min(n, 16) - 1]).all()
