@@ -59,6 +59,21 @@ __device__ __forceinline__ void root_pair(float d, float& root, float& rinv) {
   rinv = __builtin_fmaf(__builtin_fmaf(-t, g, 1.f), t, t);
 }
 
+// Row I of column c of the inverse of the lower triangular block whose rows
+// the 16 lanes hold (m: row `lane % 16`, rinv: the reciprocal of its diagonal);
+// ny is the inverse's column negated.
+template <int I, typename T>
+__device__ __forceinline__ void invert_rows(const T (&m)[16], T rinv, int c, T (&ny)[16]) {
+  if constexpr (I < 16) {
+    T s0 = I == c ? T(1) : T(0), s1 = T(0);
+#pragma unroll
+    for (int j = 0; j < I; j++) fmac_bcast<I>(j & 1 ? s1 : s0, m[j], ny[j]);
+    const T q = (s0 + s1) * row_bcast<I>(rinv);
+    ny[I] = I < c ? T(0) : -q;
+    invert_rows<I + 1, T>(m, rinv, c, ny);
+  }
+}
+
 // m[C] -= l * (lane C's m[J]) for the columns right of J
 template <int J, int C, typename T>
 __device__ __forceinline__ void chol_update(T (&m)[16], T nl) {

@@ -76,12 +76,6 @@ __device__ __forceinline__ int seg_min(int v) {
   return v;
 }
 
-// LDS written by some lanes of a wavefront is read by the others of it
-__device__ __forceinline__ void wave_lds_order() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // One elimination step.  row: this segment's LDS buffer, NP + 1 entries.
 template <int K, typename T, int NP, int SEG, int KIND>
 __device__ __forceinline__ void seg_step(T (&m)[NP], T& v, int& pos, int i, T* row) {

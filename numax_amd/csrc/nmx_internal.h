@@ -277,3 +277,9 @@ __device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
 __device__ __forceinline__ float readlane_f(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
+
+// LDS written by some lanes of a wavefront is read by the others of it
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}

@@ -1,13 +1,14 @@
 // Panel kernels of the blocked factorizations: the cooperative pivoting leaf,
-// row interchanges, triangular solves, the Cholesky diagonal block, and the
-// small gather / tril helpers.
+// row interchanges, the recursion of the triangular solves, and the small
+// gather / tril helpers.
 //
 // numax runs its panels as single-workgroup kernels over the whole remaining
 // height (numax/linalg/panel.mojo:289-431) while the rest of the device idles;
 // its own docstring names that as the ceiling (panel.mojo:41-49).  Here the
-// leaf of the recursive panel is spread over up to 32 workgroups of 1024
-// threads, one matrix row per thread held in registers, and the per-column
-// pivot search is one exchange through a mailbox in device memory.
+// leaf of the recursive panel is spread over up to 32 workgroups of 512
+// threads, one matrix row per thread held in registers (two above 16384 rows),
+// and the per-column pivot search is one exchange through a mailbox in device
+// memory; up to 1024 rows one workgroup holds them all.
 #include <limits.h>
 
 #include "tile16.h"
@@ -16,11 +17,6 @@ namespace {
 
 constexpr double kPivotFloor = 1e-30;  // numax/linalg/common.mojo:27-29
 constexpr long kSpinLimit = 1L << 23;  // bounded waits: a few seconds at worst
-
-template <typename T>
-__device__ __forceinline__ bool better(T ma, int ra, T mb, int rb) {
-  return ma > mb || (ma == mb && ra < rb);
-}
 
 // ---- mailbox ----------------------------------------------------------------
 // Every word a participant publishes is a 64-bit atomic holding 32 bits of
@@ -42,16 +38,6 @@ __device__ __forceinline__ uint64_t mb_pack(uint32_t payload, uint32_t epoch) {
 }
 __device__ __forceinline__ void mb_put(uint64_t* w, uint32_t payload, uint32_t epoch) {
   __hip_atomic_store(w, mb_pack(payload, epoch), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void mb_put_value(uint64_t* w, T v, uint32_t epoch) {
-  if (sizeof(T) == 8) {
-    const uint64_t bits = __double_as_longlong((double)v);
-    mb_put(w, (uint32_t)bits, epoch);           // low half first
-    mb_put(w + 1, (uint32_t)(bits >> 32), epoch);
-  } else {
-    mb_put(w, __float_as_uint((float)v), epoch);
-  }
 }
 
 // Pivot keys: a candidate's magnitude as its (order-preserving) bit pattern

@@ -147,11 +147,12 @@ __device__ int lds_lu_piv(T* M, T* v, int n, int lane) {
 // forward_substitution (_array/triangular.mojo:24-43) of the vector in v,
 // in place: row i subtracts l_ij x_j for j = 0 .. i-1 in that order, which
 // the column sweep keeps (lane i accumulates row i's total as x_j appear).
+// Unit diagonal.
 template <typename T>
-__device__ void lds_forward(const T* M, T* v, int n, int lane, bool unit) {
+__device__ void lds_forward(const T* M, T* v, int n, int lane) {
   T total = lane < n ? v[lane] : (T)0;
   for (int j = 0; j < n; j++) {
-    if (lane == j) v[j] = unit ? total : total / guard(M[j * kLd + j]);
+    if (lane == j) v[j] = total;
     __syncthreads();
     const T xj = v[j];
     if (lane > j && lane < n) total = total - M[lane * kLd + j] * xj;
@@ -161,15 +162,14 @@ __device__ void lds_forward(const T* M, T* v, int n, int lane, bool unit) {
 
 // back_substitution (_array/triangular.mojo:46-63), in place: row i
 // subtracts u_ij x_j for j = i+1 .. n-1 in that order, so every row waits
-// for the one below it -- one lane walks it.  TRANS reads U = M^T (the
-// Cholesky solve's L^T).
-template <typename T, bool TRANS>
+// for the one below it -- one lane walks it.
+template <typename T>
 __device__ void lds_back(const T* M, T* v, int n, int lane) {
   if (lane == 0) {
     for (int s = 0; s < n; s++) {
       const int i = n - 1 - s;
       T total = v[i];
-      for (int j = i + 1; j < n; j++) total = total - (TRANS ? M[j * kLd + i] : M[i * kLd + j]) * v[j];
+      for (int j = i + 1; j < n; j++) total = total - M[i * kLd + j] * v[j];
       v[i] = total / guard(M[i * kLd + i]);
     }
   }
@@ -195,8 +195,8 @@ __global__ void __launch_bounds__(64) small_wave_kernel(SmallArgs<T> a) {
         break;
       case OP_SOLVE:
         lds_lu(M, n, lane);
-        lds_forward(M, V, n, lane, true);
-        lds_back<T, false>(M, V, n, lane);
+        lds_forward(M, V, n, lane);
+        lds_back(M, V, n, lane);
         if (lane < n) a.X[xo + lane] = V[lane];
         break;
       case OP_INVERSE:

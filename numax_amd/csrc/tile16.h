@@ -1,5 +1,5 @@
-// 16 x 16 tiles on MFMA and on 16-lane rows: what the triangular and Cholesky
-// block kernels share.
+// 16 x 16 tiles on MFMA and on 16-lane rows, and correctly rounded quotients:
+// what the triangular, Cholesky, LU and QR kernels share.
 #pragma once
 
 #include "nmx_internal.h"
@@ -104,21 +104,6 @@ __device__ __forceinline__ int magnitude(float x) { return __builtin_amdgcn_frex
 template <typename T>
 constexpr int plain_magnitude() { return sizeof(T) == 8 ? 600 : 90; }  // dividends of 2^-this .. 2^this
 
-// Row I of column c of the inverse of the lower triangular block whose rows
-// the 16 lanes hold (m: row `lane % 16`, rinv: the reciprocal of its diagonal);
-// ny is the inverse's column negated.
-template <int I, typename T>
-__device__ __forceinline__ void invert_rows(const T (&m)[16], T rinv, int c, T (&ny)[16]) {
-  if constexpr (I < 16) {
-    T s0 = I == c ? T(1) : T(0), s1 = T(0);
-#pragma unroll
-    for (int j = 0; j < I; j++) fmac_bcast<I>(j & 1 ? s1 : s0, m[j], ny[j]);
-    const T q = (s0 + s1) * row_bcast<I>(rinv);
-    ny[I] = I < c ? T(0) : -q;
-    invert_rows<I + 1, T>(m, rinv, c, ny);
-  }
-}
-
 // acc += x(lane K of the 16-lane row) * y for four registers, the broadcast as
 // the multiply-add's DPP operand (the compiler makes a move of it, which would
 // double the instructions and keep R broadcast values live).  s_nop 1: the two
@@ -157,12 +142,6 @@ __device__ __forceinline__ void fmac_self4(float& x0, float& x1, float& x2, floa
 template <int K>
 __device__ __forceinline__ void fmac_self4(double& x0, double& x1, double& x2, double& x3, double s) {
   NMX_FMAC_DPP4_SELF("f64", x0, x1, x2, x3, s, K);
-}
-
-// LDS written by some lanes of a wavefront is read by the others of it
-__device__ __forceinline__ void wave_lds_order() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
 }
 
 }  // namespace

@@ -687,8 +687,8 @@ int tslu_panel_launch(nmx_ctx* ctx, void* scratch, size_t scratch_bytes, int n, 
     const int rows = m - w, cols = pc1 - c0 - w;
     if (rows > 0 && cols > 0)
       NMX_TRY(gemm_launch<float>(ctx, 0, 0, rows, cols, w, -1.0f, A + (int64_t)(r0 + w) * lda + c0, lda,
-                                A + (int64_t)r0 * lda + c0 + w, lda, 1.0f, A + (int64_t)(r0 + w) * lda + c0 + w, lda,
-                                0));
+                                 A + (int64_t)r0 * lda + c0 + w, lda, 1.0f, A + (int64_t)(r0 + w) * lda + c0 + w, lda,
+                                 0));
   }
   if (swap_outside) {
     NMX_TRY(tslu_swap_columns(ctx, scratch, A, lda, k, nb, 0, k, slot));
