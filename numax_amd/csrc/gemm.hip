@@ -341,10 +341,12 @@ int gemm_launch(nmx_ctx* ctx, int transa, int transb, int m, int n, int k, T alp
   // 96 x 96 10.1 / 5.8, 512 x 512 x 16 6.2 / 5.9).  Of up to four a CU a short
   // chain loses to the reuse of operands (1024 x 512 x 32 7.3 / 8.7, x 192 17.1
   // / 15.0, 4096 x 128 x 128 12.6 / 12.6), of more any (1024 x 1024 x 192 17 /
-  // 24).  The order of every sum is the same.
+  // 24).  The order of every sum is the same.  Its offsets are 32-bit over the
+  // 64 rows of an operand that a buffer of slabs spans.
   const int nf = n <= 16 ? 1 : 2;
   const int64_t thin_tiles = (int64_t)ceil_div(m, 16) * ceil_div(n, 16 * nf) / (lower_only ? 2 : 1);
-  if (thin_tiles <= (k < 128 ? 2 : 4) * ctx->num_cus && !(transa && transb)) {
+  const bool near_rows = 64 * (int64_t)std::max(lda, ldb) * (int64_t)sizeof(T) < 0x7FFFFFFF;
+  if (thin_tiles <= (k < 128 ? 2 : 4) * ctx->num_cus && !(transa && transb) && near_rows) {
     auto thin = [&](auto nf_tag) {
       constexpr int NF = decltype(nf_tag)::value;
       const dim3 tg(ceil_div(m, 16), ceil_div(n, 16 * NF));

@@ -61,6 +61,24 @@ def test_gemm_tile_shapes_agree_bitwise(dtype, transa, transb):
     assert np.max(np.abs(full - ref)) <= tol * max(1.0, np.max(np.abs(ref))) * np.sqrt(k)
 
 
+@pytest.mark.parametrize("transa", [0, 1])
+def test_gemm_of_few_columns_in_very_wide_rows(transa):
+    """Rows so far apart that 64 of them span more than 2 GiB: the operand that
+    is walked down its rows is B, or A transposed."""
+    from numax_amd import _lib
+    m, n, k, wide = 20, 16, 70, 4_300_000
+    rng = np.random.default_rng(transa)
+    a, b, c = rng.standard_normal((m, k)), rng.standard_normal((k, n)), rng.standard_normal((m, n))
+    far = torch.empty((k, wide), dtype=torch.float64, device="cuda")
+    far[:, :m if transa else n] = torch.as_tensor(a.T if transa else b, device="cuda")
+    near = torch.as_tensor(b if transa else a, device="cuda").contiguous()
+    C = torch.as_tensor(c, device="cuda")
+    A, B = (far, near) if transa else (near, far)
+    _lib.check(nl._fn("gemm", torch.float64)(nl._ctx(C).handle, transa, 0, m, n, k, -1.0, nl._ptr(A), A.shape[1], nl._ptr(B),
+                                             B.shape[1], 1.0, nl._ptr(C), n), "gemm")
+    assert np.max(np.abs(_np(C) - (c - a @ b))) <= 1e-12
+
+
 @pytest.mark.parametrize("n", [1, 7, 64, 65, 200, 300])
 @pytest.mark.parametrize("upper,unit,trans", [(0, 0, 0), (0, 1, 0), (1, 0, 0), (0, 0, 1), (1, 0, 1), (1, 1, 1)])
 def test_solve_triangular_matches_oracle(n, upper, unit, trans):
