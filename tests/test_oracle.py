@@ -127,6 +127,66 @@ def test_getrf_block_invariance(block, base):
     np.testing.assert_allclose(lu, ref, atol=1e-12)
 
 
+def _fma(a, b, c):
+    """a b + c rounded once, through exact rationals."""
+    return float(Fraction(float(a)) * Fraction(float(b)) + Fraction(float(c)))
+
+
+@pytest.mark.parametrize("upper", [False, True])
+def test_device_order_trsm_is_the_fused_substitution_it_names(upper):
+    """70 rows: 64 + 6, each block substituted column by column, the product
+    between them from zero in ascending order, every multiply-add rounded once."""
+    rng = np.random.default_rng(70)
+    n, n1 = 70, 64
+    a = rng.standard_normal((n, n)) / 8 + 2 * np.eye(n)
+    x = rng.standard_normal((n, 1))
+    got = oracle.device_order_trsm(a, x, upper)
+    w = [float(v) for v in x[:, 0]]
+
+    def block(lo, hi):
+        for j in (range(hi - 1, lo - 1, -1) if upper else range(lo, hi)):
+            w[j] = float(Fraction(w[j]) / Fraction(float(a[j, j])))
+            for i in (range(lo, j) if upper else range(j + 1, hi)):
+                w[i] = _fma(-a[i, j], w[j], w[i])
+
+    first, second = ((n1, n), (0, n1)) if upper else ((0, n1), (n1, n))
+    block(*first)
+    for i in range(*second):
+        acc = 0.0
+        for k in range(*first):
+            acc = _fma(a[i, k], w[k], acc)
+        w[i] -= acc
+    block(*second)
+    np.testing.assert_array_equal(got[:, 0], w)
+    t = np.triu(a) if upper else np.tril(a)
+    np.testing.assert_allclose(oracle.device_order_trsm(a.T.copy(), x, upper, trans=True), got, rtol=0)
+    np.testing.assert_allclose(t @ got, x, atol=1e-12)
+
+
+def test_device_order_getrf_is_gepp():
+    """The pivots of the panel recursion above, P A = L U, and one leaf's
+    arithmetic through exact rationals, in both types."""
+    for n, block, base in ((70, 16, 16), (200, 64, 32), (200, 100, 25)):
+        a = R.normal(n, (n, n))
+        lu, piv, info = oracle.device_order_getrf(a, block, base)
+        np.testing.assert_array_equal(piv, oracle.getrf(a)[1])
+        assert info == 0
+        np.testing.assert_allclose(a[perm_from_ipiv(piv)], (np.tril(lu, -1) + np.eye(n)) @ np.triu(lu), atol=1e-12)
+        lu32, piv32, _ = oracle.device_order_getrf(a.astype(np.float32), block, base)
+        assert lu32.dtype == np.float32
+        np.testing.assert_allclose(a[perm_from_ipiv(piv32)], (np.tril(lu32, -1) + np.eye(n)) @ np.triu(lu32), atol=1e-3)
+    n = 9
+    a = R.normal(n, (n, n))
+    lu, piv, _ = oracle.device_order_getrf(a, 32, 32)
+    w = a[perm_from_ipiv(piv)].tolist()
+    for j in range(n):
+        for i in range(j + 1, n):
+            w[i][j] = float(Fraction(w[i][j]) / Fraction(w[j][j]))
+            for c in range(j + 1, n):
+                w[i][c] = _fma(-w[i][j], w[j][c], w[i][c])
+    np.testing.assert_array_equal(lu, w)
+
+
 def test_getrf_invariant_pa_eq_lu():
     a = R.normal(5, (200, 200))
     lu, piv, _, _ = oracle.getrf(a)
